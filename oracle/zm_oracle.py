@@ -29,7 +29,7 @@ assert Q8K_DTYPE.itemsize == 292
 
 def build() -> None:
     subprocess.run(["make", "-s", "-C", HERE], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/bench/q2k_dot_bench.cpp"):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
