@@ -1,0 +1,100 @@
+"""The grouped int8-MFMA product (MUL_MAT_ID of batches and prefill) at the
+edges of its tiling: buckets around 16, 32 and 64 pairs, rows off the 16- and
+64-row tiles, one to seven K blocks, weights that do not start on a dword, and
+the pair count from which it is taken.
+
+Bar: 2e-5 of sum_i |w x| per output.  The integer block sums are exact; what is
+left is f32 rounding of at most 7 block terms and of the two products each is
+the difference of (2^-24 each, the terms up to a few times the sum): below
+2e-6 of the bound, and as much in the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import zm_oracle as O
+from moe_cases import CONFIGS, IQ2, IQ3, IQ4, Q2, Q3, Q4, Q5, Q6, Built, reduced
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [Q2, Q3, Q4, Q5, Q6, IQ2, IQ3, IQ4]
+TOL = 2e-5
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    import zeromoe_amd as Z
+
+    assert torch.cuda.is_available(), "GPU tests need a device"
+    Z.init()
+    yield
+
+
+def _place(W, offset):
+    """W on the device, starting `offset` bytes past an aligned address."""
+    buf = torch.zeros(W.size + 16, dtype=torch.uint8, device="cuda")
+    v = buf[offset:offset + W.size].view(W.shape)
+    v.copy_(torch.from_numpy(W))
+    return v
+
+
+def _check(t, I, rows, sizes, offset=0, extra=()):
+    import zeromoe_amd as Z
+
+    E = len(sizes)
+    ids = np.concatenate([np.full(n, e) for e, n in enumerate(sizes)] + [np.array(extra, int)]).astype(np.int32)
+    ids = np.random.default_rng(I + rows).permutation(ids).reshape(-1, 1)
+    S = len(ids)
+    print(f"mmq t={t} I={I} O={rows} sizes={sizes} offset={offset}", flush=True)
+    W = O.random_blocks(t, E * rows, I, seed=t + I).reshape(E, rows, -1)
+    x = np.random.default_rng(S).standard_normal((S, 1, I)).astype(np.float32)
+    out = torch.full((S, 1, rows), 7.0, device="cuda")
+    Z.mul_mat_id(_place(W, offset), t, I, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), out=out)
+    got = out.cpu().numpy()[:, 0]
+    ok = (ids[:, 0] >= 0) & (ids[:, 0] < E)
+    assert not got[ids[:, 0] < 0].any() and np.isnan(got[ids[:, 0] >= E]).all()
+    ref = O.mul_mat_id(t, W, x, np.where(ok[:, None], ids, 0).astype(np.int32), nthreads=8)[:, 0]
+    for e in range(E):
+        m = ok & (ids[:, 0] == e)
+        if m.any():
+            bound = O.f32_matmul_absbound(t, W[e], x[m, 0])
+            err = np.abs(got[m].astype(np.float64) - ref[m])
+            assert (err <= TOL * bound + 1e-30).all(), (e, float((err / (bound + 1e-30)).max()))
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("I,rows", [(256, 16), (512, 37), (768, 130), (1280, 64), (1792, 1)])
+def test_bucket_and_row_edges(t, I, rows):
+    _check(t, I, rows, [1, 15, 16, 17, 31, 32, 33, 0, 2])                      # 32-pair items
+    _check(t, I, rows, [1, 16, 33, 47, 48, 49, 63, 64, 65, 129], extra=(-1, 10, 99))  # 64-pair items
+
+
+@pytest.mark.parametrize("t", [Q4, Q3, Q6, IQ2, IQ3, IQ4])
+@pytest.mark.parametrize("offset", [1, 2, 3, 4, 6])
+def test_weights_off_a_dword(t, offset):
+    """Odd row counts of 110-, 210-, 66- and 98-byte blocks put experts and rows
+    on either half of a dword; other alignments take the GEMV."""
+    _check(t, 768, 33, [20, 5, 40, 1], offset=offset)
+
+
+@pytest.mark.parametrize("pairs", [63, 64, 65])
+def test_smallest_pair_count(pairs):
+    _check(Q3, 512, 48, [pairs - 3, 2, 1])
+
+
+@pytest.mark.parametrize("tg,off_g,off_u", [(Q3, 0, 2), (Q3, 2, 2), (Q4, 0, 4), (Q4, 2, 0), (IQ2, 2, 0)])
+def test_gate_and_up_on_different_halves(tg, off_g, off_u):
+    """The layer with gate and up weights shifted against each other: bit-equal
+    where the same kernel runs, else within the re-quantization ties of the
+    layer bar (1e-3 of the token's largest output)."""
+    c = reduced(CONFIGS["c3"], tg=tg, td=Q4, S=48, H=512, F=256, E=8)
+    b = Built(c, seed=3)
+    x, lg = torch.from_numpy(b.x).cuda(), torch.from_numpy(b.logits).cuda()
+    ref = b.layer().forward(x, lg)[0].cpu().numpy()
+    b.wg = _place(b.wg.cpu().numpy(), off_g)
+    b.wu = _place(b.wu.cpu().numpy(), off_u)
+    out = b.layer().forward(x, lg)[0].cpu().numpy()
+    if off_g % 4 == off_u % 4 and off_g % (2 if tg != Q4 else 4) == 0:
+        np.testing.assert_array_equal(out, ref)
+    else:
+        slack = 1e-3 * np.abs(ref).max(axis=1, keepdims=True)
+        assert (np.abs(out - ref) <= 4 * slack).all()

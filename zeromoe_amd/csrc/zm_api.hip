@@ -260,77 +260,60 @@ int launch_gemv(int type, bool gateup, int np, const GemvArgs &a0, int n_groups,
   return 0;
 }
 
-// MFMA path for prefill-sized buckets: Q4_K, Q5_K, Q6_K, IQ2_XXS, IQ3_XXS and IQ4_XS weights with at least 8
-// pairs per active expert on average, Q2_K weights with at least 2.  a.items / a.n_items (or a.dense_S) must be set;
-// max_items bounds *a.n_items.  Returns 1 when the path does not apply (the
-// caller takes the GEMV path).
-bool mmq_applies(int type, double avg_pairs) {
-  return (((type == T_Q4_K || type == T_Q5_K || type == T_Q6_K || type == T_IQ4_XS || type == T_IQ2_XXS ||
-            type == T_IQ3_XXS) &&
-           avg_pairs >= 8.0) ||
-          (type == T_Q2_K && avg_pairs >= 2.0)) &&
-         !getenv_flag_off("ZEROMOE_MMQ");
+// ------------------------------------------------------------------ grouped MFMA dispatch
+
+// 16-pair tiles per work item: 64-pair items share the weight unpacking where
+// buckets are large, 32-pair items take fewer registers and less LDS.  512
+// tokens, Q4_K gate/up (32 pairs per expert): 260 against 289 us; 333 tokens
+// (21 pairs), Q3_K down: 155 against 126.
+int mmq_tiles(double avg_pairs) { return avg_pairs >= 32.0 ? 4 : 2; }
+// work items of n_pairs pairs over n_experts buckets: at most one partial run
+// per bucket besides the full ones
+int mmq_max_items(int n_pairs, int n_experts, int tok) {
+  return (n_pairs + tok - 1) / tok + std::min(n_pairs, n_experts);
 }
-// 16-token tiles per work item: routed buckets take 4 (the weight unpacking is
-// shared by 64 pairs); Q2_K (small buckets of resident slots) and dense
-// shared-expert rows 2
-int mmq_tt(int type, bool dense) { return type != T_Q2_K && !dense ? 4 : 2; }
-int launch_mmq(int type, bool gateup, const GemvArgs &a, int max_items, double avg_pairs, int tt, hipStream_t st,
-               int nw = 4);
-template <int T, int TT, int NW = 4>
-void launch_mmq_t(bool gateup, dim3 grid, const GemvArgs &a, hipStream_t st) {
-  grid.x = (unsigned)((a.nrows + 16 * NW - 1) / (16 * NW));  // NW waves of 16 weight rows per workgroup
-  if (gateup)
-    hipLaunchKernelGGL((k_mmq<T, true, TT, NW>), grid, dim3(64 * NW), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_mmq<T, false, TT, NW>), grid, dim3(64 * NW), 0, st, a);
+// Whether the grouped MFMA kernel takes this product (the caller then
+// quantizes the activations to records); the GEMV takes what is left.
+//   - rows, activations: 32-bit buffer offsets;
+//   - alignment: blocks of a multiple of 4 bytes are loaded by dwords, the
+//     others start on 2 bytes (gate and up alike within a dword);
+//   - pairs: below MMQ_MIN_PAIRS its workgroups are too few and too long.
+constexpr int MMQ_MIN_PAIRS = 64;
+bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride, int n_pairs,
+                 size_t xq_rows, int nb) {
+  if (n_pairs < MMQ_MIN_PAIRS || getenv_flag_off("ZEROMOE_MMQ")) return false;
+  if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
+  if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 32 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
+  const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
+  if (lo & (block_bytes(type) % 4 ? 1 : 3)) return false;
+  return !w1 || !(((uintptr_t)w0 ^ (uintptr_t)w1) & 3);
 }
-// tt: 16-token tiles per work item (the tiling the item list was cut with);
-// nw: waves (16 weight rows each) per workgroup -- 1 for a Q4_K matrix whose
-// 64-row tiles alone would leave most CUs idle (a dense shared expert)
-int launch_mmq(int type, bool gateup, const GemvArgs &a, int max_items, double avg_pairs, int tt, hipStream_t st,
-               int nw) {
-  if (!mmq_applies(type, avg_pairs)) return 1;
-  if ((size_t)a.nrows * a.w_rstride >= (1ull << 31) || max_items <= 0) return 1;
-  const dim3 grid((unsigned)((a.nrows + 63) / 64), (unsigned)max_items);
-  if (type == T_Q4_K) {
-    if (tt == 8) {
-      if (getenv_flag_off("ZEROMOE_MMQ_NW8")) launch_mmq_t<T_Q4_K, 8, 4>(gateup, grid, a, st);
-      else launch_mmq_t<T_Q4_K, 8, 8>(gateup, grid, a, st);
-    }
-    else if (tt == 4) launch_mmq_t<T_Q4_K, 4>(gateup, grid, a, st);
-    else if (nw == 1) launch_mmq_t<T_Q4_K, 2, 1>(gateup, grid, a, st);
-    else launch_mmq_t<T_Q4_K, 2>(gateup, grid, a, st);
-  } else if (type == T_Q5_K) {
-    if (tt == 4) launch_mmq_t<T_Q5_K, 4>(gateup, grid, a, st);
-    else launch_mmq_t<T_Q5_K, 2>(gateup, grid, a, st);
-  } else if (type == T_IQ4_XS || type == T_IQ3_XXS || type == T_IQ2_XXS) {
-    GemvArgs b = a;
-    if (device_table(type, &b.grid)) return -1;
-    if (type == T_IQ4_XS) {
-      if (tt == 4) launch_mmq_t<T_IQ4_XS, 4>(gateup, grid, b, st);
-      else launch_mmq_t<T_IQ4_XS, 2>(gateup, grid, b, st);
-    } else if (type == T_IQ3_XXS) {
-      if (tt == 4) launch_mmq_t<T_IQ3_XXS, 4>(gateup, grid, b, st);
-      else launch_mmq_t<T_IQ3_XXS, 2>(gateup, grid, b, st);
-    } else {
-      if (tt == 4) launch_mmq_t<T_IQ2_XXS, 4>(gateup, grid, b, st);
-      else launch_mmq_t<T_IQ2_XXS, 2>(gateup, grid, b, st);
-    }
-  } else if (type == T_Q6_K) {
-    if (tt == 4) launch_mmq_t<T_Q6_K, 4>(gateup, grid, a, st);
-    else launch_mmq_t<T_Q6_K, 2>(gateup, grid, a, st);
-  } else {
-    if (tt == 4) launch_mmq_t<T_Q2_K, 4>(gateup, grid, a, st);
-    else launch_mmq_t<T_Q2_K, 2>(gateup, grid, a, st);
-  }
+// tt: 16-pair tiles per item (the list's); items: bound of *a.n_items (or the
+// exact count of a dense product); nw = 1: one-wave workgroups (tt == 2 only)
+int launch_mmq(int type, bool gateup, int tt, int nw, int items, const GemvArgs &a0, hipStream_t st) {
+  GemvArgs a = a0;
+  if ((type == T_IQ4_XS || type == T_IQ3_XXS || type == T_IQ2_XXS) && device_table(type, &a.grid)) return -1;
+  const unsigned n = (unsigned)items;
+  if (!mmq_launch_a(type, gateup, tt, nw, n, a, st) && !mmq_launch_b(type, gateup, tt, nw, n, a, st) &&
+      !mmq_launch_c(type, gateup, tt, nw, n, a, st) && !mmq_launch_d(type, gateup, tt, nw, n, a, st))
+    return fail("unsupported weight type %d", type);
   HIP_OK(hipGetLastError());
   return 0;
 }
-int mmq_max_items(int n_pairs, int n_experts) {
-  return (n_pairs + MMQ_TOK - 1) / MMQ_TOK + std::min(n_pairs, n_experts);
+void launch_items(const int32_t *n_active, const int32_t *active, const int32_t *offs, int32_t *items,
+                  int32_t *n_items, int tt, hipStream_t st) {
+  hipLaunchKernelGGL(k_mmq_items, dim3(1), dim3(1024), 0, st, n_active, active, offs, items, n_items, 16 * tt);
 }
 
+// records for the grouped MFMA kernel, value order of `type`
+int launch_quant_rec(const float *x, size_t x_rstride, int nb, int rows, uint8_t *y, int type, hipStream_t st) {
+  if (rows <= 0) return 0;
+  const long blocks = (long)rows * nb;  // 16 per workgroup
+  hipLaunchKernelGGL(k_quant_rec, dim3((unsigned)((blocks + 15) / 16)), dim3(256), 0, st, x, x_rstride, nb, rows, y,
+                     xrec_row_bytes(nb), mmq_order(type));
+  HIP_OK(hipGetLastError());
+  return 0;
+}
 int launch_quant(const float *x, size_t x_rstride, int nb, int rows, uint8_t *y, size_t y_rstride, int planar,
                  hipStream_t st) {
   if (rows <= 0) return 0;
@@ -455,14 +438,14 @@ struct MmidWs {
 size_t mmid_carve(const MmidShape &m, uint8_t *base, MmidWs *out) {
   Bump b{base};
   MmidWs w{};
-  w.xq = b.take<uint8_t>((size_t)m.nq * q8_row_bytes(m.nb));
+  w.xq = b.take<uint8_t>((size_t)m.nq * xrec_row_bytes(m.nb));  // planar rows are smaller
   w.idc = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.counts = b.take<int32_t>((size_t)m.E * 4);
   w.offs = b.take<int32_t>((size_t)(m.E + 1) * 4);
   w.pairs = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.active = b.take<int32_t>((size_t)m.E * 4);
   w.n_active = b.take<int32_t>(4);
-  w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E) * 4);
+  w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 32) * 4);
   w.n_items = b.take<int32_t>(4);
   if (out) *out = w;
   return b.off + 256;
@@ -508,16 +491,18 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
   const int64_t S = m.S, n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
-  // 1. quantize src1 rows (token t, row i11) -> planar Q8_K row t*ne11 + i11
+  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
+  // 1. quantize src1 rows: (token t, row i11) -> row t*ne11 + i11
+  const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
+  auto quant = [&](const float *xt, int rows, uint8_t *y) {
+    return mmq ? launch_quant_rec(xt, x->nb[1] / 4, nb, rows, y, w->type, st)
+               : launch_quant(xt, x->nb[1] / 4, nb, rows, y, xrow, 1, st);
+  };
   if (x->nb[2] == (size_t)ne11 * x->nb[1]) {
-    if (launch_quant((const float *)x->data, x->nb[1] / 4, nb, (int)nq, b.xq, q8_row_bytes(nb), 1, st)) return 0;
+    if (quant((const float *)x->data, (int)nq, b.xq)) return 0;
   } else {
-    for (int64_t t = 0; t < S; ++t) {
-      const float *xt = (const float *)((const char *)x->data + t * x->nb[2]);
-      if (launch_quant(xt, x->nb[1] / 4, nb, ne11, b.xq + (size_t)t * ne11 * q8_row_bytes(nb), q8_row_bytes(nb), 1,
-                       st))
-        return 0;
-    }
+    for (int64_t t = 0; t < S; ++t)
+      if (quant((const float *)((const char *)x->data + t * x->nb[2]), ne11, b.xq + (size_t)t * ne11 * xrow)) return 0;
   }
   // 2. ids -> contiguous [S][n_ids] (strided copy), then bucket
   if (ids->nb[1] == (size_t)n_ids * 4) {
@@ -544,7 +529,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   a.nrows = (int)O;
   a.nb = nb;
   a.xq = b.xq;
-  a.xq_rstride = q8_row_bytes(nb);
+  a.xq_rstride = xrow;
   a.ne11 = ne11;
   a.K = (int)n_ids;
   a.n_active = b.n_active;
@@ -557,17 +542,15 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   a.grid = d->grid;
   a.signs = d->signs;
   const int groups = (int)std::min<int64_t>(E, n_pairs);
-  {
-    // the MFMA path addresses the activations through a 32-bit buffer offset
-    const double avg = (size_t)nq * q8_row_bytes(nb) < (1ull << 31) ? (double)n_pairs / groups : 0.0;
-    if (mmq_applies(w->type, avg))
-      hipLaunchKernelGGL(k_mmq_items, dim3(1), dim3(1024), 0, st, b.n_active, b.active, b.offs, b.items, b.n_items,
-                         16 * mmq_tt(w->type, false));
+  if (mmq) {
+    const int tt = mmq_tiles((double)n_pairs / groups);
+    launch_items(b.n_active, b.active, b.offs, b.items, b.n_items, tt, st);
     a.items = b.items;
     a.n_items = b.n_items;
-    a.xq_bytes = (uint32_t)((size_t)nq * q8_row_bytes(nb));
-    const int rc = launch_mmq(w->type, false, a, mmq_max_items((int)n_pairs, (int)E), avg, mmq_tt(w->type, false), st);
-    if (rc < 0 || (rc > 0 && launch_gemv(w->type, false, pick_np((int)n_pairs, (int)E), a, groups, st))) return 0;
+    a.xq_bytes = (uint32_t)((size_t)nq * xrow);
+    if (launch_mmq(w->type, false, tt, 4, mmq_max_items((int)n_pairs, (int)E, 16 * tt), a, st)) return 0;
+  } else if (launch_gemv(w->type, false, pick_np((int)n_pairs, (int)E), a, groups, st)) {
+    return 0;
   }
   count_mmid_launch();
   return hipPeekAtLastError() == hipSuccess ? 1 : 0;
@@ -769,12 +752,11 @@ struct LayerWs {
   uint8_t *aq;
   float *y;
   float *act_s;
-  uint8_t *aq_s;
+  uint8_t *xq_s, *aq_s;
   float *y_s;
   float *f_act;
   uint32_t *f_sync;
-  int32_t *items, *n_items;    // MFMA work items of the gate/up launch
-  int32_t *items2, *n_items2;  // and of the down launch when its tiling differs
+  int32_t *items, *n_items;  // MFMA work items
 };
 
 size_t layer_ws(const zm_moe_layer *L, int S, uint8_t *base, LayerWs *w) {
@@ -785,22 +767,21 @@ size_t layer_ws(const zm_moe_layer *L, int S, uint8_t *base, LayerWs *w) {
   t.logits = b.take<float>((size_t)S * E * 4);
   t.ids = b.take<int32_t>((size_t)S * K * 4);
   t.weights = b.take<float>((size_t)S * K * 4);
-  t.xq = b.take<uint8_t>((size_t)S * q8_row_bytes(nbH));
+  t.xq = b.take<uint8_t>((size_t)S * xrec_row_bytes(nbH));  // records; planar rows are smaller
   t.counts = b.take<int32_t>((size_t)NS * 4);
   t.offs = b.take<int32_t>((size_t)(NS + 1) * 4);
   t.pairs = b.take<int32_t>((size_t)S * K * 4);
   t.active = b.take<int32_t>((size_t)NS * 4);
   t.n_active = b.take<int32_t>(4);
-  t.items = b.take<int32_t>((size_t)mmq_max_items(S * K, NS) * 4);
+  t.items = b.take<int32_t>((size_t)mmq_max_items(S * K, NS, 32) * 4);
   t.n_items = b.take<int32_t>(4);
-  t.items2 = b.take<int32_t>((size_t)mmq_max_items(S * K, NS) * 4);
-  t.n_items2 = b.take<int32_t>(4);
   t.act = b.take<float>((size_t)S * K * F * 4);
-  t.aq = b.take<uint8_t>((size_t)S * K * q8_row_bytes(nbF));
+  t.aq = b.take<uint8_t>((size_t)S * K * xrec_row_bytes(nbF));
   t.y = b.take<float>((size_t)S * K * H * 4);
   if (L->F_shared > 0) {
     t.act_s = b.take<float>((size_t)S * L->F_shared * 4);
-    t.aq_s = b.take<uint8_t>((size_t)S * q8_row_bytes(L->F_shared / QK));
+    t.xq_s = b.take<uint8_t>((size_t)S * xrec_row_bytes(nbH));
+    t.aq_s = b.take<uint8_t>((size_t)S * xrec_row_bytes(L->F_shared / QK));
     t.y_s = b.take<float>((size_t)S * H * 4);
   }
   // fused decode: act rows of every pair then the shared rows, their Q8_K
@@ -1046,23 +1027,38 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   }
   if (zm_router(&L->router, lg, L->logit_bias, L->sel_bias, L->route_map, L->route_mask, S, ids, wts, st))
     return -1;
-  // activations -> Q8_K, buckets
-  if (launch_quant(x, (size_t)H, nbH, S, w.xq, q8_row_bytes(nbH), 1, st)) return -1;
+  // activations -> Q8_K rows: records for the grouped MFMA kernel, planar rows for the GEMV
+  const size_t g_row = row_bytes(L->type_gate, H), d_row = row_bytes(L->type_down, F);
+  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, S * K, (size_t)S, nbH);
+  const bool mmq_d = mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, S * K, (size_t)S * K, nbF);
+  auto quant = [&](bool rec, int type, const float *v, int n, int rows, uint8_t *y, hipStream_t q) {
+    return rec ? launch_quant_rec(v, (size_t)n, n / QK, rows, y, type, q)
+               : launch_quant(v, (size_t)n, n / QK, rows, y, q8_row_bytes(n / QK), 1, q);
+  };
+  auto qrow = [](bool rec, int nb) { return rec ? xrec_row_bytes(nb) : q8_row_bytes(nb); };
+  if (quant(mmq_g, L->type_gate, x, H, S, w.xq, st)) return -1;
   // shared expert (dense over all tokens) on the side stream: it needs only
   // the Q8_K rows of x, and its gate/up, act quantization and down overlap
   // the router-dependent kernels; the combine waits for it
   auto launch_shared = [&](hipStream_t ss) -> int {
-    const int Fs = L->F_shared, nbS = Fs / QK;
+    const int ts = L->type_shared, Fs = L->F_shared, nbS = Fs / QK;
+    const size_t gr = row_bytes(ts, H), dr = row_bytes(ts, Fs);
+    // one bucket of S pairs; from 8 tokens on (as the pairs of a bucket, not of a batch)
+    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MIN_PAIRS, (size_t)S, nbH);
+    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MIN_PAIRS, (size_t)S, nbS);
+    // x in the layout of this type: the routed experts' rows where they are the same
+    const bool same = mg == mmq_g && (!mg || mmq_order(ts) == mmq_order(L->type_gate));
+    if (!same && quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;
     GemvArgs c{};
     c.w0 = (const uint8_t *)L->ws_gate;
     c.w1 = (const uint8_t *)L->ws_up;
-    c.w_rstride = row_bytes(L->type_shared, H);
+    c.w_rstride = gr;
     c.w_estride = 0;
     c.nrows = Fs;
     c.nb = nbH;
-    c.xq = w.xq;
-    c.xq_rstride = q8_row_bytes(nbH);
-    c.xq_bytes = (uint32_t)((size_t)S * q8_row_bytes(nbH));
+    c.xq = same ? w.xq : w.xq_s;
+    c.xq_rstride = qrow(mg, nbH);
+    c.xq_bytes = (uint32_t)((size_t)S * c.xq_rstride);
     c.ne11 = 1;
     c.K = 1;
     c.dense_S = S;
@@ -1072,31 +1068,29 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     c.grid = d->grid;
     c.signs = d->signs;
     const int nps = S >= 4 ? 4 : (S >= 2 ? 2 : 1);
-    {
-      // 64-row tiles of the shared expert's F rows times (S / 32) items: a
-      // one-wave workgroup per 16 rows when that leaves CUs idle
-      const int cus = d->n_cu > 0 ? d->n_cu : 256;
-      const int nw = (long)((Fs + 63) / 64) * ((S + 31) / 32) < cus ? 1 : 4;
-      const int rc = launch_mmq(L->type_shared, true, c, (S + 31) / 32, (double)S, 2, ss, nw);
-      if (rc < 0 || (rc > 0 && launch_gemv(L->type_shared, true, nps, c, 1, ss))) return -1;
-    }
-    if (launch_quant(w.act_s, (size_t)Fs, nbS, S, w.aq_s, q8_row_bytes(nbS), 1, ss)) return -1;
+    const int tt = mmq_tiles((double)S);
+    // one-wave workgroups of 16 rows where 64-row tiles of 32 tokens would leave CUs idle
+    const int cus = d->n_cu > 0 ? d->n_cu : 256;
+    auto dense = [&](bool mmq, bool gu, const GemvArgs &v) {
+      const bool few = (long)((v.nrows + 63) / 64) * ((S + 31) / 32) < cus;
+      const int t = few ? 2 : tt;
+      return mmq ? launch_mmq(ts, gu, t, few ? 1 : 4, (S + 16 * t - 1) / (16 * t), v, ss)
+                 : launch_gemv(ts, gu, nps, v, 1, ss);
+    };
+    if (dense(mg, true, c)) return -1;
+    if (quant(md, ts, w.act_s, Fs, S, w.aq_s, ss)) return -1;
     GemvArgs e2 = c;
     e2.w0 = (const uint8_t *)L->ws_down;
     e2.w1 = nullptr;
-    e2.w_rstride = row_bytes(L->type_shared, Fs);
+    e2.w_rstride = dr;
     e2.nrows = H;
     e2.nb = nbS;
     e2.xq = w.aq_s;
-    e2.xq_rstride = q8_row_bytes(nbS);
-    e2.xq_bytes = (uint32_t)((size_t)S * q8_row_bytes(nbS));
+    e2.xq_rstride = qrow(md, nbS);
+    e2.xq_bytes = (uint32_t)((size_t)S * e2.xq_rstride);
     e2.out = w.y_s;
     e2.out_s = H;
-    {
-      const int rc = launch_mmq(L->type_shared, false, e2, (S + 31) / 32, (double)S, 2, ss);
-      if (rc < 0 || (rc > 0 && launch_gemv(L->type_shared, false, nps, e2, 1, ss))) return -1;
-    }
-    return 0;
+    return dense(md, false, e2) ? -1 : 0;
   };
   std::unique_lock<std::mutex> fork_lk;
   if (L->F_shared > 0) {
@@ -1114,12 +1108,13 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   GemvArgs a{};
   a.w0 = (const uint8_t *)L->w_gate;
   a.w1 = (const uint8_t *)L->w_up;
-  a.w_rstride = row_bytes(L->type_gate, H);
-  a.w_estride = a.w_rstride * F;
+  a.w_rstride = g_row;
+  a.w_estride = g_row * F;
   a.nrows = F;
   a.nb = nbH;
   a.xq = w.xq;
-  a.xq_rstride = q8_row_bytes(nbH);
+  a.xq_rstride = qrow(mmq_g, nbH);
+  a.xq_bytes = (uint32_t)((size_t)S * a.xq_rstride);
   a.ne11 = 1;
   a.K = K;
   a.n_active = w.n_active;
@@ -1131,36 +1126,16 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   a.out_k = F;
   a.grid = d->grid;
   a.signs = d->signs;
-  const double avg_pairs = (double)(S * K) / std::max(1, std::min(NS, S * K));
-  // 16-token tiles per routed work item, per projection (mmq_tt); gate/up and
-  // down take separate item lists when their tilings differ
-  int tt_g = mmq_tt(L->type_gate, false), tt_d = mmq_tt(L->type_down, false);
-  // items: at most one partial run per active expert plus the full runs
-  auto max_items_for = [&](int tt) {
-    return std::min(mmq_max_items(S * K, NS), (S * K + 16 * tt - 1) / (16 * tt) + std::min(NS, S * K));
-  };
-  auto cut_items = [&](int tt, int32_t *items, int32_t *n_items) {
-    if (getenv_flag_off("ZEROMOE_MMQ_LPT") || NS > 1024)
-      hipLaunchKernelGGL(k_mmq_items, dim3(1), dim3(1024), 0, st, w.n_active, w.active, w.offs, items, n_items,
-                         16 * tt);
-    else
-      hipLaunchKernelGGL(k_mmq_items_lpt, dim3(1), dim3(1024), 0, st, w.n_active, w.active, w.offs, items, n_items,
-                         16 * tt);
-  };
-  const bool mmq_g = mmq_applies(L->type_gate, avg_pairs), mmq_d = mmq_applies(L->type_down, avg_pairs);
-  const bool split_items = mmq_g && mmq_d && tt_d != tt_g;
-  if (!mmq_g && mmq_d) tt_g = tt_d;  // one list, cut for the down launch
-  if (mmq_g || mmq_d) cut_items(tt_g, w.items, w.n_items);
-  if (split_items) cut_items(tt_d, w.items2, w.n_items2);
+  const int tt = mmq_tiles((double)(S * K) / groups);
+  const int max_items = mmq_max_items(S * K, NS, 16 * tt);
+  if (mmq_g || mmq_d) launch_items(w.n_active, w.active, w.offs, w.items, w.n_items, tt, st);
   a.items = w.items;
   a.n_items = w.n_items;
-  a.xq_bytes = (uint32_t)((size_t)S * q8_row_bytes(nbH));
-  {
-    const int rc = launch_mmq(L->type_gate, true, a, max_items_for(tt_g), avg_pairs, tt_g, st);
-    if (rc < 0 || (rc > 0 && launch_gemv(L->type_gate, true, np, a, groups, st))) return -1;
-  }
+  if (mmq_g ? launch_mmq(L->type_gate, true, tt, 4, max_items, a, st)
+            : launch_gemv(L->type_gate, true, np, a, groups, st))
+    return -1;
   // act -> Q8_K
-  if (launch_quant(w.act, (size_t)F, nbF, S * K, w.aq, q8_row_bytes(nbF), 1, st)) return -1;
+  if (quant(mmq_d, L->type_down, w.act, F, S * K, w.aq, st)) return -1;
   // skipped routes (slot table -1) read as zero rows; router ids are always valid otherwise
   if (L->route_map)
     hipLaunchKernelGGL(k_fill_skipped, dim3((unsigned)std::min((H + 255) / 256, 64), (unsigned)std::min(S * K, 65535)), dim3(256), 0,
@@ -1169,27 +1144,20 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   GemvArgs b = a;
   b.w0 = (const uint8_t *)L->w_down;
   b.w1 = nullptr;
-  b.w_rstride = row_bytes(L->type_down, F);
-  b.w_estride = b.w_rstride * H;
+  b.w_rstride = d_row;
+  b.w_estride = d_row * H;
   b.nrows = H;
   b.nb = nbF;
   b.xq = w.aq;
-  b.xq_rstride = q8_row_bytes(nbF);
-  b.xq_bytes = (uint32_t)((size_t)S * K * q8_row_bytes(nbF));
+  b.xq_rstride = qrow(mmq_d, nbF);
+  b.xq_bytes = (uint32_t)((size_t)S * K * b.xq_rstride);
   b.ne11 = K;
   b.out = w.y;
   b.out_s = (size_t)K * H;
   b.out_k = H;
-  if (split_items) {
-    b.items = w.items2;
-    b.n_items = w.n_items2;
-  } else {
-    tt_d = tt_g;
-  }
-  {
-    const int rc = launch_mmq(L->type_down, false, b, max_items_for(tt_d), avg_pairs, tt_d, st);
-    if (rc < 0 || (rc > 0 && launch_gemv(L->type_down, false, np, b, groups, st))) return -1;
-  }
+  if (mmq_d ? launch_mmq(L->type_down, false, tt, 4, max_items, b, st)
+            : launch_gemv(L->type_down, false, np, b, groups, st))
+    return -1;
   if (L->F_shared > 0) HIP_OK(hipStreamWaitEvent(st, d->ev_join, 0));  // the shared expert's y_s
   const float *ys = L->F_shared > 0 ? w.y_s : nullptr;
   if ((uintptr_t)out & 15)

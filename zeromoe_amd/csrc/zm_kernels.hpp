@@ -626,8 +626,9 @@ struct GemvArgs {
   int tile_rows;
   const uint64_t *grid;   // IQ2_XXS / IQ3_XXS grid or IQ4_XS value table (global), staged into LDS
   const uint64_t *signs;
-  // int8-MFMA path: (expert, first pair) work items of up to 32 pairs each
+  // int8-MFMA path: (expert, first pair) work items, row tiles per item
   const int32_t *items, *n_items;
+  int row_tiles;
   uint32_t xq_bytes;  // extent of the xq buffer
 };
 

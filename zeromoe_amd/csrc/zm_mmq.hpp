@@ -1,67 +1,61 @@
-// zm_mmq.hpp -- bucketed MUL_MAT_ID for prefill-sized buckets on int8 MFMA.
+// zm_mmq.hpp -- bucketed MUL_MAT_ID for batches and prefill on int8 MFMA.
 //
 // Per active expert, out[pair][row] = W_e[row] . q8(x[pair]) for the pairs of
 // the expert's bucket (the CSR of /root/reference/core/batched_dispatch_pipeline.cpp:1181-1202),
 // gate/up optionally fused with SwiGLU (moe_routed_ggml.hpp:166-191).
 //
-// Tile: one wave computes 16 tokens x 16 weight rows with
-// v_mfma_i32_16x16x64_i8, tokens as the A operand and weight rows as the B
-// operand, so every lane's four outputs belong to ONE weight row (lane % 16)
-// and every lane's 16 B-operand bytes to one 32-weight sub-block of that row,
-// whose 6-bit scale sc = 8*hi + lo the lane has decoded itself.  The scale is
-// folded into the weights: the lane multiplies its nibbles by lo and by hi
-// (products <= 105, int8), and two MFMA chains accumulate over the block:
-//   isum[t][r] = D_lo + 8 * D_hi = sum_sb sc[r][sb] * (q[r] . x[t])_sb  (int32, exact)
-//   mn[t][r]   = sum_sb bsum[t][sb] * (-dmin[r] * m[r][sb])   (v_mfma_f32_16x16x4f32;
-//                -dmin * m is exact in fp32, so mn is -dmin * imin to fp32 rounding)
-//   f[t][r]   += d_x[t] * (d[r] * isum + mn)  (ggml's vec_dot_q4_K_q8_K combine)
-// Q4_K / Q5_K K order of a 64-weight chunk i (qs group i, bytes 32i..32i+31,
-// holding sub-block 2i in its low nibbles and 2i + 1 in its high nibbles):
-// k-group g holds bytes 8g..8g+7 of the group, low nibbles then high nibbles,
-// i.e. weights 64i + 8g .. +7 and 64i + 32 + 8g .. +7, so every qs byte is
-// loaded by one lane only (Q5_K: the fifth bits are bits 2i, 2i + 1 of the
-// lane's qh bytes 8g..8g+7); the activation operand is read in the same order
-// (two 8-byte LDS reads).  The weight unpacking is done once per block for all
-// token tiles of the work item.  No dequantized weight copy is materialized.
-// Activations reach LDS by direct buffer-to-LDS loads (no register staging),
-// token rows XOR-swizzled in 16-byte chunks by the token index.
+// Work split.  A work item is a run of up to 16 * TT pairs of one bucket; a
+// workgroup takes one item and 16 * NW weight rows, a wave 16 of them.  K runs
+// in super-blocks of 256.  Per block a wave unpacks its 16 rows (gate, then up)
+// once and dots them with the item's 16-pair tiles on v_mfma_i32_16x16x64_i8
+// (or 16x16x32): pairs are the A operand, weight rows the B operand, so a
+// lane's four outputs belong to ONE weight row (lane % 16) and the per-row
+// scales are per-lane values.  The K loop is instantiated per tile count of the
+// item, so it has no branch per tile.
 //
-// IQ2_XXS / IQ3_XXS (grid values up to 43 / 62 with per-8-weight signs, and a
-// (2 ls + 1) <= 31 scale per 32-weight sub-block) dot each sub-block on its own
-// v_mfma_i32_16x16x32_i8 (K = the sub-block; lane group g holds its 8-weight
-// group g): signed grid bytes from the LDS-staged grid and sign masks, scales
-// per lane on the integer results.
+// What bounds it, and the layout that follows.  Loading each lane's few bytes
+// of its row straight into registers (16 rows per instruction, 8-16 bytes
+// each) kept the vector memory unit busy with addresses: without the weight
+// loads the Q4_K gate/up product of 512 tokens (4096 x 1536, 128 experts) took
+// 204 us instead of 341, and with loads that always hit the cache 295.  So
+// weights come in as they lie in memory: a row's block as consecutive 16-byte
+// units, 64 units per direct buffer-to-LDS load, into a slot private to the
+// wave, and the lanes pick their fields out of LDS.  The slot is read at the
+// start of a block and its next block requested at once, so a request has the
+// whole block's arithmetic to land.  Activations are staged the same way, one
+// 304-byte record per pair and block (ST stages, one barrier per block).
+// Units per row are odd (Q6_K padded), and so is a record, counted in 16-byte
+// units: 16 rows read 16 different bank groups.
+// On the vector units the unpacking and the tile epilogue (about 100 + 25 per
+// tile instructions per matrix and block for Q4_K) are the floor at many pairs
+// per expert, the weight stream at few.
+//   512 tokens, Q4_K, skewed loads: gate/up 367 -> 280 us, down 185 -> 142 us
+//   333 tokens, even loads: Q2_K gate/up 230 -> 167 us; Q3_K down 888 (GEMV) -> 142 us
+//   24 tokens, Q4_K gate/up: 207 (GEMV) -> 144 us, 4.9 TB/s of weights
 //
-// IQ4_XS (a 16-entry value table, up to |127|, and a 6-bit signed scale per
-// 32-weight sub-block) dots each 64-weight chunk as its two sub-blocks on
-// v_mfma_i32_16x16x64_i8 with half of B zeroed, values looked up from the
-// table in registers; the scales apply per lane as for Q6_K, no min term.
+// Activation record of one 256-value block (k_quant_rec): 256 int8 | 16 f16
+// sums of 16 values (integers up to 2032: exact) | f32 d | pad.  The int8 of a
+// 64-value chunk are ordered so that k-group g of an MFMA operand is 16
+// consecutive bytes: natural order for Q2_K / Q3_K, else the 8-byte group g of
+// the chunk's first 32 values, then that of its second 32.
 //
-// Q5_K adds the fifth bit of each value as a third chain: the bit (0/1) times
-// the whole 6-bit scale (<= 63) is int8 too, and isum = D_lo + 8 D_hi + 16 D_5.
-//
-// Q2_K uses v_mfma_i32_16x16x64_i8 with the 4-bit sub-block scale folded into
-// the weights (q * sc <= 45 fits int8): lane (row n, k-group g) of 64-weight
-// chunk c = 2h + jp holds bit-plane j = 2jp + (g >> 1) of qs bytes
-// 32h + 16(g & 1) .. +15, i.e. weights 64c + 16g .. +15 of sub-block
-// 8h + 2j + (g & 1), each byte multiplied by that sub-block's scale; one MFMA
-// chain over the 4 chunks gives isum = sum_sb sc * (q . x)_sb exactly, the
-// mins term sum_sb (-dmin * m) * bsum16 goes through four v_mfma_f32_16x16x4f32
-// (K = 16 sub-blocks), and f += d_x * (d * isum + mn) (ggml's vec_dot_q2_K_q8_K).  Activations are the planar Q8_K rows of the decode
-// path (qs | bsums | d).
-//
-// Q6_K (a 6-bit value and a signed 8-bit scale per 16-weight sub-block: the
-// product does not fit int8) keeps the scales out of the weights and uses
-// v_mfma_i32_16x16x32_i8, whose K = 32 spans two sub-blocks (lane groups 0-1
-// and 2-3): each pair of sub-blocks is issued twice with the other half of
-// the B operand zeroed, giving one exact 16x16 integer dot per sub-block,
-// scaled per lane (a lane's outputs share one weight row) and summed:
-//   isum[t][r] = sum_sb sc[r][sb] * (q[r] . x[t])_sb            (q = 0..63)
-//   off[t][r]  = sum_sb sc[r][sb] * bsum16[t][sb]               (v_mfma_f32_16x16x4f32, exact)
-//   f[t][r]   += d_x[t] * d[r] * (isum - 32 * off)   (the value is q - 32; ggml's vec_dot_q6_K_q8_K)
-// Lane (row n, group g) of sub-block pair p holds weights 32p + 8g .. +7:
-// low (p & 3 < 2) or high nibbles of ql bytes 64(p >> 2) + 32(p & 1) + 8g .. +7,
-// top bits 2(p & 3) of qh bytes 32(p >> 2) + 8g .. +7.
+// Per type (lane = row n = lane % 16, k-group g = lane / 16):
+// Q4_K, Q5_K: the 6-bit sub-block scale sc = 8*hi + lo is folded into the
+//   weights (nibble * lo and nibble * hi <= 105: int8), two chains over the
+//   block give isum = D_lo + 8 D_hi = sum_sb sc * (q . x)_sb exactly; Q5_K's
+//   fifth bit is a third chain with the whole scale, + 16 D_5.
+// Q2_K: q * sc <= 45, one chain.
+// Q3_K: (4 - q') * sc (q' = 0..7 the quant with its high bit, sc = -32..31) lies in
+//   -128..124: one byte permute on an 8-entry table of the scale per 4 weights
+//   (tables of all 64 scales in LDS), one chain, isum = -D.
+// Their mins: imin = sum_sb m * bsum (f16 operands, exact f32 sums) on one
+//   v_mfma_f32_16x16x16_f16 (16 cycles; on f32 operands it took 2 to 4 of 32).
+//   f += d_x * (d * isum - dmin * imin), ggml's vec_dot combine.
+// Q6_K (signed 8-bit scale per 16 weights; 4 * (q - 32) is int8): one
+//   v_mfma_i32_16x16x32_i8 per 16-weight sub-block (half of B zeroed), scaled
+//   per lane on the integer sums.
+// IQ2_XXS, IQ3_XXS, IQ4_XS (grid or table values, one scale per 32 weights): one
+//   v_mfma_i32_16x16x32_i8 per sub-block, scaled per lane.
 #pragma once
 
 #include "zm_kernels.hpp"
@@ -70,15 +64,16 @@ namespace zm {
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
+typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
 typedef unsigned short v2u16_t __attribute__((ext_vector_type(2)));
-typedef short v2i16_t __attribute__((ext_vector_type(2)));
 typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
 
-// buffer-to-LDS loads (lane L's `bytes` land at lds + bytes * L; out-of-range
-// lanes write zeros) issued as inline asm: the compiler's wait insertion does not
-// track them, so the reads of the other LDS buffer are not held behind them.
-// The caller waits for them itself (vmcnt(0)) before the barrier that publishes
-// the buffer.
+// ---------------------------------------------------------------- buffer-to-LDS loads
+//
+// Lane L's 16 bytes land at lds + 16 * L (inactive lanes write nothing,
+// out-of-range dwords write zeros).  Inline asm: the compiler's wait insertion
+// does not track them, so the caller counts them and waits itself.
 __device__ __forceinline__ v4u_t dma_rsrc(const void *p, uint32_t bytes) {
   const uint64_t a = (uint64_t)(uintptr_t)p;
   return v4u_t{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
@@ -88,19 +83,47 @@ __device__ __forceinline__ uint32_t lds_addr(const void *p) {
 }
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is written by the asm and by nothing else here
-__device__ __forceinline__ void dma_lds16(v4u_t rs, uint32_t lds, int vo) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+__device__ __forceinline__ void dma_lds16(v4u_t rs, uint32_t lds, int vo, int so) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :
-               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(vo), "s"(rs)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void dma_lds4(v4u_t rs, uint32_t lds, int vo) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(vo), "s"(rs)
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(vo), "s"(rs), "s"(so)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop
+// at most N vector memory operations of this wave outstanding
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// the same, then the workgroup barrier (this wave's LDS reads are complete)
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <class P>
+__device__ __forceinline__ P lds_get(const uint8_t *p) {
+  return *reinterpret_cast<const P *>(p);
+}
+// N dwords that start 0, 2 or 4 bytes past the dword p: N + 1 aligned dwords and
+// one byte permute each (sel: align_sel).  LDS reads at the 2-byte address itself
+// are correct but stall: a third of the Q6_K kernel's LDS time.
+template <int N>
+struct Dwords {
+  uint32_t v[N];
+};
+template <int N, int A>
+__device__ __forceinline__ Dwords<N> lds_get_at(const uint8_t *p, uint32_t sel) {
+  uint32_t r[N + 1];
+  __builtin_memcpy(r, __builtin_assume_aligned(p, A), 4 * N);
+  r[N] = lds_get<uint32_t>(p + 4 * N);
+  Dwords<N> o;
+#pragma unroll
+  for (int i = 0; i < N; ++i) o.v[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
+  return o;
+}
+__device__ __forceinline__ uint32_t align_sel(int bytes) { return 0x03020100u + 0x01010101u * (uint32_t)bytes; }
 
 // four packed bytes times a small factor, bytewise (every product < 256: no
 // carry crosses a byte): one packed 16-bit multiply
@@ -109,48 +132,64 @@ __device__ __forceinline__ uint32_t mul_bytes(uint32_t packed, uint32_t f) {
   const v2u16_t m = {(unsigned short)f, (unsigned short)f};
   return __builtin_bit_cast(uint32_t, p * m);
 }
-
-constexpr int MMQ_TOK = 32;            // pairs per work item of the 2-tile kernels (item count bound)
-
-
-// Work items: every active expert's bucket cut into runs of `tok` pairs,
-// item = expert | (first pair offset within the bucket) << 12.  One workgroup.
-__global__ __launch_bounds__(1024) void k_mmq_items(const int32_t *__restrict__ n_active,
-                                                    const int32_t *__restrict__ active,
-                                                    const int32_t *__restrict__ offs, int32_t *__restrict__ items,
-                                                    int32_t *__restrict__ n_items, int tok) {
-  __shared__ int s_n[1024];
-  const int na = *n_active;
-  int total = 0;
-  for (int base = 0; base < na; base += 1024) {
-    const int i = base + (int)threadIdx.x;
-    const int e = i < na ? active[i] : 0;
-    const int np = i < na ? (offs[e + 1] - offs[e] + tok - 1) / tok : 0;
-    s_n[threadIdx.x] = np;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {  // inclusive scan
-      const int v = threadIdx.x >= (unsigned)d ? s_n[threadIdx.x - d] : 0;
-      __syncthreads();
-      s_n[threadIdx.x] += v;
-      __syncthreads();
-    }
-    const int start = total + s_n[threadIdx.x] - np;
-    for (int q = 0; q < np; ++q) items[start + q] = e | ((q * tok) << 12);
-    total += s_n[1023];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *n_items = total;
+// two bytes of w, picked into 16-bit halves by the permute selector, as f16 (1024 + b, less 1024)
+__device__ __forceinline__ v2h_t bytes_f16(uint32_t w, uint32_t sel) {
+  const uint32_t u = __builtin_amdgcn_perm(0, w, sel) | 0x64006400u;
+  return __builtin_bit_cast(v2h_t, u) - v2h_t{(_Float16)1024.f, (_Float16)1024.f};
 }
 
-// The same work items, largest first: full runs of `tok` pairs, then every
-// expert's remaining run in descending order of its 16-pair tiles, so the
+// ---------------------------------------------------------------- activation records
+
+constexpr int XREC = 304;           // bytes of one block's record
+constexpr int XUNITS = XREC / 16;   // 19
+__host__ __device__ constexpr size_t xrec_row_bytes(int nb) { return (size_t)nb * XREC; }
+// value order of a record's int8: 0 natural, 1 the 8-byte groups of the two 32-value halves of a chunk alternating
+__host__ __device__ constexpr int mmq_order(int type) { return type == T_Q2_K || type == T_Q3_K ? 0 : 1; }
+
+// f32 rows -> records, 16 lanes per block
+static __global__ __launch_bounds__(256) void k_quant_rec(const float *__restrict__ x, size_t x_rstride, int nb,
+                                                          int rows, uint8_t *__restrict__ y, size_t y_rstride,
+                                                          int order) {
+  const int l16 = threadIdx.x & 15;
+  const int gb = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int row = gb / nb, b = gb % nb;
+  if (row >= rows) return;
+  const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)row * x_rstride + (size_t)b * QK + 16 * l16);
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 f = src[i];
+    v[4 * i] = f.x;
+    v[4 * i + 1] = f.y;
+    v[4 * i + 2] = f.z;
+    v[4 * i + 3] = f.w;
+  }
+  const Q8Out16 o = quant_block16(v, l16);
+  uint8_t *r = y + (size_t)row * y_rstride + (size_t)b * XREC;
+  if (order == 0) {
+    *reinterpret_cast<uint4 *>(r + 16 * l16) = o.q;
+  } else {  // values 16 * l16 .. +15 are groups 2q, 2q + 1 of half h of chunk c
+    const int c = l16 >> 2, h = (l16 >> 1) & 1, q = l16 & 1;
+    *reinterpret_cast<uint2 *>(r + 64 * c + 32 * q + 8 * h) = make_uint2(o.q.x, o.q.y);
+    *reinterpret_cast<uint2 *>(r + 64 * c + 32 * q + 16 + 8 * h) = make_uint2(o.q.z, o.q.w);
+  }
+  reinterpret_cast<_Float16 *>(r + 256)[l16] = (_Float16)(float)o.bsum;
+  if (l16 == 0) *reinterpret_cast<float *>(r + 288) = o.d;
+}
+
+// ---------------------------------------------------------------- work items
+
+// Every active expert's bucket cut into runs of `tok` pairs, item = expert |
+// (first pair offset within the bucket) << 12, largest first: full runs, then
+// every expert's remaining run in descending order of its 16-pair tiles, so the
 // short items fill the tail of the launch.  The order of items with the same
 // size is not fixed; no result depends on it (every item writes its own pairs).
-// Needs n_active <= 1024 and tok <= 256.
-__global__ __launch_bounds__(1024) void k_mmq_items_lpt(const int32_t *__restrict__ n_active,
-                                                        const int32_t *__restrict__ active,
-                                                        const int32_t *__restrict__ offs, int32_t *__restrict__ items,
-                                                        int32_t *__restrict__ n_items, int tok) {
+// One workgroup; needs n_active <= 1024 and tok <= 256.
+static __global__ __launch_bounds__(1024) void k_mmq_items(const int32_t *__restrict__ n_active,
+                                                           const int32_t *__restrict__ active,
+                                                           const int32_t *__restrict__ offs,
+                                                           int32_t *__restrict__ items, int32_t *__restrict__ n_items,
+                                                           int tok) {
   constexpr int NK = 18;  // size classes: 1..16 tiles of a partial run, 17 = full run
   __shared__ int hist[NK], cur[NK];
   const int tid = threadIdx.x;
@@ -187,106 +226,345 @@ __global__ __launch_bounds__(1024) void k_mmq_items_lpt(const int32_t *__restric
   }
 }
 
-// One work item (up to 16*TT pairs of one bucket) against 64 weight rows
-// (4 waves x 16 rows).  The activation block of the item is staged in LDS
-// (double buffered over the K blocks; each thread holds the next block's share
-// in registers while the current block computes); the weights of block b+1
-// are requested while block b computes.
+// ---------------------------------------------------------------- weight blocks in LDS
+
+// blocks whose bytes are a multiple of 4 start on a dword; the others (2-byte
+// types) are staged from the dword at or below their start
+template <int T>
+constexpr bool mmq_dword() {
+  return block_bytes(T) % 4 == 0;
+}
+// 16-byte units loaded per row and block (an extra 2 bytes where a block starts inside a dword)
+template <int T>
+constexpr int mmq_load_units() {
+  return (block_bytes(T) + (mmq_dword<T>() ? 0 : 2) + 15) / 16;
+}
+// units of a row's slot: odd, so that 16 rows start in 16 different 16-byte bank groups
+template <int T>
+constexpr int mmq_units() {
+  return mmq_load_units<T>() | 1;
+}
+
+// the fields of one block that a lane needs
 template <int T>
 struct MmqW;
 template <>
-struct MmqW<T_Q4_K> {  // d, dmin, scales | this lane's 8 bytes of each 32-byte qs group
+struct MmqW<T_Q4_K> {  // d, dmin, scales | the lane's 8 bytes of each 32-byte qs group
   uint4 hdr;
   uint2 qs[4];
 };
 template <>
-struct MmqW<T_Q5_K> {  // d, dmin, scales | this lane's 8 bytes of qh and of each 32-byte qs group
+struct MmqW<T_Q5_K> {  // d, dmin, scales | the lane's 8 bytes of qh and of each qs group
   uint4 hdr;
   uint2 qh;
   uint2 qs[4];
 };
 template <>
-struct MmqW<T_Q2_K> {  // scales | this lane's 2 x 16 bytes of qs | d, dmin
+struct MmqW<T_Q2_K> {  // scales | the lane's 2 x 16 bytes of qs | d, dmin
   uint4 sc;
   uint4 qs[2];
   uint32_t dd;
 };
 template <>
+struct MmqW<T_Q3_K> {  // the lane's 16 bytes of hmask and 2 x 16 of qs | scales | d
+  Dwords<4> hm;
+  Dwords<4> qs[2];
+  Dwords<3> s;
+  uint16_t d;
+};
+template <>
+struct MmqW<T_Q6_K> {  // the lane's 4 x 8 bytes of ql, 2 x 8 of qh | scales | d
+  Dwords<2> ql[4];
+  Dwords<2> qh[2];
+  Dwords<4> sc;
+  uint16_t d;
+};
+template <>
 struct MmqW<T_IQ2_XXS> {  // d | all 64 bytes of qs (grid-index and sign+scale words per sub-block)
-  uint32_t d;
-  uint4 q[4];
+  uint16_t d;
+  Dwords<16> q;
 };
 template <>
-struct MmqW<T_IQ3_XXS> {  // d | 64 grid-index bytes | 8 scale+sign words
-  uint32_t d;
-  uint4 gi[4];
-  uint4 sas[2];
+struct MmqW<T_IQ3_XXS> {  // d | the lane's 2 grid-index bytes of each sub-block | 8 scale+sign words
+  uint16_t d;
+  uint16_t gi[8];
+  Dwords<8> sas;
 };
 template <>
-struct MmqW<T_IQ4_XS> {  // d, scales_h, scales_l | this lane's 16 qs bytes of each chunk
+struct MmqW<T_IQ4_XS> {  // d, scales_h, scales_l | the lane's 8 qs bytes of each sub-block
   uint2 hdr;
-  uint4 qs[4];
-};
-template <>
-struct MmqW<T_Q6_K> {  // this lane's 4 x 8 bytes of ql, 2 x 8 bytes of qh | scales | d
-  uint2 ql[4];
-  uint2 qh[2];
-  uint4 sc;
-  uint32_t d;
+  uint2 qs[8];
 };
 
-template <int T, bool GATEUP, int TT, int NW = 4>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(T == T_Q4_K && !GATEUP && TT <= 4 && NW == 4 ? 4 : 1))) void k_mmq(GemvArgs a) {
-  constexpr int TOK = 16 * TT;  // pairs per work item
-  constexpr int NT = 64 * NW;   // threads: NW waves of 16 weight rows each
-  static_assert(T == T_Q4_K || T == T_Q5_K || T == T_Q2_K || T == T_Q6_K || T == T_IQ4_XS || T == T_IQ2_XXS ||
-                    T == T_IQ3_XXS,
-                "MFMA prefill types");
+// p: the row's slot; al: the block's first byte in it (0 or 2, 0 for dword types)
+template <int T>
+__device__ __forceinline__ void mmq_read_w(const uint8_t *p, int al, int g, MmqW<T> &w) {
+  const uint32_t sel = align_sel(al);
+  if constexpr (T == T_Q4_K || T == T_Q5_K) {
+    constexpr int QS = T == T_Q5_K ? 48 : 16;
+    w.hdr = lds_get<uint4>(p);
+    if constexpr (T == T_Q5_K) w.qh = lds_get<uint2>(p + 16 + 8 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w.qs[i] = lds_get<uint2>(p + QS + 32 * i + 8 * g);
+  } else if constexpr (T == T_Q2_K) {
+    w.sc = lds_get<uint4>(p);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get<uint4>(p + 16 + 32 * h + 16 * (g & 1));
+    w.dd = lds_get<uint32_t>(p + 80);
+  } else if constexpr (T == T_Q3_K) {
+    w.hm = lds_get_at<4, 16>(p + 16 * (g & 1), sel);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get_at<4, 16>(p + 32 + 32 * h + 16 * (g & 1), sel);
+    w.s = lds_get_at<3, 16>(p + 96, sel);
+    w.d = lds_get<uint16_t>(p + 108 + al);
+  } else if constexpr (T == T_Q6_K) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w.ql[i] = lds_get_at<2, 8>(p + 64 * (i >> 1) + 32 * (i & 1) + 8 * g, sel);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w.qh[h] = lds_get_at<2, 8>(p + 128 + 32 * h + 8 * g, sel);
+    w.sc = lds_get_at<4, 16>(p + 192, sel);
+    w.d = lds_get<uint16_t>(p + 208 + al);
+  } else if constexpr (T == T_IQ2_XXS) {
+    w.d = lds_get<uint16_t>(p + al);
+    w.q = lds_get_at<16, 16>(p, align_sel(2 + al));
+  } else if constexpr (T == T_IQ3_XXS) {
+    w.d = lds_get<uint16_t>(p + al);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w.gi[i] = lds_get<uint16_t>(p + al + 2 + 8 * i + 2 * g);
+    w.sas = lds_get_at<8, 16>(p + 64, align_sel(2 + al));
+  } else {
+    w.hdr = lds_get<uint2>(p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w.qs[i] = lds_get<uint2>(p + 8 + 16 * i + 8 * (g & 1));
+  }
+}
+
+// ---------------------------------------------------------------- B operands
+
+template <int T>
+constexpr bool mmq_folded() {  // scales in the weights: whole-block integer chains
+  return T == T_Q2_K || T == T_Q3_K || T == T_Q4_K || T == T_Q5_K;
+}
+template <int T>
+constexpr bool mmq_mins() {
+  return T == T_Q2_K || T == T_Q4_K || T == T_Q5_K;
+}
+template <int T>
+constexpr int mmq_chains() {
+  return T == T_Q5_K ? 3 : (T == T_Q4_K ? 2 : 1);
+}
+
+template <int T, bool FOLDED = mmq_folded<T>()>
+struct MmqB;
+template <int T>
+struct MmqB<T, true> {
+  v4i_t b[mmq_chains<T>()][4];  // per chain and 64-weight chunk
+  v4h_t mn;                     // mins of the 16-sums 4g .. 4g + 3
+  float d, dmin;
+};
+template <int T>
+struct MmqB<T, false> {
+  static constexpr int NB = T == T_Q6_K ? 16 : 8;  // sub-blocks
+  long b[NB];
+  int s[NB];
+  float d;
+};
+
+// tables: Q3_K 64 x 8 bytes (4 - k) * (s - 32); IQ2_XXS / IQ3_XXS grid and sign masks; IQ4_XS values in tab
+template <int T>
+__device__ __forceinline__ void mmq_unpack(const MmqW<T> &w, int g, const uint64_t *s_tab, const uint64_t *s_signs,
+                                           const uint32_t (&tab)[4], MmqB<T> &o) {
+  if constexpr (T == T_Q4_K || T == T_Q5_K) {
+    const uint32_t u0 = w.hdr.y, u1 = w.hdr.z, u2 = w.hdr.w;
+    const uint32_t sc_lo = u0 & 0x3f3f3f3fu, mn_lo = u1 & 0x3f3f3f3fu;
+    const uint32_t sc_hi = (u2 & 0x0f0f0f0fu) | (((u0 >> 6) & 0x03030303u) << 4);
+    const uint32_t mn_hi = ((u2 >> 4) & 0x0f0f0f0fu) | (((u1 >> 6) & 0x03030303u) << 4);
+    o.d = h2f((uint16_t)(w.hdr.x & 0xffffu));
+    o.dmin = h2f((uint16_t)(w.hdr.x >> 16));
+    // 16-sums 4g .. 4g + 3 belong to sub-blocks 2g (twice), 2g + 1 (twice)
+    const uint32_t mw = (g < 2 ? mn_lo : mn_hi) >> (16 * (g & 1));
+    const v2h_t h0 = bytes_f16(mw, 0x0c000c00u), h1 = bytes_f16(mw, 0x0c010c01u);
+    o.mn = v4h_t{h0[0], h0[1], h1[0], h1[1]};
+    // chunk i = qs group i: sub-block 2i in its low nibbles, 2i + 1 in its high
+    // nibbles; Q5_K: the fifth bits are bits 2i, 2i + 1 of the lane's qh bytes
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t scw = (i < 2 ? sc_lo : sc_hi) >> (16 * (i & 1));
+      const uint32_t s0 = scw & 0xffu, s1 = (scw >> 8) & 0xffu;
+      const uint2 q = w.qs[i];
+      const uint32_t n0 = q.x & 0x0f0f0f0fu, n1 = q.y & 0x0f0f0f0fu;
+      const uint32_t n2 = (q.x >> 4) & 0x0f0f0f0fu, n3 = (q.y >> 4) & 0x0f0f0f0fu;
+      o.b[0][i] = v4i_t{(int)mul_bytes(n0, s0 & 7u), (int)mul_bytes(n1, s0 & 7u), (int)mul_bytes(n2, s1 & 7u),
+                        (int)mul_bytes(n3, s1 & 7u)};
+      o.b[1][i] = v4i_t{(int)mul_bytes(n0, s0 >> 3), (int)mul_bytes(n1, s0 >> 3), (int)mul_bytes(n2, s1 >> 3),
+                        (int)mul_bytes(n3, s1 >> 3)};
+      if constexpr (T == T_Q5_K) {
+        const uint2 h = w.qh;
+        o.b[2][i] = v4i_t{(int)mul_bytes((h.x >> (2 * i)) & 0x01010101u, s0),
+                          (int)mul_bytes((h.y >> (2 * i)) & 0x01010101u, s0),
+                          (int)mul_bytes((h.x >> (2 * i + 1)) & 0x01010101u, s1),
+                          (int)mul_bytes((h.y >> (2 * i + 1)) & 0x01010101u, s1)};
+      }
+    }
+  } else if constexpr (T == T_Q2_K) {
+    o.d = h2f((uint16_t)(w.dd & 0xffffu));
+    o.dmin = h2f((uint16_t)(w.dd >> 16));
+    const uint32_t scb[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
+    const uint32_t mw = ((g < 2 ? (g == 0 ? scb[0] : scb[1]) : (g == 2 ? scb[2] : scb[3])) >> 4) & 0x0f0f0f0fu;
+    const v2h_t h0 = bytes_f16(mw, 0x0c010c00u), h1 = bytes_f16(mw, 0x0c030c02u);
+    o.mn = v4h_t{h0[0], h0[1], h1[0], h1[1]};
+    // chunk c = 2h + jp, weights 64c + 16g .. +15: bit-plane 2jp + (g >> 1) of
+    // qs bytes 32h + 16(g & 1) .. +15, sub-block 4c + g
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t sc = (scb[c] >> (8 * g)) & 15u;
+      const uint4 q = w.qs[c >> 1];
+      const int sh = 4 * (c & 1) + 2 * (g >> 1);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o.b[0][c][k] = (int)mul_bytes((u4_get(q, k) >> sh) & 0x03030303u, sc);
+    }
+  } else if constexpr (T == T_Q3_K) {
+    o.d = -h2f(w.d);  // the chain carries -(q' - 4) * sc
+    o.dmin = 0.f;
+    const uint32_t a0 = w.s.v[0] >> (8 * g), a1 = w.s.v[1] >> (8 * g), a2 = w.s.v[2] >> (8 * g);
+    // chunk c as for Q2_K (sub-block 4c + g); the high bit of plane 4h + j is bit 4h + j of the hmask byte
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t lo4 = ((c & 1 ? a1 : a0) >> (4 * (c >> 1))) & 15u;
+      const uint64_t t = s_tab[lo4 | (((a2 >> (2 * c)) & 3u) << 4)];
+      const int j = 2 * (c & 1) + (g >> 1);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t hm = w.hm.v[k];
+        const uint32_t hb = ((c >= 2 ? hm >> 2 : hm << 2) >> j) & 0x04040404u;
+        const uint32_t q = ((w.qs[c >> 1].v[k] >> (2 * j)) & 0x03030303u) | hb;
+        o.b[0][c][k] = (int)__builtin_amdgcn_perm((uint32_t)(t >> 32), (uint32_t)t, q);
+      }
+    }
+  } else if constexpr (T == T_Q6_K) {
+    o.d = 0.25f * h2f(w.d);  // the operand carries 4 * (q - 32)
+    const uint32_t (&scb)[4] = w.sc.v;
+    const uint32_t keep0 = g < 2 ? 0xffffffffu : 0u;
+    uint2 hb[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)  // the upper of the two top bits flipped: q ^ 32
+      hb[h] = make_uint2(w.qh[h].v[0] ^ 0xaaaaaaaau, w.qh[h].v[1] ^ 0xaaaaaaaau);
+    // pair p = sub-blocks 2p (lane groups 0-1), 2p + 1 (groups 2-3): low (G < 2)
+    // or high nibbles of ql bytes 64h + 32(p & 1) + 8g.., top bits 2G of qh bytes 32h + 8g..
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      const int h = p >> 2, G = p & 3;
+      const uint2 q = make_uint2(w.ql[2 * h + (p & 1)].v[0], w.ql[2 * h + (p & 1)].v[1]);
+      const uint32_t lx = (G < 2 ? q.x << 2 : q.x >> 2) & 0x3c3c3c3cu, ly = (G < 2 ? q.y << 2 : q.y >> 2) & 0x3c3c3c3cu;
+      const uint32_t vx = lx | ((hb[h].x << (6 - 2 * G)) & 0xc0c0c0c0u);
+      const uint32_t vy = ly | ((hb[h].y << (6 - 2 * G)) & 0xc0c0c0c0u);
+      o.b[2 * p] = (long)(((uint64_t)(vy & keep0) << 32) | (vx & keep0));
+      o.b[2 * p + 1] = (long)(((uint64_t)(vy & ~keep0) << 32) | (vx & ~keep0));
+      o.s[2 * p] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1)));
+      o.s[2 * p + 1] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1) + 8));
+    }
+  } else if constexpr (T == T_IQ4_XS) {
+    // sub-block sb: weights 8g .. 8g + 7 = low (g < 2) or high nibbles of its qs bytes 8(g & 1) .. +7
+    o.d = h2f((uint16_t)(w.hdr.x & 0xffffu));
+    const int ns = 4 * (g >> 1);
+#pragma unroll
+    for (int sb = 0; sb < 8; ++sb) {
+      const uint32_t v0 = lut16((w.qs[sb].x >> ns) & 0x0f0f0f0fu, tab[0], tab[1], tab[2], tab[3]);
+      const uint32_t v1 = lut16((w.qs[sb].y >> ns) & 0x0f0f0f0fu, tab[0], tab[1], tab[2], tab[3]);
+      o.b[sb] = (long)(((uint64_t)v1 << 32) | v0);
+      o.s[sb] = iq4_scale(w.hdr.x, w.hdr.y, sb);
+    }
+  } else {
+    // lane group g holds the 8-weight group g of every sub-block: grid values with
+    // their signs applied; 1/8 (IQ2_XXS) or 1/4 (IQ3_XXS) folded into d
+    o.d = (T == T_IQ2_XXS ? 0.125f : 0.25f) * h2f(w.d);
+#pragma unroll
+    for (int sb = 0; sb < 8; ++sb) {
+      uint32_t glo, ghi, aux;
+      if constexpr (T == T_IQ2_XXS) {
+        const uint32_t aux0 = w.q.v[2 * sb];
+        aux = w.q.v[2 * sb + 1];
+        const uint64_t gg = s_tab[(aux0 >> (8 * g)) & 0xffu];
+        glo = (uint32_t)gg;
+        ghi = (uint32_t)(gg >> 32);
+      } else {
+        aux = w.sas.v[sb];
+        const uint32_t *g3 = reinterpret_cast<const uint32_t *>(s_tab);
+        glo = g3[w.gi[sb] & 0xffu];
+        ghi = g3[w.gi[sb] >> 8];
+      }
+      const uint64_t mm = s_signs[(aux >> (7 * g)) & 127u];
+      const uint32_t v0 = sign_bytes(glo, (uint32_t)mm), v1 = sign_bytes(ghi, (uint32_t)(mm >> 32));
+      o.b[sb] = (long)(((uint64_t)v1 << 32) | v0);
+      o.s[sb] = 2 * (int)(aux >> 28) + 1;
+    }
+  }
+}
+
+// ---------------------------------------------------------------- the kernel
+
+// TT: 16-pair tiles per item; NW: waves (16 weight rows each); ST: activation stages
+template <int T, bool GATEUP, int TT, int NW, int ST>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 ? 4 : 2))) void k_mmq(GemvArgs a) {
+  constexpr int TOK = 16 * TT;
+  constexpr int NM = GATEUP ? 2 : 1;
+  constexpr int BB = block_bytes(T);
+  constexpr int UN = TOK * XUNITS;          // activation units of a stage
+  constexpr int NI = (UN + 64 * NW - 1) / (64 * NW);
+  constexpr int RU = mmq_units<T>(), LU = mmq_load_units<T>();
+  constexpr int NWI = (16 * RU + 63) / 64;  // weight loads per matrix and block
+  constexpr int WB = 16 * RU * 16;          // LDS bytes of one matrix block of a wave
   constexpr bool kGrid = T == T_IQ2_XXS || T == T_IQ3_XXS;
-  // the lookup tables first in LDS (largest alignment first), so their
-  // addresses fold into the LDS reads' offset field
-  __shared__ __attribute__((aligned(kGrid ? 4096 : 8))) uint64_t s_grid[kGrid ? (T == T_IQ2_XXS ? 256 : 128) : 1];  // IQ3_XXS: 256 x u32
+  constexpr int NTAB = T == T_IQ2_XXS ? 256 : (T == T_IQ3_XXS ? 128 : (T == T_Q3_K ? 64 : 1));
+  static_assert(ST == 2 || ST == 3, "activation stages");
+  // lookup tables first (largest alignment first), so that their addresses fold into the reads' offset field
+  __shared__ __attribute__((aligned(kGrid ? 4096 : 16))) uint64_t s_tab[NTAB];
   __shared__ __attribute__((aligned(kGrid ? 2048 : 8))) uint64_t s_signs[kGrid ? 128 : 1];
-  constexpr bool K45 = T == T_Q4_K || T == T_Q5_K;
-  // The activation blocks reach LDS by direct buffer-to-LDS loads (no register
-  // staging); a token's row is 256 bytes with its 16-byte chunks XOR-swizzled
-  // by the token index (chunk c of token t at c ^ (t & 15)), so the 16 tokens
-  // of an MFMA A operand read 16 different bank groups; the raw int16 16-sums
-  // are kept (and added pairwise where 32-sums are used)
-  __shared__ __attribute__((aligned(16))) uint8_t s_xq[2][TOK][QK];
-  __shared__ __attribute__((aligned(16))) int16_t s_bs16[2][TOK][16];
-  __shared__ __attribute__((aligned(16))) float s_xd[2][TOK];
-  __shared__ int s_xoff[TOK];      // byte offset of each pair's activation row (OOR: none)
-  __shared__ int s_pair[TOK];
+  __shared__ __attribute__((aligned(16))) uint8_t s_x[ST][TOK * XREC];
+  __shared__ __attribute__((aligned(16))) uint8_t s_w[NW][NM][WB];
+  __shared__ int s_xoff[TOK];   // byte offset of each pair's activation row (OOR: none)
+  __shared__ long s_out[TOK];   // float offset of each pair's output row (-1: none)
   int e, pc, p1;
+  const int item = blockIdx.x / a.row_tiles, rt = blockIdx.x - item * a.row_tiles;
   if (a.dense_S > 0) {
     e = 0;
-    pc = blockIdx.y * TOK;
+    pc = item * TOK;
     p1 = a.dense_S;
     if (pc >= p1) return;
   } else {
-    if ((int)blockIdx.y >= *a.n_items) return;
-    const int it = a.items[blockIdx.y];
+    if (item >= *a.n_items) return;
+    const int it = a.items[item];
     e = it & 0xfff;
     pc = a.offs[e] + (it >> 12);
     p1 = a.offs[e + 1];
   }
-  constexpr int NM = GATEUP ? 2 : 1;
-  constexpr int BB = block_bytes(T);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
-  const int row = blockIdx.x * (16 * NW) + wave * 16 + n;  // weight row of this lane (B operand, output column)
-  const bool rv = row < a.nrows;
-  const uint32_t wbytes = (uint32_t)((size_t)a.nrows * a.w_rstride);
-  rsrc_t rw[NM];
-  rw[0] = make_rsrc(a.w0 + (size_t)e * a.w_estride, wbytes);
-  if constexpr (GATEUP) rw[1] = make_rsrc(a.w1 + (size_t)e * a.w_estride, wbytes);
-  const v4u_t rxd = dma_rsrc(a.xq, a.xq_bytes);
-  const int vrow = rv ? row * (int)a.w_rstride : OOR;
-  const int Kp = a.dense_S > 0 ? 1 : a.K;
+  const int row0 = (rt * NW + wave) * 16;
+  const int row = row0 + n;
   const int nb = a.nb;
   const int nt = min(TT, (p1 - pc + 15) / 16);
-  uint32_t tab[4] = {0, 0, 0, 0};  // IQ4_XS value table (a.grid), wave-uniform
+  if (tid < TOK) {
+    int pair = -1;
+    if (pc + tid < p1) pair = a.dense_S > 0 ? pc + tid : a.pairs[pc + tid];
+    const int Kp = a.dense_S > 0 ? 1 : a.K;
+    const int tok = pair / Kp, k = pair - tok * Kp;
+    s_xoff[tid] = pair >= 0 ? (int)((tok * a.ne11 + k % a.ne11) * a.xq_rstride) : OOR;
+    s_out[tid] = pair >= 0 ? (long)((size_t)tok * a.out_s + (size_t)k * a.out_k) : -1;
+  }
+  if constexpr (T == T_Q3_K) {
+    if (tid < 64) {
+      uint64_t t = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t |= (uint64_t)((uint32_t)((4 - k) * (tid - 32)) & 0xffu) << (8 * k);
+      s_tab[tid] = t;
+    }
+  }
+  if constexpr (kGrid) {
+    for (int i = tid; i < NTAB; i += 64 * NW) s_tab[i] = a.grid[i];
+    for (int i = tid; i < 128; i += 64 * NW) s_signs[i] = a.signs[i];
+  }
+  uint32_t tab[4] = {0, 0, 0, 0};  // IQ4_XS value table, wave-uniform
   if constexpr (T == T_IQ4_XS) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -294,451 +572,209 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(T == T_
       tab[2 * i + 1] = (uint32_t)(a.grid[i] >> 32);
     }
   }
-
-  if constexpr (kGrid) {
-    for (int i = tid; i < (T == T_IQ2_XXS ? 256 : 128); i += NT) s_grid[i] = a.grid[i];
-    if (tid < 128) s_signs[tid] = a.signs[tid];
-  }
-  if (tid < TOK) {
-    const int p = pc + tid;
-    const bool ok = p < p1;
-    const int pair = ok ? (a.dense_S > 0 ? p : a.pairs[p]) : -1;
-    s_pair[tid] = pair;
-    s_xoff[tid] = ok ? (int)(((pair / Kp) * a.ne11 + (pair % Kp) % a.ne11) * a.xq_rstride) : OOR;
-  }
   __syncthreads();
-
-  using WBlk = MmqW<T>;
-  auto load_w = [&](int b, WBlk (&w)[NM]) {
-    const int vo = b < nb ? vrow + b * BB : OOR;
+  // activation units of this wave: record u / 19, unit u % 19
+  int xo[NI];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      if constexpr (T == T_Q4_K) {
-        w[m].hdr = bld16(rw[m], vo, 0);
+  for (int i = 0; i < NI; ++i) {
+    const int u = (i * NW + wave) * 64 + lane;
+    const int t = u / XUNITS, p = u - XUNITS * t;
+    const int o = t < TOK ? s_xoff[t] : OOR;
+    xo[i] = o != OOR ? o + 16 * p : OOR;
+  }
+  const v4u_t rx = dma_rsrc(a.xq, a.xq_bytes);
+  // weight units: row u / RU of the wave's 16, unit u % RU.  The resource starts
+  // on a dword; of a 2-byte type the even and the odd blocks of a row start on
+  // either half of a dword (al), so each parity has its offsets.  Gate and up
+  // lie alike within a dword (the host checks).
+  const uint8_t *wm[2] = {a.w0 + (size_t)e * a.w_estride, GATEUP ? a.w1 + (size_t)e * a.w_estride : nullptr};
+  const int sh = mmq_dword<T>() ? 0 : (int)((uintptr_t)wm[0] & 3);
+  const uint32_t wbytes = ((uint32_t)((size_t)a.nrows * a.w_rstride) + sh + 3) & ~3u;
+  v4u_t rw[NM];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[m].qs[i] = bld8(rw[m], vo + 16 + 32 * i + 8 * g, 0);
-      } else if constexpr (T == T_Q5_K) {
-        w[m].hdr = bld16(rw[m], vo, 0);
-        w[m].qh = bld8(rw[m], vo + 16 + 8 * g, 0);
+  for (int m = 0; m < NM; ++m) rw[m] = dma_rsrc(wm[m] - sh, wbytes);
+  const int al = mmq_dword<T>() ? 0 : (sh + row * (int)a.w_rstride) & 3;
+  int wo[mmq_dword<T>() ? 1 : 2][NWI];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[m].qs[i] = bld8(rw[m], vo + 48 + 32 * i + 8 * g, 0);
-      } else if constexpr (T == T_IQ2_XXS) {
-        w[m].d = bld2(rw[m], vo, 0);
+  for (int i = 0; i < NWI; ++i) {
+    const int u = i * 64 + lane;
+    const int r = u / RU, p = u - RU * r;
+    const bool ok = r < 16 && p < LU && row0 + r < a.nrows;
+    const int st = sh + (row0 + r) * (int)a.w_rstride;
+    wo[0][i] = ok ? (st & ~3) + 16 * p : OOR;
+    if constexpr (!mmq_dword<T>()) wo[1][i] = ok ? ((st + BB) & ~3) + 16 * p : OOR;
+  }
+  auto dma_w = [&](int m, int b) {
+    const uint32_t base = lds_addr(&s_w[wave][m][0]);
+    const int par = mmq_dword<T>() ? 0 : b & 1;
+    const int so = (b - par) * BB;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[m].q[i] = bld16(rw[m], vo + 2 + 16 * i, 0);
-      } else if constexpr (T == T_IQ3_XXS) {
-        w[m].d = bld2(rw[m], vo, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[m].gi[i] = bld16(rw[m], vo + 2 + 16 * i, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) w[m].sas[i] = bld16(rw[m], vo + 66 + 16 * i, 0);
-      } else if constexpr (T == T_IQ4_XS) {
-        w[m].hdr = bld8(rw[m], vo, 0);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) w[m].qs[c] = bld16(rw[m], vo + 8 + 32 * c + 16 * (g >> 1), 0);
-      } else if constexpr (T == T_Q6_K) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[m].ql[i] = bld8(rw[m], vo + 64 * (i >> 1) + 32 * (i & 1) + 8 * g, 0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) w[m].qh[h] = bld8(rw[m], vo + 128 + 32 * h + 8 * g, 0);
-        w[m].sc = bld16(rw[m], vo + 192, 0);
-        w[m].d = bld2(rw[m], vo + 208, 0);
-      } else {
-        w[m].sc = bld16(rw[m], vo, 0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) w[m].qs[h] = bld16(rw[m], vo + 16 + 32 * h + 16 * (g & 1), 0);
-        w[m].dd = bld4(rw[m], vo + 80, 0);
-      }
+    for (int i = 0; i < NWI; ++i) {
+      if (64 * (i + 1) > 16 * RU && 64 * i + lane >= 16 * RU) continue;
+      const int vo = par ? wo[mmq_dword<T>() ? 0 : 1][i] : wo[0][i];
+      // rows that fill their units exactly never reach past the resource, whose
+      // bounds the scalar offset is not part of; the others add it per lane
+      if constexpr (16 * LU == BB) dma_lds16(rw[m], base + i * 1024u, vo, so);
+      else dma_lds16(rw[m], base + i * 1024u, vo == OOR ? OOR : vo + so, 0);
     }
   };
-  // direct loads of block b's activations into buffer buf: the qs of
-  // TOK tokens (1 KB = 4 tokens per wave instruction), their 16 bsums (32 B per
-  // token) and d; out-of-range lanes write zeros
-  auto dma_x = [&](int b, int buf) {
-    {
-      const bool bv = b < nb;
-      constexpr int QI = TOK / 4 / NW;  // qs instructions per wave
-      static_assert(TOK % (4 * NW) == 0, "qs instructions per wave");
-#pragma unroll
-      for (int i = 0; i < QI; ++i) {
-        const int t0 = 4 * (QI * wave + i);
-        const int t = t0 + (lane >> 4), c = (lane & 15) ^ (t & 15);
-        const int o = s_xoff[t];
-        dma_lds16(rxd, lds_addr(&s_xq[buf][t0][0]), (bv && o != OOR) ? o + b * QK + 16 * c : OOR);
-      }
-      for (int i = wave; 32 * i < TOK; i += NW) {  // bsums: 2 lanes per token
-        const int t = 32 * i + (lane >> 1);
-        if (t >= TOK) break;  // lanes past the tile write nothing
-        const int o = s_xoff[t];
-        dma_lds16(rxd, lds_addr(&s_bs16[buf][32 * i][0]),
-                  (bv && o != OOR) ? o + (int)q8_bs_off(nb) + b * 32 + 16 * (lane & 1) : OOR);
-      }
-      for (int i = wave; 64 * i < TOK; i += NW) {  // d: one float per token
-        const int t = 64 * i + lane;
-        if (t >= TOK) break;
-        const int o = s_xoff[t];
-        dma_lds4(rxd, lds_addr(&s_xd[buf][64 * i]), (bv && o != OOR) ? o + (int)q8_d_off(nb) + 4 * b : OOR);
-      }
-    }
-  };
+  const uint8_t *wl = &s_w[wave][0][0] + n * (RU * 16);
 
-  // reads of the staged activations: logical 16-byte chunk c (or its 8-byte
-  // half h) of token tok, and its raw 16-sum j / 32-sum j (16-sums 2j, 2j + 1)
-  auto xq16 = [&](int buf, int tok, int c) {
-    return *reinterpret_cast<const v4i_t *>(&s_xq[buf][tok][16 * (c ^ (tok & 15))]);
-  };
-  auto xq8 = [&](int buf, int tok, int c, int h) {
-    return *reinterpret_cast<const uint2 *>(&s_xq[buf][tok][16 * (c ^ (tok & 15)) + 8 * h]);
-  };
-  auto bsum16 = [&](int buf, int tok, int j) { return (int)s_bs16[buf][tok][j]; };
-  auto bsum32 = [&](int buf, int tok, int j) {
-    const int w = reinterpret_cast<const int *>(&s_bs16[buf][tok][0])[j];
-    return __builtin_amdgcn_sdot2(__builtin_bit_cast(v2i16_t, w), v2i16_t{1, 1}, 0, false);
-  };
-
-  // per (matrix, token tile, output): f += d_x * (d * isum + mn), as
-  // two fmas (the tile epilogue is most of the per-tile VALU work)
-  float f[NM][TT][4];
+  auto body = [&](auto nt_tag) {
+    constexpr int NT = decltype(nt_tag)::value;
+    constexpr int NC = mmq_chains<T>();
+    constexpr int NIT = (NT * 16 * XUNITS + 64 * NW - 1) / (64 * NW);
+    constexpr int NIM = (NT * 16 * XUNITS) / (64 * NW);  // of these, issued by every wave
+    auto dma_x = [&](int b, int slot) {
+      const uint32_t base = lds_addr(&s_x[0][0]) + slot * (uint32_t)sizeof(s_x[0]) + wave * 1024u;
 #pragma unroll
-  for (int m = 0; m < NM; ++m)
+      for (int i = 0; i < NIT; ++i) {
+        if ((i * NW + NW) * 64 > UN && (i * NW + wave) * 64 + lane >= UN) continue;
+        dma_lds16(rx, base + i * NW * 1024u, xo[i], b * XREC);
+      }
+    };
+    v4i_t zero = {0, 0, 0, 0};
+    asm("" : "+v"(zero));  // one zero operand for the first MFMA of every chain
+    float f[NM][NT][4];
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+    for (int m = 0; m < NM; ++m)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) f[m][t][j] = 0.f;
-
-  // one block of the K loop from the weights in wcur and activation buffer buf
-  auto step = [&](int buf, const WBlk(&wcur)[NM]) {
-    if constexpr (K45) {
-      // both matrices' operands first, then one pass over the token tiles: the
-      // activation operand (and the bsums of the min product) is read from LDS
-      // once per tile for gate and up together
-      constexpr int N5 = T == T_Q5_K ? 4 : 1;
-      v4i_t bl[NM][4], bh[NM][4], b5[NM][N5];
-      float dd[NM], dm[NM], mb0[NM], mb1[NM];
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[m][t][j] = 0.f;
+    // request order: x(0) W0(0) x(1) .. W1(0), then per block W0(b + 1), x(b + ST - 1), W1(b + 1)
+    dma_x(0, 0);
+    dma_w(0, 0);
+    if constexpr (ST > 2) dma_x(min(1, nb - 1), 1);
+    if constexpr (NM == 2) dma_w(1, 0);
+    int slot = 0, pslot = ST - 1;
+    for (int b = 0; b < nb; ++b) {
+      // W0(b) and x(b) have landed once only younger requests are outstanding:
+      // W1(b) and, with a third stage, x(b + 1)
+      wait_barrier<(NM - 1) * NWI + (ST > 2 ? NIM : 0)>();
+      const uint8_t *xs = &s_x[0][0] + slot * sizeof(s_x[0]);
+      const int bn = min(b + 1, nb - 1);  // past the end: the last block again, never read
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
-        const uint32_t u0 = wcur[m].hdr.y, u1 = wcur[m].hdr.z, u2 = wcur[m].hdr.w;
-        const uint32_t sc_lo = u0 & 0x3f3f3f3fu, mn_lo = u1 & 0x3f3f3f3fu;
-        const uint32_t sc_hi = (u2 & 0x0f0f0f0fu) | (((u0 >> 6) & 0x03030303u) << 4);
-        const uint32_t mn_hi = ((u2 >> 4) & 0x0f0f0f0fu) | (((u1 >> 6) & 0x03030303u) << 4);
-        dd[m] = h2f((uint16_t)(wcur[m].hdr.x & 0xffffu));
-        dm[m] = h2f((uint16_t)(wcur[m].hdr.x >> 16));
-        // B operand of the min product: m[row][sb] for sb = g and g + 4
-        // with -dmin folded in (exact: an f16 times a 6-bit integer), so the
-        // product comes out as the whole min term
-        mb0[m] = -dm[m] * (float)((mn_lo >> (8 * g)) & 0xffu);
-        mb1[m] = -dm[m] * (float)((mn_hi >> (8 * g)) & 0xffu);
-        // scale-folded weights of the 4 chunks: lane's sub-block 2i + (g >> 1),
-        // sc = 8 * hi + lo; Q5_K: the fifth bit (bit 2i + (g >> 1) of the lane's
-        // qh bytes) is a third chain with the whole scale, isum = D_lo + 8 D_hi + 16 D_5
-        {
-          // chunk i = qs group i (sub-blocks 2i, 2i + 1): the lane's 8 bytes
-          // 8g .. 8g + 7 give 8 weights of each sub-block, low nibbles then
-          // high nibbles (the activation operand is read in the same order);
-          // Q5_K: their fifth bits are bits 2i, 2i + 1 of the lane's 8 qh bytes
+        if (m == 1) wait_vm<NWI + NIM>();  // W1(b); younger: W0(b + 1) and x(b + ST - 1)
+        MmqW<T> w;
+        mmq_read_w<T>(wl + m * WB, mmq_dword<T>() ? 0 : al ^ (2 * (b & 1)), g, w);
+        wait_lds();
+        dma_w(m, bn);                                               // the slot has been read
+        if (m == 0) dma_x(min(b + ST - 1, nb - 1), pslot);          // every wave is past block b - 1
+        MmqB<T> B;
+        mmq_unpack<T>(w, g, s_tab, s_signs, tab, B);
+        asm("" : "+v"(B.d));  // a plain f32 from here on
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t scw = (i < 2 ? sc_lo : sc_hi) >> (16 * (i & 1));
-            const uint32_t s0 = scw & 0xffu, s1 = (scw >> 8) & 0xffu;
-            const uint2 q = wcur[m].qs[i];
-            const uint32_t n0 = q.x & 0x0f0f0f0fu, n1 = q.y & 0x0f0f0f0fu;
-            const uint32_t n2 = (q.x >> 4) & 0x0f0f0f0fu, n3 = (q.y >> 4) & 0x0f0f0f0fu;
-            bl[m][i] = v4i_t{(int)mul_bytes(n0, s0 & 7u), (int)mul_bytes(n1, s0 & 7u), (int)mul_bytes(n2, s1 & 7u),
-                             (int)mul_bytes(n3, s1 & 7u)};
-            bh[m][i] = v4i_t{(int)mul_bytes(n0, s0 >> 3), (int)mul_bytes(n1, s0 >> 3), (int)mul_bytes(n2, s1 >> 3),
-                             (int)mul_bytes(n3, s1 >> 3)};
-            if constexpr (T == T_Q5_K) {
-              const uint2 h = wcur[m].qh;
-              b5[m][i] = v4i_t{(int)mul_bytes((h.x >> (2 * i)) & 0x01010101u, s0),
-                               (int)mul_bytes((h.y >> (2 * i)) & 0x01010101u, s0),
-                               (int)mul_bytes((h.x >> (2 * i + 1)) & 0x01010101u, s1),
-                               (int)mul_bytes((h.y >> (2 * i + 1)) & 0x01010101u, s1)};
+        for (int t = 0; t < NT; ++t) {
+          const uint8_t *xt = xs + (16 * t + n) * XREC;
+          v4i_t xa[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) xa[c] = *reinterpret_cast<const v4i_t *>(xt + 64 * c + 16 * g);
+          float xd[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xd[j] = *reinterpret_cast<const float *>(xs + (16 * t + 4 * g + j) * XREC + 288);
+          if constexpr (mmq_folded<T>()) {
+            v4i_t D[NC];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+              for (int k = 0; k < NC; ++k)
+                D[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[c], B.b[k][c], c == 0 ? zero : D[k], 0, 0, 0);
+            v4f_t mn;
+            if constexpr (mmq_mins<T>()) {
+              const v4h_t bs = *reinterpret_cast<const v4h_t *>(xt + 256 + 8 * g);
+              mn = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, B.mn, __builtin_bit_cast(v4f_t, zero), 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              int is = D[0][j];
+              if constexpr (NC > 1) is += 8 * D[NC > 1 ? 1 : 0][j];
+              if constexpr (NC > 2) is += 16 * D[NC > 2 ? 2 : 0][j];
+              float v;
+              if constexpr (mmq_mins<T>()) v = __builtin_fmaf(B.d, (float)is, -(B.dmin * mn[j]));
+              else v = B.d * (float)is;
+              f[m][t][j] = __builtin_fmaf(xd[j], v, f[m][t][j]);
+              asm volatile("" : "+v"(f[m][t][j]));  // as below
+            }
+          } else {
+            int is[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {  // half h of the chunk's operand: 32 values
+                const uint2 xh = h ? make_uint2((uint32_t)xa[c][2], (uint32_t)xa[c][3]) : make_uint2((uint32_t)xa[c][0], (uint32_t)xa[c][1]);
+                const long x8 = __builtin_bit_cast(long, xh);
+                constexpr int PS = MmqB<T>::NB / 8;  // sub-blocks per 32 values
+#pragma unroll
+                for (int q = 0; q < PS; ++q) {
+                  const int sb = (2 * c + h) * PS + q;
+                  const v4i_t D = __builtin_amdgcn_mfma_i32_16x16x32_i8(x8, B.b[sb], zero, 0, 0, 0);
+#pragma unroll
+                  for (int j = 0; j < 4; ++j) is[j] = __mul24(B.s[sb], D[j]) + is[j];
+                }
+              }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              f[m][t][j] = __builtin_fmaf(xd[j], B.d * (float)is[j], f[m][t][j]);
+              // computed here: left to float, the tile's operands stay live into the next matrix
+              asm volatile("" : "+v"(f[m][t][j]));
             }
           }
         }
       }
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= nt) continue;
-        const int tok = 16 * t + n;
-        v4i_t xa[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // activations 64i + 8g .. +7 and 64i + 32 + 8g .. +7 (logical 16-byte
-          // chunks 4i + g/2 and 4i + 2 + g/2, half g & 1)
-          const uint2 lo8 = xq8(buf, tok, 4 * i + (g >> 1), g & 1);
-          const uint2 hi8 = xq8(buf, tok, 4 * i + 2 + (g >> 1), g & 1);
-          xa[i] = v4i_t{(int)lo8.x, (int)lo8.y, (int)hi8.x, (int)hi8.y};
-        }
-        // 32-sums of sub-blocks g and g + 4
-        const float bs0 = (float)bsum32(buf, tok, g), bs1 = (float)bsum32(buf, tok, g + 4);
-        float xdj[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xdj[j] = s_xd[buf][16 * t + 4 * g + j];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-          v4i_t dlo = {0, 0, 0, 0}, dhi = {0, 0, 0, 0}, d5 = {0, 0, 0, 0};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            dlo = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[i], bl[m][i], dlo, 0, 0, 0);
-            dhi = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[i], bh[m][i], dhi, 0, 0, 0);
-            if constexpr (T == T_Q5_K) d5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[i], b5[m][i], d5, 0, 0, 0);
-          }
-          v4f_t mn = {0.f, 0.f, 0.f, 0.f};
-          mn = __builtin_amdgcn_mfma_f32_16x16x4f32(bs0, mb0[m], mn, 0, 0, 0);
-          mn = __builtin_amdgcn_mfma_f32_16x16x4f32(bs1, mb1[m], mn, 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            f[m][t][j] = __builtin_fmaf(xdj[j], __builtin_fmaf(dd[m], (float)(dlo[j] + 8 * dhi[j] + 16 * d5[j]), mn[j]), f[m][t][j]);
-        }
-      }
-    } else if constexpr (kGrid) {
-      // one v_mfma_i32_16x16x32_i8 per 32-weight sub-block (K = the sub-block):
-      // lane group g holds 8-weight group l = g of every sub-block, grid values
-      // with their signs applied (conditional byte negate); the scale (2 ls + 1)
-      // multiplies the sub-block's integer dot per lane, the 1/8 (IQ2_XXS) or
-      // 1/4 (IQ3_XXS) is folded into d
-      long B[NM][8];
-      int S[NM][8];
-      float DD[NM];
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        constexpr float kf = T == T_IQ2_XXS ? 0.125f : 0.25f;
-        DD[m] = kf * h2f((uint16_t)(wcur[m].d & 0xffffu));
-#pragma unroll
-        for (int sb = 0; sb < 8; ++sb) {
-          uint32_t glo, ghi, aux;
-          if constexpr (T == T_IQ2_XXS) {
-            // sub-block sb: words 2sb (grid indices), 2sb + 1 (signs, scale)
-            const uint32_t aux0 = u4_get(wcur[m].q[sb >> 1], 2 * (sb & 1));
-            aux = u4_get(wcur[m].q[sb >> 1], 2 * (sb & 1) + 1);
-            const uint64_t gg = s_grid[(aux0 >> (8 * g)) & 0xffu];
-            glo = (uint32_t)gg;
-            ghi = (uint32_t)(gg >> 32);
-          } else {
-            // sub-block sb: grid-index bytes 8sb + 2g, +1 (two 4-value entries), word sb
-            const uint32_t iw = u4_get(wcur[m].gi[sb >> 1], 2 * (sb & 1) + (g >> 1));
-            aux = u4_get(wcur[m].sas[sb >> 2], sb & 3);
-            const uint32_t *g3 = reinterpret_cast<const uint32_t *>(s_grid);
-            glo = g3[(iw >> (16 * (g & 1))) & 0xffu];
-            ghi = g3[(iw >> (16 * (g & 1) + 8)) & 0xffu];
-          }
-          const uint64_t mm = s_signs[(aux >> (7 * g)) & 127u];
-          const uint32_t mlo = (uint32_t)mm, mhi = (uint32_t)(mm >> 32);
-          const uint32_t v0 = sign_bytes(glo, mlo), v1 = sign_bytes(ghi, mhi);
-          B[m][sb] = (long)(((uint64_t)v1 << 32) | v0);
-          S[m][sb] = 2 * (int)(aux >> 28) + 1;
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= nt) continue;
-        const int tok = 16 * t + n;
-        float xdj[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xdj[j] = s_xd[buf][16 * t + 4 * g + j];
-        long xa[8];
-#pragma unroll
-        for (int sb = 0; sb < 8; ++sb) xa[sb] = __builtin_bit_cast(long, xq8(buf, tok, 2 * sb + (g >> 1), g & 1));
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-          int isum[4] = {0, 0, 0, 0};
-#pragma unroll
-          for (int sb = 0; sb < 8; ++sb) {
-            const v4i_t z = {0, 0, 0, 0};
-            const v4i_t d = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa[sb], B[m][sb], z, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) isum[j] = __mul24(S[m][sb], d[j]) + isum[j];
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j) f[m][t][j] = __builtin_fmaf(xdj[j], DD[m] * (float)isum[j], f[m][t][j]);
-        }
-      }
-    } else if constexpr (T == T_IQ4_XS) {
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      const float d = h2f((uint16_t)(wcur[m].hdr.x & 0xffffu));
-      // chunk c = sub-blocks 2c (lane groups 0-1) and 2c + 1 (groups 2-3); group
-      // g takes the low (g even) or high nibbles of its sub-block's 16 qs bytes,
-      // through the value table; each chunk is issued twice, the other
-      // sub-block's half of B zeroed
-      const uint32_t keep0 = g < 2 ? 0xffffffffu : 0u;
-      const int ns = 4 * (g & 1);
-      v4i_t b0[4], b1[4];
-      int s0[4], s1[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint4 q = wcur[m].qs[c];
-        const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t v = lut16((qw[k] >> ns) & 0x0f0f0f0fu, tab[0], tab[1], tab[2], tab[3]);
-          b0[c][k] = (int)(v & keep0);
-          b1[c][k] = (int)(v & ~keep0);
-        }
-        s0[c] = iq4_scale(wcur[m].hdr.x, wcur[m].hdr.y, 2 * c);
-        s1[c] = iq4_scale(wcur[m].hdr.x, wcur[m].hdr.y, 2 * c + 1);
-      }
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= nt) continue;
-        const int tok = 16 * t + n;
-        int isum[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const v4i_t xa = xq16(buf, tok, 4 * c + g);
-          const v4i_t z = {0, 0, 0, 0};
-          const v4i_t d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa, b0[c], z, 0, 0, 0);
-          const v4i_t d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa, b1[c], z, 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) isum[j] = __mul24(s0[c], d0[j]) + __mul24(s1[c], d1[j]) + isum[j];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[m][t][j] = __builtin_fmaf(s_xd[buf][16 * t + 4 * g + j], d * (float)isum[j], f[m][t][j]);
-      }
+      slot = slot + 1 == ST ? 0 : slot + 1;
+      pslot = pslot + 1 == ST ? 0 : pslot + 1;
     }
-    } else if constexpr (T == T_Q6_K) {
+    wait_vm<0>();  // the requests past the last block land before the LDS is given up
+    if (row < a.nrows) {
+      // the lane holds (pair 16t + 4g + j, row)
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      const float d = h2f((uint16_t)(wcur[m].d & 0xffffu));
-      const uint32_t scb[4] = {wcur[m].sc.x, wcur[m].sc.y, wcur[m].sc.z, wcur[m].sc.w};
-      // B operand of the offset product: sc[row][sb] for sb = 4i + g
-      float mb[4];
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mb[i] = (float)(int)(int8_t)(scb[i] >> (8 * g));
-      // 6-bit values of the 8 sub-block pairs, each issued with the lane's half
-      // (groups 0-1: sub-block 2p, groups 2-3: 2p + 1) and zeros in the other
-      const uint32_t keep0 = g < 2 ? 0xffffffffu : 0u;
-      long b0[8], b1[8];
-      int s0[8], s1[8];
-#pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        const int h = p >> 2, G = p & 3;
-        const uint2 q = wcur[m].ql[2 * h + (p & 1)];
-        const uint2 hb = wcur[m].qh[h];
-        const uint32_t lx = G < 2 ? (q.x & 0x0f0f0f0fu) : ((q.x >> 4) & 0x0f0f0f0fu);
-        const uint32_t ly = G < 2 ? (q.y & 0x0f0f0f0fu) : ((q.y >> 4) & 0x0f0f0f0fu);
-        const uint32_t vx = lx | (((hb.x >> (2 * G)) & 0x03030303u) << 4);
-        const uint32_t vy = ly | (((hb.y >> (2 * G)) & 0x03030303u) << 4);
-        b0[p] = (long)(((uint64_t)(vy & keep0) << 32) | (vx & keep0));
-        b1[p] = (long)(((uint64_t)(vy & ~keep0) << 32) | (vx & ~keep0));
-        s0[p] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1)));
-        s1[p] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1) + 8));
-      }
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= nt) continue;
-        const int tok = 16 * t + n;
-        int isum[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int p = 0; p < 8; ++p) {
-          const long xa = __builtin_bit_cast(long, xq8(buf, tok, 2 * p + (g >> 1), g & 1));
-          const v4i_t z = {0, 0, 0, 0};
-          const v4i_t d0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, b0[p], z, 0, 0, 0);
-          const v4i_t d1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, b1[p], z, 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) isum[j] = __mul24(s0[p], d0[j]) + __mul24(s1[p], d1[j]) + isum[j];
+        for (int j = 0; j < 4; ++j) {
+          const long o = s_out[16 * t + 4 * g + j];
+          if (o < 0) continue;
+          a.out[o + row] = GATEUP ? silu_f32(f[0][t][j]) * f[NM - 1][t][j] : f[0][t][j];
         }
-        v4f_t off = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          off = __builtin_amdgcn_mfma_f32_16x16x4f32((float)bsum16(buf, tok, 4 * i + g), mb[i], off, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          f[m][t][j] = __builtin_fmaf(s_xd[buf][16 * t + 4 * g + j], d * (float)(isum[j] - 32 * (int)off[j]), f[m][t][j]);
-      }
-    }
-    } else {
-      // Q2_K: both matrices' operands first, then one pass over the token tiles
-      // (the activation tile and its bsums read once for gate and up)
-      v4i_t bq[NM][4];
-      float dd[NM], dm[NM], mb[NM][4];
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        dd[m] = h2f((uint16_t)(wcur[m].dd & 0xffffu));
-        dm[m] = h2f((uint16_t)(wcur[m].dd >> 16));
-        const uint32_t scb[4] = {wcur[m].sc.x, wcur[m].sc.y, wcur[m].sc.z, wcur[m].sc.w};
-        // B operand of the min product: m[row][sb] for sb = 4i + g
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mb[m][i] = -dm[m] * (float)((scb[i] >> (8 * g + 4)) & 15u);  // -dmin folded in (exact)
-        // scale-folded weights of the 4 chunks c = 2h + jp: plane j = 2jp + (g >> 1),
-        // sub-block 8h + 2j + (g & 1)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int h = c >> 1, jp = c & 1;
-          const int j = 2 * jp + (g >> 1);
-          const int sb = 8 * h + 2 * j + (g & 1);
-          const uint32_t sc = (scb[sb >> 2] >> (8 * (sb & 3))) & 15u;
-          const uint4 q = wcur[m].qs[h];
-          const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-          for (int k = 0; k < 4; ++k) bq[m][c][k] = (int)mul_bytes((qw[k] >> (2 * j)) & 0x03030303u, sc);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= nt) continue;
-        const int tok = 16 * t + n;
-        v4i_t xa[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) xa[c] = xq16(buf, tok, 4 * c + g);
-        float bs[4], xdj[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bs[i] = (float)bsum16(buf, tok, 4 * i + g);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xdj[j] = s_xd[buf][16 * t + 4 * g + j];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-          v4i_t isum = {0, 0, 0, 0};
-#pragma unroll
-          for (int c = 0; c < 4; ++c) isum = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[c], bq[m][c], isum, 0, 0, 0);
-          v4f_t mn = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mn = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[i], mb[m][i], mn, 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            f[m][t][j] = __builtin_fmaf(xdj[j], __builtin_fmaf(dd[m], (float)isum[j], mn[j]), f[m][t][j]);
-        }
-      }
     }
   };
-  // one block ahead: each step issues block b + 1's activations and weights and
-  // waits for all of it at its end.  The loop is unrolled by two, so the two
-  // weight register sets and activation buffers alternate without copies.
-  WBlk w0[NM], w1[NM];
-  load_w(0, w0);
-  dma_x(0, 0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the direct loads have landed
-  __syncthreads();
-  for (int b = 0;; b += 2) {
-    dma_x(b + 1, 1);  // buffer 1's readers finished at the last barrier
-    load_w(b + 1, w1);
-    step(0, w0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (b + 1 >= nb) break;
-    dma_x(b + 2, 0);
-    load_w(b + 2, w0);
-    step(1, w1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (b + 2 >= nb) break;
-  }
-  // lane holds (pair pc + 16t + 4g + j, row): store out[tok][k][row]
-  if (rv) {
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      if (t >= nt) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int pair = s_pair[16 * t + 4 * g + j];
-        if (pair < 0) continue;
-        const int tok = pair / Kp, k = pair % Kp;
-        const float v = GATEUP ? silu_f32(f[0][t][j]) * f[NM - 1][t][j] : f[0][t][j];
-        a.out[(size_t)tok * a.out_s + (size_t)k * a.out_k + row] = v;
-      }
-    }
+  if constexpr (TT == 2) {
+    if (nt == 1) body(std::integral_constant<int, 1>{});
+    else body(std::integral_constant<int, 2>{});
+  } else {
+    static_assert(TT == 4, "tiles per item");
+    if (nt == 1) body(std::integral_constant<int, 1>{});
+    else if (nt == 2) body(std::integral_constant<int, 2>{});
+    else if (nt == 3) body(std::integral_constant<int, 3>{});
+    else body(std::integral_constant<int, 4>{});
   }
 }
+
+// ---------------------------------------------------------------- launch
+
+// waves per workgroup: 8 with 64-pair items, 4 with 32-pair items, 1 where even their 64-row tiles leave CUs idle
+// (4 waves per SIMD in each case but Q5_K / Q6_K gate/up).  512 tokens, Q4_K gate/up: 64-pair items with 8 waves
+// 270 us, with 4 waves 294, 32-pair items 302; 333 tokens (21 pairs per expert) Q2_K: 182 / 197 / 174.
+template <int T, bool GU>
+void mmq_launch_t(int tt, int nw, unsigned items, const GemvArgs &a0, hipStream_t st) {
+  GemvArgs a = a0;
+  if (tt == 4) nw = 8;
+  a.row_tiles = (a.nrows + 16 * nw - 1) / (16 * nw);
+  const dim3 grid((unsigned)a.row_tiles * items);
+  if (tt == 4) hipLaunchKernelGGL((k_mmq<T, GU, 4, 8, 2>), grid, dim3(512), 0, st, a);
+  else if (nw == 1) hipLaunchKernelGGL((k_mmq<T, GU, 2, 1, 2>), grid, dim3(64), 0, st, a);
+  else hipLaunchKernelGGL((k_mmq<T, GU, 2, 4, 2>), grid, dim3(256), 0, st, a);
+}
+template <int T>
+void mmq_launch(bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st) {
+  if (gateup) mmq_launch_t<T, true>(tt, nw, items, a, st);
+  else mmq_launch_t<T, false>(tt, nw, items, a, st);
+}
+// per translation unit: false when the type is not instantiated there
+bool mmq_launch_a(int type, bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st);
+bool mmq_launch_b(int type, bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st);
+bool mmq_launch_c(int type, bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st);
+bool mmq_launch_d(int type, bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st);
 
 }  // namespace zm
