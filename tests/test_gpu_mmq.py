@@ -65,6 +65,7 @@ def _check(t, I, rows, sizes, offset=0, extra=()):
 @pytest.mark.parametrize("I,rows", [(256, 16), (512, 37), (768, 130), (1280, 64), (1792, 1)])
 def test_bucket_and_row_edges(t, I, rows):
     _check(t, I, rows, [1, 15, 16, 17, 31, 32, 33, 0, 2])                      # 32-pair items
+    _check(t, I, rows, [1, 0, 2, 15, 16, 3, 17, 7, 5, 9], extra=(-1, 10))      # 16-pair items
     _check(t, I, rows, [1, 16, 33, 47, 48, 49, 63, 64, 65, 129], extra=(-1, 10, 99))  # 64-pair items
 
 

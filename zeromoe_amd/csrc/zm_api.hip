@@ -262,11 +262,14 @@ int launch_gemv(int type, bool gateup, int np, const GemvArgs &a0, int n_groups,
 
 // ------------------------------------------------------------------ grouped MFMA dispatch
 
-// 16-pair tiles per work item: 64-pair items share the weight unpacking where
-// buckets are large, 32-pair items take fewer registers and less LDS.  512
-// tokens, Q4_K gate/up (32 pairs per expert): 260 against 289 us; 333 tokens
-// (21 pairs), Q3_K down: 155 against 126.
-int mmq_tiles(double avg_pairs) { return avg_pairs >= 32.0 ? 4 : 2; }
+// 16-pair tiles per work item, by the pairs per expert: 64-pair items share the
+// weight unpacking where buckets are large, 32-pair items take fewer registers
+// and less LDS, 16-pair items leave LDS for two blocks of weights per stage (at
+// 10 pairs per expert 3% of even loads exceed them and read their weights twice).
+// 64 / 32: 512 tokens, Q4_K gate/up (32 pairs) 260 / 289 us, 333 tokens (21
+// pairs), Q3_K down 155 / 126.  32 / 16: 98 tokens (6 pairs), IQ3_XXS gate/up 240
+// / 219; 24 tokens (2 pairs), Q6_K down 172 / 113; 333 tokens, Q2_K gate/up 171 / 284.
+int mmq_tiles(double avg_pairs) { return avg_pairs >= 32.0 ? 4 : (avg_pairs >= 10.0 ? 2 : 1); }
 // work items of n_pairs pairs over n_experts buckets: at most one partial run
 // per bucket besides the full ones
 int mmq_max_items(int n_pairs, int n_experts, int tok) {
@@ -283,7 +286,7 @@ bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int
                  size_t xq_rows, int nb) {
   if (n_pairs < MMQ_MIN_PAIRS || getenv_flag_off("ZEROMOE_MMQ")) return false;
   if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
-  if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 32 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
+  if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 16 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
   if (lo & (block_bytes(type) % 4 ? 1 : 3)) return false;
   return !w1 || !(((uintptr_t)w0 ^ (uintptr_t)w1) & 3);
@@ -445,7 +448,7 @@ size_t mmid_carve(const MmidShape &m, uint8_t *base, MmidWs *out) {
   w.pairs = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.active = b.take<int32_t>((size_t)m.E * 4);
   w.n_active = b.take<int32_t>(4);
-  w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 32) * 4);
+  w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 16) * 4);
   w.n_items = b.take<int32_t>(4);
   if (out) *out = w;
   return b.off + 256;
@@ -773,7 +776,7 @@ size_t layer_ws(const zm_moe_layer *L, int S, uint8_t *base, LayerWs *w) {
   t.pairs = b.take<int32_t>((size_t)S * K * 4);
   t.active = b.take<int32_t>((size_t)NS * 4);
   t.n_active = b.take<int32_t>(4);
-  t.items = b.take<int32_t>((size_t)mmq_max_items(S * K, NS, 32) * 4);
+  t.items = b.take<int32_t>((size_t)mmq_max_items(S * K, NS, 16) * 4);
   t.n_items = b.take<int32_t>(4);
   t.act = b.take<float>((size_t)S * K * F * 4);
   t.aq = b.take<uint8_t>((size_t)S * K * xrec_row_bytes(nbF));
@@ -1068,12 +1071,11 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     c.grid = d->grid;
     c.signs = d->signs;
     const int nps = S >= 4 ? 4 : (S >= 2 ? 2 : 1);
-    const int tt = mmq_tiles((double)S);
     // one-wave workgroups of 16 rows where 64-row tiles of 32 tokens would leave CUs idle
     const int cus = d->n_cu > 0 ? d->n_cu : 256;
     auto dense = [&](bool mmq, bool gu, const GemvArgs &v) {
       const bool few = (long)((v.nrows + 63) / 64) * ((S + 31) / 32) < cus;
-      const int t = few ? 2 : tt;
+      const int t = few ? 2 : mmq_tiles((double)S);
       return mmq ? launch_mmq(ts, gu, t, few ? 1 : 4, (S + 16 * t - 1) / (16 * t), v, ss)
                  : launch_gemv(ts, gu, nps, v, 1, ss);
     };

@@ -23,15 +23,15 @@
 // wave, and the lanes pick their fields out of LDS.  The slot is read at the
 // start of a block and its next block requested at once, so a request has the
 // whole block's arithmetic to land.  Activations are staged the same way, one
-// 304-byte record per pair and block (ST stages, one barrier per block).
-// Units per row are odd (Q6_K padded), and so is a record, counted in 16-byte
-// units: 16 rows read 16 different bank groups.
+// 304-byte record per pair and block (two stages, one barrier per stage; a third
+// stage gained nothing).  Units per row are odd (padded), and so is a record,
+// counted in 16-byte units: 16 rows read 16 different bank groups.
 // On the vector units the unpacking and the tile epilogue (about 100 + 25 per
 // tile instructions per matrix and block for Q4_K) are the floor at many pairs
 // per expert, the weight stream at few.
-//   512 tokens, Q4_K, skewed loads: gate/up 367 -> 280 us, down 185 -> 142 us
-//   333 tokens, even loads: Q2_K gate/up 230 -> 167 us; Q3_K down 888 (GEMV) -> 142 us
-//   24 tokens, Q4_K gate/up: 207 (GEMV) -> 144 us, 4.9 TB/s of weights
+//   512 tokens, Q4_K, skewed loads: gate/up 367 -> 260 us, down 185 -> 139 us
+//   333 tokens, even loads: Q2_K gate/up 230 -> 167 us; Q3_K down 888 (GEMV) -> 126 us
+//   24 tokens: Q4_K gate/up 207 (GEMV) -> 145 us, 4.9 TB/s; Q6_K down 168 (GEMV) -> 113 us, 4.5 TB/s
 //
 // Activation record of one 256-value block (k_quant_rec): 256 int8 | 16 f16
 // sums of 16 values (integers up to 2032: exact) | f32 d | pad.  The int8 of a
@@ -51,9 +51,9 @@
 // Their mins: imin = sum_sb m * bsum (f16 operands, exact f32 sums) on one
 //   v_mfma_f32_16x16x16_f16 (16 cycles; on f32 operands it took 2 to 4 of 32).
 //   f += d_x * (d * isum - dmin * imin), ggml's vec_dot combine.
-// Q6_K (signed 8-bit scale per 16 weights; 4 * (q - 32) is int8): one
-//   v_mfma_i32_16x16x32_i8 per 16-weight sub-block (half of B zeroed), scaled
-//   per lane on the integer sums.
+// Q6_K (signed 8-bit scale per 16 weights; 4 * (q - 32) is int8): two
+//   v_mfma_i32_16x16x32_i8 per pair of 16-weight sub-blocks (the first alone,
+//   then both), scaled per lane on the integer sums.
 // IQ2_XXS, IQ3_XXS, IQ4_XS (grid or table values, one scale per 32 weights): one
 //   v_mfma_i32_16x16x32_i8 per sub-block, scaled per lane.
 #pragma once
@@ -102,9 +102,11 @@ __device__ __forceinline__ void wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <class P>
+template <class P, int A>
 __device__ __forceinline__ P lds_get(const uint8_t *p) {
-  return *reinterpret_cast<const P *>(p);
+  P v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, A), sizeof(P));
+  return v;
 }
 // N dwords that start 0, 2 or 4 bytes past the dword p: N + 1 aligned dwords and
 // one byte permute each (sel: align_sel).  LDS reads at the 2-byte address itself
@@ -117,7 +119,7 @@ template <int N, int A>
 __device__ __forceinline__ Dwords<N> lds_get_at(const uint8_t *p, uint32_t sel) {
   uint32_t r[N + 1];
   __builtin_memcpy(r, __builtin_assume_aligned(p, A), 4 * N);
-  r[N] = lds_get<uint32_t>(p + 4 * N);
+  r[N] = lds_get<uint32_t, 4>(p + 4 * N);
   Dwords<N> o;
 #pragma unroll
   for (int i = 0; i < N; ++i) o.v[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
@@ -234,15 +236,15 @@ template <int T>
 constexpr bool mmq_dword() {
   return block_bytes(T) % 4 == 0;
 }
-// 16-byte units loaded per row and block (an extra 2 bytes where a block starts inside a dword)
-template <int T>
+// 16-byte units loaded per row and stage of C blocks (an extra 2 bytes where a block starts inside a dword)
+template <int T, int C>
 constexpr int mmq_load_units() {
-  return (block_bytes(T) + (mmq_dword<T>() ? 0 : 2) + 15) / 16;
+  return (C * block_bytes(T) + (mmq_dword<T>() ? 0 : 2) + 15) / 16;
 }
 // units of a row's slot: odd, so that 16 rows start in 16 different 16-byte bank groups
-template <int T>
+template <int T, int C>
 constexpr int mmq_units() {
-  return mmq_load_units<T>() | 1;
+  return mmq_load_units<T, C>() | 1;
 }
 
 // the fields of one block that a lane needs
@@ -296,46 +298,47 @@ struct MmqW<T_IQ4_XS> {  // d, scales_h, scales_l | the lane's 8 qs bytes of eac
   uint2 qs[8];
 };
 
-// p: the row's slot; al: the block's first byte in it (0 or 2, 0 for dword types)
-template <int T>
+// p: the dword of the row's slot that holds the block's first byte, al: that byte's place in it (0 or 2; 0 for dword
+// types); A: alignment of p
+template <int T, int A>
 __device__ __forceinline__ void mmq_read_w(const uint8_t *p, int al, int g, MmqW<T> &w) {
   const uint32_t sel = align_sel(al);
   if constexpr (T == T_Q4_K || T == T_Q5_K) {
     constexpr int QS = T == T_Q5_K ? 48 : 16;
-    w.hdr = lds_get<uint4>(p);
-    if constexpr (T == T_Q5_K) w.qh = lds_get<uint2>(p + 16 + 8 * g);
+    w.hdr = lds_get<uint4, A>(p);
+    if constexpr (T == T_Q5_K) w.qh = lds_get<uint2, (A < 8 ? A : 8)>(p + 16 + 8 * g);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w.qs[i] = lds_get<uint2>(p + QS + 32 * i + 8 * g);
+    for (int i = 0; i < 4; ++i) w.qs[i] = lds_get<uint2, (A < 8 ? A : 8)>(p + QS + 32 * i + 8 * g);
   } else if constexpr (T == T_Q2_K) {
-    w.sc = lds_get<uint4>(p);
+    w.sc = lds_get<uint4, A>(p);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get<uint4>(p + 16 + 32 * h + 16 * (g & 1));
-    w.dd = lds_get<uint32_t>(p + 80);
+    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get<uint4, A>(p + 16 + 32 * h + 16 * (g & 1));
+    w.dd = lds_get<uint32_t, 4>(p + 80);
   } else if constexpr (T == T_Q3_K) {
-    w.hm = lds_get_at<4, 16>(p + 16 * (g & 1), sel);
+    w.hm = lds_get_at<4, A>(p + 16 * (g & 1), sel);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get_at<4, 16>(p + 32 + 32 * h + 16 * (g & 1), sel);
-    w.s = lds_get_at<3, 16>(p + 96, sel);
-    w.d = lds_get<uint16_t>(p + 108 + al);
+    for (int h = 0; h < 2; ++h) w.qs[h] = lds_get_at<4, A>(p + 32 + 32 * h + 16 * (g & 1), sel);
+    w.s = lds_get_at<3, A>(p + 96, sel);
+    w.d = lds_get<uint16_t, 2>(p + 108 + al);
   } else if constexpr (T == T_Q6_K) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w.ql[i] = lds_get_at<2, 8>(p + 64 * (i >> 1) + 32 * (i & 1) + 8 * g, sel);
+    for (int i = 0; i < 4; ++i) w.ql[i] = lds_get_at<2, (A < 8 ? A : 8)>(p + 64 * (i >> 1) + 32 * (i & 1) + 8 * g, sel);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w.qh[h] = lds_get_at<2, 8>(p + 128 + 32 * h + 8 * g, sel);
-    w.sc = lds_get_at<4, 16>(p + 192, sel);
-    w.d = lds_get<uint16_t>(p + 208 + al);
+    for (int h = 0; h < 2; ++h) w.qh[h] = lds_get_at<2, (A < 8 ? A : 8)>(p + 128 + 32 * h + 8 * g, sel);
+    w.sc = lds_get_at<4, A>(p + 192, sel);
+    w.d = lds_get<uint16_t, 2>(p + 208 + al);
   } else if constexpr (T == T_IQ2_XXS) {
-    w.d = lds_get<uint16_t>(p + al);
-    w.q = lds_get_at<16, 16>(p, align_sel(2 + al));
+    w.d = lds_get<uint16_t, 2>(p + al);
+    w.q = lds_get_at<16, A>(p, align_sel(2 + al));
   } else if constexpr (T == T_IQ3_XXS) {
-    w.d = lds_get<uint16_t>(p + al);
+    w.d = lds_get<uint16_t, 2>(p + al);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) w.gi[i] = lds_get<uint16_t>(p + al + 2 + 8 * i + 2 * g);
-    w.sas = lds_get_at<8, 16>(p + 64, align_sel(2 + al));
+    for (int i = 0; i < 8; ++i) w.gi[i] = lds_get<uint16_t, 2>(p + al + 2 + 8 * i + 2 * g);
+    w.sas = lds_get_at<8, A>(p + 64, align_sel(2 + al));
   } else {
-    w.hdr = lds_get<uint2>(p);
+    w.hdr = lds_get<uint2, (A < 8 ? A : 8)>(p);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) w.qs[i] = lds_get<uint2>(p + 8 + 16 * i + 8 * (g & 1));
+    for (int i = 0; i < 8; ++i) w.qs[i] = lds_get<uint2, (A < 8 ? A : 8)>(p + 8 + 16 * i + 8 * (g & 1));
   }
 }
 
@@ -450,7 +453,9 @@ __device__ __forceinline__ void mmq_unpack(const MmqW<T> &w, int g, const uint64
     for (int h = 0; h < 2; ++h)  // the upper of the two top bits flipped: q ^ 32
       hb[h] = make_uint2(w.qh[h].v[0] ^ 0xaaaaaaaau, w.qh[h].v[1] ^ 0xaaaaaaaau);
     // pair p = sub-blocks 2p (lane groups 0-1), 2p + 1 (groups 2-3): low (G < 2)
-    // or high nibbles of ql bytes 64h + 32(p & 1) + 8g.., top bits 2G of qh bytes 32h + 8g..
+    // or high nibbles of ql bytes 64h + 32(p & 1) + 8g.., top bits 2G of qh bytes
+    // 32h + 8g...  The first operand is sub-block 2p alone, the second both:
+    // s0 D0 + s1 D1 = (s0 - s1) D0 + s1 (D0 + D1)
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
       const int h = p >> 2, G = p & 3;
@@ -459,9 +464,10 @@ __device__ __forceinline__ void mmq_unpack(const MmqW<T> &w, int g, const uint64
       const uint32_t vx = lx | ((hb[h].x << (6 - 2 * G)) & 0xc0c0c0c0u);
       const uint32_t vy = ly | ((hb[h].y << (6 - 2 * G)) & 0xc0c0c0c0u);
       o.b[2 * p] = (long)(((uint64_t)(vy & keep0) << 32) | (vx & keep0));
-      o.b[2 * p + 1] = (long)(((uint64_t)(vy & ~keep0) << 32) | (vx & ~keep0));
-      o.s[2 * p] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1)));
-      o.s[2 * p + 1] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1) + 8));
+      o.b[2 * p + 1] = (long)(((uint64_t)vy << 32) | vx);
+      const int s1 = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1) + 8));
+      o.s[2 * p] = (int)(int8_t)(scb[p >> 1] >> (16 * (p & 1))) - s1;
+      o.s[2 * p + 1] = s1;
     }
   } else if constexpr (T == T_IQ4_XS) {
     // sub-block sb: weights 8g .. 8g + 7 = low (g < 2) or high nibbles of its qs bytes 8(g & 1) .. +7
@@ -503,24 +509,25 @@ __device__ __forceinline__ void mmq_unpack(const MmqW<T> &w, int g, const uint64
 
 // ---------------------------------------------------------------- the kernel
 
-// TT: 16-pair tiles per item; NW: waves (16 weight rows each); ST: activation stages
-template <int T, bool GATEUP, int TT, int NW, int ST>
+// TT: 16-pair tiles per item; NW: waves (16 weight rows each); C: K blocks per stage
+template <int T, bool GATEUP, int TT, int NW, int C>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 ? 4 : 2))) void k_mmq(GemvArgs a) {
   constexpr int TOK = 16 * TT;
   constexpr int NM = GATEUP ? 2 : 1;
   constexpr int BB = block_bytes(T);
-  constexpr int UN = TOK * XUNITS;          // activation units of a stage
+  constexpr int UN = TOK * XUNITS;          // activation units of a block
   constexpr int NI = (UN + 64 * NW - 1) / (64 * NW);
-  constexpr int RU = mmq_units<T>(), LU = mmq_load_units<T>();
-  constexpr int NWI = (16 * RU + 63) / 64;  // weight loads per matrix and block
-  constexpr int WB = 16 * RU * 16;          // LDS bytes of one matrix block of a wave
+  constexpr int RU = mmq_units<T, C>(), LU = mmq_load_units<T, C>();
+  constexpr int NWI = (16 * RU + 63) / 64;  // weight loads per matrix and stage
+  constexpr int WB = 16 * RU * 16;          // LDS bytes of one matrix stage of a wave
+  // a stage starts on either half of a dword only where its bytes are no multiple of 4
+  constexpr bool kParity = (C * BB) % 4 != 0;
   constexpr bool kGrid = T == T_IQ2_XXS || T == T_IQ3_XXS;
   constexpr int NTAB = T == T_IQ2_XXS ? 256 : (T == T_IQ3_XXS ? 128 : (T == T_Q3_K ? 64 : 1));
-  static_assert(ST == 2 || ST == 3, "activation stages");
   // lookup tables first (largest alignment first), so that their addresses fold into the reads' offset field
   __shared__ __attribute__((aligned(kGrid ? 4096 : 16))) uint64_t s_tab[NTAB];
   __shared__ __attribute__((aligned(kGrid ? 2048 : 8))) uint64_t s_signs[kGrid ? 128 : 1];
-  __shared__ __attribute__((aligned(16))) uint8_t s_x[ST][TOK * XREC];
+  __shared__ __attribute__((aligned(16))) uint8_t s_x[2][C][TOK * XREC];
   __shared__ __attribute__((aligned(16))) uint8_t s_w[NW][NM][WB];
   __shared__ int s_xoff[TOK];   // byte offset of each pair's activation row (OOR: none)
   __shared__ long s_out[TOK];   // float offset of each pair's output row (-1: none)
@@ -594,7 +601,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
 #pragma unroll
   for (int m = 0; m < NM; ++m) rw[m] = dma_rsrc(wm[m] - sh, wbytes);
   const int al = mmq_dword<T>() ? 0 : (sh + row * (int)a.w_rstride) & 3;
-  int wo[mmq_dword<T>() ? 1 : 2][NWI];
+  int wo[kParity ? 2 : 1][NWI];
 #pragma unroll
   for (int i = 0; i < NWI; ++i) {
     const int u = i * 64 + lane;
@@ -602,18 +609,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
     const bool ok = r < 16 && p < LU && row0 + r < a.nrows;
     const int st = sh + (row0 + r) * (int)a.w_rstride;
     wo[0][i] = ok ? (st & ~3) + 16 * p : OOR;
-    if constexpr (!mmq_dword<T>()) wo[1][i] = ok ? ((st + BB) & ~3) + 16 * p : OOR;
+    if constexpr (kParity) wo[1][i] = ok ? ((st + C * BB) & ~3) + 16 * p : OOR;
   }
-  auto dma_w = [&](int m, int b) {
+  auto dma_w = [&](int m, int s) {  // stage s: blocks s * C ..
     const uint32_t base = lds_addr(&s_w[wave][m][0]);
-    const int par = mmq_dword<T>() ? 0 : b & 1;
-    const int so = (b - par) * BB;
+    const int par = kParity ? s & 1 : 0;
+    const int so = (s - par) * (C * BB);
 #pragma unroll
     for (int i = 0; i < NWI; ++i) {
       if (64 * (i + 1) > 16 * RU && 64 * i + lane >= 16 * RU) continue;
-      const int vo = par ? wo[mmq_dword<T>() ? 0 : 1][i] : wo[0][i];
-      // rows that fill their units exactly never reach past the resource, whose
-      // bounds the scalar offset is not part of; the others add it per lane
+      const int vo = par ? wo[kParity ? 1 : 0][i] : wo[0][i];
+      // a stage that is one block and fills its units exactly never reaches past
+      // the resource, whose bounds the scalar offset is not part of; the others
+      // add it per lane
       if constexpr (16 * LU == BB) dma_lds16(rw[m], base + i * 1024u, vo, so);
       else dma_lds16(rw[m], base + i * 1024u, vo == OOR ? OOR : vo + so, 0);
     }
@@ -625,12 +633,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
     constexpr int NC = mmq_chains<T>();
     constexpr int NIT = (NT * 16 * XUNITS + 64 * NW - 1) / (64 * NW);
     constexpr int NIM = (NT * 16 * XUNITS) / (64 * NW);  // of these, issued by every wave
-    auto dma_x = [&](int b, int slot) {
-      const uint32_t base = lds_addr(&s_x[0][0]) + slot * (uint32_t)sizeof(s_x[0]) + wave * 1024u;
+    auto dma_x = [&](int s, int slot) {
 #pragma unroll
-      for (int i = 0; i < NIT; ++i) {
-        if ((i * NW + NW) * 64 > UN && (i * NW + wave) * 64 + lane >= UN) continue;
-        dma_lds16(rx, base + i * NW * 1024u, xo[i], b * XREC);
+      for (int c = 0; c < C; ++c) {
+        const uint32_t base = lds_addr(&s_x[0][0][0]) + (slot * C + c) * (uint32_t)(TOK * XREC) + wave * 1024u;
+        const int so = min(s * C + c, nb - 1) * XREC;
+#pragma unroll
+        for (int i = 0; i < NIT; ++i) {
+          if ((i * NW + NW) * 64 > UN && (i * NW + wave) * 64 + lane >= UN) continue;
+          dma_lds16(rx, base + i * NW * 1024u, xo[i], so);
+        }
       }
     };
     v4i_t zero = {0, 0, 0, 0};
@@ -642,89 +654,100 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < 4; ++j) f[m][t][j] = 0.f;
-    // request order: x(0) W0(0) x(1) .. W1(0), then per block W0(b + 1), x(b + ST - 1), W1(b + 1)
+    // request order: x(0) W0(0) W1(0), then per stage W0(s + 1), x(s + 1), W1(s + 1)
+    const int ns = (nb + C - 1) / C;
     dma_x(0, 0);
     dma_w(0, 0);
-    if constexpr (ST > 2) dma_x(min(1, nb - 1), 1);
     if constexpr (NM == 2) dma_w(1, 0);
-    int slot = 0, pslot = ST - 1;
-    for (int b = 0; b < nb; ++b) {
-      // W0(b) and x(b) have landed once only younger requests are outstanding:
-      // W1(b) and, with a third stage, x(b + 1)
-      wait_barrier<(NM - 1) * NWI + (ST > 2 ? NIM : 0)>();
-      const uint8_t *xs = &s_x[0][0] + slot * sizeof(s_x[0]);
-      const int bn = min(b + 1, nb - 1);  // past the end: the last block again, never read
+    for (int s = 0; s < ns; ++s) {
+      wait_barrier<(NM - 1) * NWI>();  // W0(s) and x(s) have landed; younger: W1(s)
+      const uint8_t *xs0 = &s_x[0][0][0] + (s & 1) * (C * TOK * XREC);
+      const int sn = min(s + 1, ns - 1);  // past the end: the last stage again, never read
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
-        if (m == 1) wait_vm<NWI + NIM>();  // W1(b); younger: W0(b + 1) and x(b + ST - 1)
-        MmqW<T> w;
-        mmq_read_w<T>(wl + m * WB, mmq_dword<T>() ? 0 : al ^ (2 * (b & 1)), g, w);
+        if (m == 1) wait_vm<NWI + C * NIM>();  // W1(s); younger: W0(s + 1) and x(s + 1)
+        MmqW<T> w[C];
+        const int al0 = kParity ? al ^ (2 * (s & 1)) : al;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          // block c starts al0 + c * BB bytes into the slot
+          const int o = (c * BB) & ~3, r = (c * BB) & 3;
+          if (c == 0) mmq_read_w<T, 16>(wl + m * WB, al0, g, w[c]);
+          else if (r == 0) mmq_read_w<T, (BB % 16 ? (BB % 8 ? 4 : 8) : 16)>(wl + m * WB + o, al0, g, w[c]);
+          else mmq_read_w<T, 4>(wl + m * WB + o + (al0 ? 4 : 0), al0 ^ 2, g, w[c]);
+        }
         wait_lds();
-        dma_w(m, bn);                                               // the slot has been read
-        if (m == 0) dma_x(min(b + ST - 1, nb - 1), pslot);          // every wave is past block b - 1
-        MmqB<T> B;
-        mmq_unpack<T>(w, g, s_tab, s_signs, tab, B);
-        asm("" : "+v"(B.d));  // a plain f32 from here on
+        dma_w(m, sn);                                 // the slot has been read
+        if (m == 0) dma_x(sn, (s + 1) & 1);           // every wave is past stage s - 1
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const uint8_t *xt = xs + (16 * t + n) * XREC;
-          v4i_t xa[4];
+        for (int c = 0; c < C; ++c) {
+          if (C > 1 && s * C + c >= nb) break;
+          const uint8_t *xs = xs0 + c * (TOK * XREC);
+          MmqB<T> B;
+          mmq_unpack<T>(w[c], g, s_tab, s_signs, tab, B);
+          asm("" : "+v"(B.d));  // a plain f32 from here on
 #pragma unroll
-          for (int c = 0; c < 4; ++c) xa[c] = *reinterpret_cast<const v4i_t *>(xt + 64 * c + 16 * g);
-          float xd[4];
+          for (int t = 0; t < NT; ++t) {
+            const uint8_t *xt = xs + (16 * t + n) * XREC;
+            v4i_t xa[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) xd[j] = *reinterpret_cast<const float *>(xs + (16 * t + 4 * g + j) * XREC + 288);
-          if constexpr (mmq_folded<T>()) {
-            v4i_t D[NC];
+            for (int h = 0; h < 4; ++h) xa[h] = *reinterpret_cast<const v4i_t *>(xt + 64 * h + 16 * g);
+            float xd[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+            for (int j = 0; j < 4; ++j) xd[j] = *reinterpret_cast<const float *>(xs + (16 * t + 4 * g + j) * XREC + 288);
+            if constexpr (mmq_folded<T>()) {
+              v4i_t D[NC];
 #pragma unroll
-              for (int k = 0; k < NC; ++k)
-                D[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[c], B.b[k][c], c == 0 ? zero : D[k], 0, 0, 0);
-            v4f_t mn;
-            if constexpr (mmq_mins<T>()) {
-              const v4h_t bs = *reinterpret_cast<const v4h_t *>(xt + 256 + 8 * g);
-              mn = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, B.mn, __builtin_bit_cast(v4f_t, zero), 0, 0, 0);
-            }
+              for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              int is = D[0][j];
-              if constexpr (NC > 1) is += 8 * D[NC > 1 ? 1 : 0][j];
-              if constexpr (NC > 2) is += 16 * D[NC > 2 ? 2 : 0][j];
-              float v;
-              if constexpr (mmq_mins<T>()) v = __builtin_fmaf(B.d, (float)is, -(B.dmin * mn[j]));
-              else v = B.d * (float)is;
-              f[m][t][j] = __builtin_fmaf(xd[j], v, f[m][t][j]);
-              asm volatile("" : "+v"(f[m][t][j]));  // as below
-            }
-          } else {
-            int is[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-              for (int h = 0; h < 2; ++h) {  // half h of the chunk's operand: 32 values
-                const uint2 xh = h ? make_uint2((uint32_t)xa[c][2], (uint32_t)xa[c][3]) : make_uint2((uint32_t)xa[c][0], (uint32_t)xa[c][1]);
-                const long x8 = __builtin_bit_cast(long, xh);
-                constexpr int PS = MmqB<T>::NB / 8;  // sub-blocks per 32 values
-#pragma unroll
-                for (int q = 0; q < PS; ++q) {
-                  const int sb = (2 * c + h) * PS + q;
-                  const v4i_t D = __builtin_amdgcn_mfma_i32_16x16x32_i8(x8, B.b[sb], zero, 0, 0, 0);
-#pragma unroll
-                  for (int j = 0; j < 4; ++j) is[j] = __mul24(B.s[sb], D[j]) + is[j];
-                }
+                for (int k = 0; k < NC; ++k)
+                  D[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[q], B.b[k][q], q == 0 ? zero : D[k], 0, 0, 0);
+              v4f_t mn;
+              if constexpr (mmq_mins<T>()) {
+                const v4h_t bs = *reinterpret_cast<const v4h_t *>(xt + 256 + 8 * g);
+                mn = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, B.mn, __builtin_bit_cast(v4f_t, zero), 0, 0, 0);
               }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              f[m][t][j] = __builtin_fmaf(xd[j], B.d * (float)is[j], f[m][t][j]);
-              // computed here: left to float, the tile's operands stay live into the next matrix
-              asm volatile("" : "+v"(f[m][t][j]));
+              for (int j = 0; j < 4; ++j) {
+                int is = D[0][j];
+                if constexpr (NC > 1) is += 8 * D[NC > 1 ? 1 : 0][j];
+                if constexpr (NC > 2) is += 16 * D[NC > 2 ? 2 : 0][j];
+                float v;
+                if constexpr (mmq_mins<T>()) v = __builtin_fmaf(B.d, (float)is, -(B.dmin * mn[j]));
+                else v = B.d * (float)is;
+                f[m][t][j] = __builtin_fmaf(xd[j], v, f[m][t][j]);
+                asm volatile("" : "+v"(f[m][t][j]));  // as below
+              }
+            } else {
+              int is[4] = {0, 0, 0, 0};
+#pragma unroll
+              for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {  // half h of chunk k's operand: 32 values
+                  const uint2 xh = h ? make_uint2((uint32_t)xa[k][2], (uint32_t)xa[k][3]) : make_uint2((uint32_t)xa[k][0], (uint32_t)xa[k][1]);
+                  const long x8 = __builtin_bit_cast(long, xh);
+                  constexpr int PS = MmqB<T>::NB / 8;  // sub-blocks per 32 values
+#pragma unroll
+                  for (int q = 0; q < PS; ++q) {
+                    const int sb = (2 * k + h) * PS + q;
+                    const v4i_t D = __builtin_amdgcn_mfma_i32_16x16x32_i8(x8, B.b[sb], zero, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                      is[j] = __mul24(B.s[sb], D[j]) + is[j];
+                      asm("" : "+v"(is[j]));  // one multiply-add, not two multiplies and an add of three
+                    }
+                  }
+                }
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                f[m][t][j] = __builtin_fmaf(xd[j], B.d * (float)is[j], f[m][t][j]);
+                // computed here: left to float, the tile's operands stay live into the next matrix
+                asm volatile("" : "+v"(f[m][t][j]));
+              }
             }
           }
         }
       }
-      slot = slot + 1 == ST ? 0 : slot + 1;
-      pslot = pslot + 1 == ST ? 0 : pslot + 1;
     }
     wait_vm<0>();  // the requests past the last block land before the LDS is given up
     if (row < a.nrows) {
@@ -739,7 +762,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
         }
     }
   };
-  if constexpr (TT == 2) {
+  if constexpr (TT == 1) {
+    body(std::integral_constant<int, 1>{});
+  } else if constexpr (TT == 2) {
     if (nt == 1) body(std::integral_constant<int, 1>{});
     else body(std::integral_constant<int, 2>{});
   } else {
@@ -753,18 +778,32 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
 
 // ---------------------------------------------------------------- launch
 
-// waves per workgroup: 8 with 64-pair items, 4 with 32-pair items, 1 where even their 64-row tiles leave CUs idle
-// (4 waves per SIMD in each case but Q5_K / Q6_K gate/up).  512 tokens, Q4_K gate/up: 64-pair items with 8 waves
-// 270 us, with 4 waves 294, 32-pair items 302; 333 tokens (21 pairs per expert) Q2_K: 182 / 197 / 174.
+// K blocks per stage of 16-pair items: two where a row's block is no whole
+// number of 16-byte units, so that fewer 128-byte lines are fetched twice (a
+// line shared by two blocks of a row does not always stay in the L2 from one
+// stage to the next: 1.48 times the weights from memory for Q6_K).  24 tokens,
+// one / two blocks: Q6_K down 160 / 118 us, Q2_K gate/up 108 / 98, IQ3_XXS gate/up
+// 178 / 171, but IQ4_XS gate/up 168 / 188, Q4_K 147 / 150.
+template <int T>
+constexpr int mmq_stage() {
+  return T == T_Q4_K || T == T_IQ4_XS ? 1 : 2;
+}
+// waves per workgroup: 8 with 64-pair items (4 where 8 waves' weights leave LDS
+// for one workgroup only: Q5_K gate/up 288 against 304 us), else 4, or 1 where even their 64-row tiles leave CUs
+// idle.  512 tokens, Q4_K gate/up: 64-pair items with 8 waves 260 us, with 4
+// waves 294, 32-pair items 289; 333 tokens (21 pairs per expert), Q3_K down: 155
+// / 170 / 126.
 template <int T, bool GU>
 void mmq_launch_t(int tt, int nw, unsigned items, const GemvArgs &a0, hipStream_t st) {
+  constexpr int NW4 = GU && (T == T_Q5_K || T == T_Q6_K) ? 4 : 8;
   GemvArgs a = a0;
-  if (tt == 4) nw = 8;
+  if (tt == 4) nw = NW4;
   a.row_tiles = (a.nrows + 16 * nw - 1) / (16 * nw);
   const dim3 grid((unsigned)a.row_tiles * items);
-  if (tt == 4) hipLaunchKernelGGL((k_mmq<T, GU, 4, 8, 2>), grid, dim3(512), 0, st, a);
-  else if (nw == 1) hipLaunchKernelGGL((k_mmq<T, GU, 2, 1, 2>), grid, dim3(64), 0, st, a);
-  else hipLaunchKernelGGL((k_mmq<T, GU, 2, 4, 2>), grid, dim3(256), 0, st, a);
+  if (tt == 4) hipLaunchKernelGGL((k_mmq<T, GU, 4, NW4, 1>), grid, dim3(64 * NW4), 0, st, a);
+  else if (nw == 1) hipLaunchKernelGGL((k_mmq<T, GU, 2, 1, 1>), grid, dim3(64), 0, st, a);
+  else if (tt == 1) hipLaunchKernelGGL((k_mmq<T, GU, 1, 4, mmq_stage<T>()>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((k_mmq<T, GU, 2, 4, 1>), grid, dim3(256), 0, st, a);
 }
 template <int T>
 void mmq_launch(bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st) {
