@@ -280,8 +280,12 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 //   - rows, activations: 32-bit buffer offsets;
 //   - alignment: blocks of a multiple of 4 bytes are loaded by dwords, the
 //     others start on 2 bytes (gate and up alike within a dword);
-//   - pairs: below MMQ_MIN_PAIRS its workgroups are too few and too long.
-constexpr int MMQ_MIN_PAIRS = 64;
+//   - pairs: below MMQ_MIN_PAIRS its workgroups are too few and too long.  One
+//     op over 128 experts, GEMV / this, us, by pairs (1536 rows of 4096, Q4_K):
+//     8 13.1 / 21.5, 32 28.7 / 30.2, 48 40.5 / 40.5, 64 52.0 / 48.1, 128 97.1 /
+//     72.1; (4096 rows of 1536, Q6_K): 8 18.3 / 19.9, 32 45.3 / 44.0, 48 64.9 /
+//     57.5, 128 165.2 / 100.8.
+constexpr int MMQ_MIN_PAIRS = 40;
 bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride, int n_pairs,
                  size_t xq_rows, int nb) {
   if (n_pairs < MMQ_MIN_PAIRS || getenv_flag_off("ZEROMOE_MMQ")) return false;
@@ -303,9 +307,14 @@ int launch_mmq(int type, bool gateup, int tt, int nw, int items, const GemvArgs 
   HIP_OK(hipGetLastError());
   return 0;
 }
-void launch_items(const int32_t *n_active, const int32_t *active, const int32_t *offs, int32_t *items,
-                  int32_t *n_items, int tt, hipStream_t st) {
-  hipLaunchKernelGGL(k_mmq_items, dim3(1), dim3(1024), 0, st, n_active, active, offs, items, n_items, 16 * tt);
+// sort the pairs (b), quantize the rows of x, write the rows of skipped routes (a.out): one launch
+int launch_prep(PrepArgs a, hipStream_t st) {
+  const long blocks = (long)a.rows * a.nb;
+  a.q_wgs = (int)((blocks + PREP_QBLOCKS - 1) / PREP_QBLOCKS);
+  const int f_wgs = a.out ? (a.b.n_pairs + PREP_FPAIRS - 1) / PREP_FPAIRS : 0;
+  hipLaunchKernelGGL(k_prep, dim3(1 + a.q_wgs + f_wgs), dim3(1024), 0, st, a);
+  HIP_OK(hipGetLastError());
+  return 0;
 }
 
 // records for the grouped MFMA kernel, value order of `type`
@@ -412,8 +421,8 @@ int zm_bucket(const int32_t *ids, int S, int K, int E, int32_t *counts, int32_t 
   if (!ids || !counts || !offs || !pairs || !active || !n_active) return fail("zm_bucket: null argument");
   if (E <= 0 || E > BUCKET_MAX_E) return fail("zm_bucket: E out of range (1..%d)", BUCKET_MAX_E);
   if (S < 0 || K <= 0) return fail("zm_bucket: bad S/K");
-  hipLaunchKernelGGL(k_bucket, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, S * K, E, counts, offs, pairs,
-                     active, n_active);
+  const BucketArgs a{ids, (size_t)K, K, S * K, E, counts, offs, pairs, active, n_active, nullptr, nullptr, 0};
+  hipLaunchKernelGGL(k_bucket, dim3(1), dim3(1024), 0, (hipStream_t)stream, a);
   HIP_OK(hipGetLastError());
   return 0;
 }
@@ -425,8 +434,7 @@ int zm_bucket(const int32_t *ids, int S, int K, int E, int32_t *counts, int32_t 
 namespace {
 
 // A validated MUL_MAT_ID shape (see zm_mul_mat_id's rules) and the workspace
-// it needs: planar Q8_K rows of src1, a contiguous copy of ids, the bucket
-// arrays and the MFMA work list.
+// it needs: Q8_K rows of src1, the bucket arrays and the MFMA work list.
 struct MmidShape {
   int64_t I, O, E, n_ids, S, ne11, n_pairs, nq;
   int nb;
@@ -435,14 +443,13 @@ struct MmidShape {
 
 struct MmidWs {
   uint8_t *xq;
-  int32_t *idc, *counts, *offs, *pairs, *active, *n_active, *items, *n_items;
+  int32_t *counts, *offs, *pairs, *active, *n_active, *items, *n_items;
 };
 
 size_t mmid_carve(const MmidShape &m, uint8_t *base, MmidWs *out) {
   Bump b{base};
   MmidWs w{};
   w.xq = b.take<uint8_t>((size_t)m.nq * xrec_row_bytes(m.nb));  // planar rows are smaller
-  w.idc = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.counts = b.take<int32_t>((size_t)m.E * 4);
   w.offs = b.take<int32_t>((size_t)(m.E + 1) * 4);
   w.pairs = b.take<int32_t>((size_t)m.n_pairs * 4);
@@ -493,38 +500,30 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   mmid_carve(m, ws, &b);
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
-  const int64_t S = m.S, n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
+  const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
   const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
-  // 1. quantize src1 rows: (token t, row i11) -> row t*ne11 + i11
+  // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
-  auto quant = [&](const float *xt, int rows, uint8_t *y) {
-    return mmq ? launch_quant_rec(xt, x->nb[1] / 4, nb, rows, y, w->type, st)
-               : launch_quant(xt, x->nb[1] / 4, nb, rows, y, xrow, 1, st);
-  };
-  if (x->nb[2] == (size_t)ne11 * x->nb[1]) {
-    if (quant((const float *)x->data, (int)nq, b.xq)) return 0;
-  } else {
-    for (int64_t t = 0; t < S; ++t)
-      if (quant((const float *)((const char *)x->data + t * x->nb[2]), ne11, b.xq + (size_t)t * ne11 * xrow)) return 0;
-  }
-  // 2. ids -> contiguous [S][n_ids] (strided copy), then bucket
-  if (ids->nb[1] == (size_t)n_ids * 4) {
-    if (hipMemcpyAsync(b.idc, ids->data, (size_t)n_pairs * 4, hipMemcpyDeviceToDevice, st) != hipSuccess) return 0;
-  } else {
-    if (hipMemcpy2DAsync(b.idc, (size_t)n_ids * 4, ids->data, ids->nb[1], (size_t)n_ids * 4, (size_t)S,
-                         hipMemcpyDeviceToDevice, st) != hipSuccess)
-      return 0;
-  }
-  hipLaunchKernelGGL(k_bucket, dim3(1), dim3(1024), 0, st, b.idc, (int)n_pairs, (int)E, b.counts, b.offs, b.pairs,
-                     b.active, b.n_active);
-  // 3. skipped / invalid routes (pairs over grid x and y, each <= 65535)
-  {
-    const unsigned gy = (unsigned)std::min<int64_t>(n_pairs, 65535);
-    hipLaunchKernelGGL(k_fill_skipped, dim3((unsigned)std::min<int64_t>((O + 255) / 256, 64), gy), dim3(256), 0, st,
-                       b.idc, (size_t)n_ids, (size_t)1, (int)n_ids, (int)S, (int)E, (int)O, (float *)y->data,
-                       y->nb[2] / 4, y->nb[1] / 4);
-  }
-  // 4. bucketed GEMV or MFMA
+  const int groups = (int)std::min<int64_t>(E, n_pairs);
+  const int tt = mmq_tiles((double)n_pairs / groups);
+  PrepArgs p{};
+  p.b = BucketArgs{(const int32_t *)ids->data, ids->nb[1] / 4, (int)n_ids, (int)n_pairs, (int)E, b.counts, b.offs,
+                   b.pairs, b.active, b.n_active, b.items, b.n_items, mmq ? 16 * tt : 0};
+  p.x = (const float *)x->data;
+  p.x_tok = x->nb[2] / 4;
+  p.x_row = x->nb[1] / 4;
+  p.ne11 = ne11;
+  p.nb = nb;
+  p.rows = (int)nq;
+  p.y = b.xq;
+  p.y_rstride = xrow;
+  p.order = mmq ? mmq_order(w->type) : -1;
+  p.out = (float *)y->data;
+  p.out_s = y->nb[2] / 4;
+  p.out_k = y->nb[1] / 4;
+  p.O = (int)O;
+  if (launch_prep(p, st)) return 0;
+  // 2. bucketed GEMV or MFMA
   GemvArgs a{};
   a.w0 = (const uint8_t *)w->data;
   a.w_estride = w->nb[2];
@@ -544,10 +543,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   a.out_k = y->nb[1] / 4;
   a.grid = d->grid;
   a.signs = d->signs;
-  const int groups = (int)std::min<int64_t>(E, n_pairs);
   if (mmq) {
-    const int tt = mmq_tiles((double)n_pairs / groups);
-    launch_items(b.n_active, b.active, b.offs, b.items, b.n_items, tt, st);
     a.items = b.items;
     a.n_items = b.n_items;
     a.xq_bytes = (uint32_t)((size_t)nq * xrow);
@@ -1039,7 +1035,27 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
                : launch_quant(v, (size_t)n, n / QK, rows, y, q8_row_bytes(n / QK), 1, q);
   };
   auto qrow = [](bool rec, int nb) { return rec ? xrec_row_bytes(nb) : q8_row_bytes(nb); };
-  if (quant(mmq_g, L->type_gate, x, H, S, w.xq, st)) return -1;
+  const int groups = std::min(NS, S * K);
+  const int tt = mmq_tiles((double)(S * K) / groups);
+  {
+    PrepArgs p{};
+    p.b = BucketArgs{ids, (size_t)K, K, S * K, NS, w.counts, w.offs, w.pairs, w.active, w.n_active, w.items,
+                     w.n_items, mmq_g || mmq_d ? 16 * tt : 0};
+    p.x = x;
+    p.x_tok = p.x_row = (size_t)H;
+    p.ne11 = 1;
+    p.nb = nbH;
+    p.rows = S;
+    p.y = w.xq;
+    p.y_rstride = qrow(mmq_g, nbH);
+    p.order = mmq_g ? mmq_order(L->type_gate) : -1;
+    // skipped routes (slot table -1) read as zero rows; router ids are always valid otherwise
+    p.out = L->route_map ? w.y : nullptr;
+    p.out_s = (size_t)K * H;
+    p.out_k = (size_t)H;
+    p.O = H;
+    if (launch_prep(p, st)) return -1;
+  }
   // shared expert (dense over all tokens) on the side stream: it needs only
   // the Q8_K rows of x, and its gate/up, act quantization and down overlap
   // the router-dependent kernels; the combine waits for it
@@ -1102,10 +1118,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     if (launch_shared(d->side)) return -1;
     HIP_OK(hipEventRecord(d->ev_join, d->side));
   }
-  hipLaunchKernelGGL(k_bucket, dim3(1), dim3(1024), 0, st, ids, S * K, NS, w.counts, w.offs, w.pairs, w.active,
-                     w.n_active);
   // gate/up + SwiGLU
-  const int groups = std::min(NS, S * K);
   const int np = pick_np(S * K, NS);
   GemvArgs a{};
   a.w0 = (const uint8_t *)L->w_gate;
@@ -1128,9 +1141,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   a.out_k = F;
   a.grid = d->grid;
   a.signs = d->signs;
-  const int tt = mmq_tiles((double)(S * K) / groups);
   const int max_items = mmq_max_items(S * K, NS, 16 * tt);
-  if (mmq_g || mmq_d) launch_items(w.n_active, w.active, w.offs, w.items, w.n_items, tt, st);
   a.items = w.items;
   a.n_items = w.n_items;
   if (mmq_g ? launch_mmq(L->type_gate, true, tt, 4, max_items, a, st)
@@ -1138,10 +1149,6 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     return -1;
   // act -> Q8_K
   if (quant(mmq_d, L->type_down, w.act, F, S * K, w.aq, st)) return -1;
-  // skipped routes (slot table -1) read as zero rows; router ids are always valid otherwise
-  if (L->route_map)
-    hipLaunchKernelGGL(k_fill_skipped, dim3((unsigned)std::min((H + 255) / 256, 64), (unsigned)std::min(S * K, 65535)), dim3(256), 0,
-                     st, ids, (size_t)K, (size_t)1, K, S, NS, H, w.y, (size_t)K * H, (size_t)H);
   // down
   GemvArgs b = a;
   b.w0 = (const uint8_t *)L->w_down;

@@ -100,6 +100,18 @@ __device__ __forceinline__ void store_q8_16(uint8_t *row, int nb, int blk, const
   reinterpret_cast<int16_t *>(row + q8_bs_off(nb))[blk * 16 + l16] = (int16_t)o.bsum;
 }
 
+// 16 consecutive floats, 16-byte aligned
+__device__ __forceinline__ void load16(const float *x, float (&v)[16]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 f = reinterpret_cast<const float4 *>(x)[i];
+    v[4 * i] = f.x;
+    v[4 * i + 1] = f.y;
+    v[4 * i + 2] = f.z;
+    v[4 * i + 3] = f.w;
+  }
+}
+
 // rows x nb blocks, 16 lanes per block (quant_block16); planar != 0 writes the
 // internal planar layout, else ggml block_q8_K
 static __global__ __launch_bounds__(256) void k_quant_q8K(const float *__restrict__ x, size_t x_rstride, int nb, int rows,
@@ -108,16 +120,8 @@ static __global__ __launch_bounds__(256) void k_quant_q8K(const float *__restric
   const int gb = blockIdx.x * 16 + (threadIdx.x >> 4);
   const int row = gb / nb, b = gb % nb;
   if (row >= rows) return;
-  const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)row * x_rstride + (size_t)b * QK + 16 * l16);
   float v[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float4 f = src[i];
-    v[4 * i] = f.x;
-    v[4 * i + 1] = f.y;
-    v[4 * i + 2] = f.z;
-    v[4 * i + 3] = f.w;
-  }
+  load16(x + (size_t)row * x_rstride + (size_t)b * QK + 16 * l16, v);
   const Q8Out16 o = quant_block16(v, l16);
   uint8_t *yr = y + (size_t)row * y_rstride;
   if (planar) {
@@ -481,47 +485,72 @@ static __global__ __launch_bounds__(256) void k_router(RouterArgs a, int S) {
 
 // ============================================================ bucketing
 //
-// Stable counting sort of the flat pair ids p = s*K + k by expert, the CSR of
+// Stable counting sort of the pairs p = s*K + k by expert, the CSR of
 // /root/reference/core/batched_dispatch_pipeline.cpp:1181-1202 (token-major
-// inside each bucket).  One workgroup of 1024 threads; pairs are ranked in
-// chunks of 1024 with a wave "match" loop (ballot per distinct expert) plus
-// per-wave counts, so the order is exactly the sequential one.
+// inside each bucket).  One workgroup of 16 waves; each wave takes a contiguous
+// run of the pairs, counts it per expert, and after the scans over waves and
+// experts places it 64 pairs at a time (a pair's rank among the wave's lanes
+// with its expert comes from one ballot per id bit), so the order is exactly the
+// sequential one.  A latency chain: five workgroup barriers whatever the pair
+// count (four per 1024 pairs before: 2048 tokens x 8 33.5 -> 11 us with the work
+// list below, 512 x 8 10.2 + 4.7 for the list -> 9.5).
 constexpr int BUCKET_MAX_E = 512;
+constexpr int BUCKET_CH = 16;  // 64-pair chunks per wave whose ids stay in registers
 
-// Every thread reads its pairs' expert ids once (pair c * 1024 + tid for chunk
-// c, up to BUCKET_CH chunks held in registers; larger inputs re-read ids per
-// chunk), so the count, scan and ranking passes wait for memory only once.
-constexpr int BUCKET_CH = 8;
+struct BucketArgs {
+  const int32_t *ids;  // of pair p: ids[(p / K) * id_s + p % K]
+  size_t id_s;
+  int K, n_pairs, E;
+  int32_t *counts, *offs, *pairs, *active, *n_active;
+  // work items of the grouped MFMA kernel (tok pairs each; 0: none): expert |
+  // (first pair offset within the bucket) << 12, largest first -- full runs,
+  // then every expert's remaining run in descending order of its 16-pair tiles,
+  // so the short items fill the tail of the launch.  The order of items of one
+  // size is not fixed; no result depends on it (every item writes its own pairs).
+  int32_t *items, *n_items;
+  int tok;
+};
 
-static __global__ __launch_bounds__(1024) void k_bucket(const int32_t *__restrict__ ids, int n_pairs, int E,
-                                                 int32_t *__restrict__ counts, int32_t *__restrict__ offs,
-                                                 int32_t *__restrict__ pairs, int32_t *__restrict__ active,
-                                                 int32_t *__restrict__ n_active) {
-  __shared__ int cnt[BUCKET_MAX_E];
-  __shared__ int base[BUCKET_MAX_E];
-  __shared__ int wcnt[16][BUCKET_MAX_E];
+struct BucketLds {
+  int cnt[16][BUCKET_MAX_E];
+  int tot[BUCKET_MAX_E], off[BUCKET_MAX_E];
+  int hist[18], cur[18];  // size classes of items: 1..16 tiles of a partial run, 17 = full run
+};
+
+__device__ __forceinline__ void bucket_wg(const BucketArgs &a, BucketLds &l) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int nch = (n_pairs + 1023) / 1024;
+  const int seg = (a.n_pairs + 1023) / 1024 * 64;  // pairs per wave
+  const int p0 = w * seg, p1 = min(p0 + seg, a.n_pairs);
+  auto load = [&](int p) {
+    if (p >= p1) return -1;
+    const int s = a.id_s == (size_t)a.K ? 0 : p / a.K;
+    const int e = a.ids[s ? (size_t)s * a.id_s + (p - s * a.K) : (size_t)p];
+    return e >= 0 && e < a.E ? e : -1;
+  };
   int eid[BUCKET_CH];
 #pragma unroll
-  for (int c = 0; c < BUCKET_CH; ++c) {
-    const int i = c * 1024 + tid;
-    const int e = i < n_pairs ? ids[i] : -1;
-    eid[c] = e >= 0 && e < E ? e : -1;
-  }
-  for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+  for (int c = 0; c < BUCKET_CH; ++c) eid[c] = 64 * c < seg ? load(p0 + 64 * c + lane) : -1;
+  for (int i = tid; i < 16 * a.E; i += 1024) l.cnt[i / a.E][i % a.E] = 0;
+  if (tid < 18) l.hist[tid] = 0;
   __syncthreads();
-  for (int c = 0; c < nch; ++c) {
-    const int i = c * 1024 + tid;
-    int e = -1;
-    if (c < BUCKET_CH) {
 #pragma unroll
-      for (int q = 0; q < BUCKET_CH; ++q) e = q == c ? eid[q] : e;
-    } else if (i < n_pairs) {
-      e = ids[i];
-      e = e >= 0 && e < E ? e : -1;
+  for (int c = 0; c < BUCKET_CH; ++c)
+    if (eid[c] >= 0) atomicAdd(&l.cnt[w][eid[c]], 1);
+  for (int p = p0 + 64 * BUCKET_CH + lane; p < p1; p += 64) {
+    const int e = load(p);
+    if (e >= 0) atomicAdd(&l.cnt[w][e], 1);
+  }
+  __syncthreads();
+  // per expert: exclusive scan over the waves
+  if (tid < a.E) {
+    int run = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int c = l.cnt[v][tid];
+      l.cnt[v][tid] = run;
+      run += c;
     }
-    if (e >= 0) atomicAdd(&cnt[e], 1);
+    l.tot[tid] = run;
   }
   __syncthreads();
   if (w == 0) {
@@ -531,7 +560,7 @@ static __global__ __launch_bounds__(1024) void k_bucket(const int32_t *__restric
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int e = lane * 8 + j;
-      local[j] = e < E ? cnt[e] : 0;
+      local[j] = e < a.E ? l.tot[e] : 0;
       acc += local[j];
       nz += local[j] > 0;
     }
@@ -549,58 +578,72 @@ static __global__ __launch_bounds__(1024) void k_bucket(const int32_t *__restric
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int e = lane * 8 + j;
-      if (e < E) {
-        offs[e] = run;
-        base[e] = run;
-        counts[e] = local[j];
-        if (local[j] > 0) active[runz++] = e;
+      if (e < a.E) {
+        l.off[e] = run;
+        a.offs[e] = run;
+        a.counts[e] = local[j];
+        if (local[j] > 0) a.active[runz++] = e;
         run += local[j];
       }
     }
     if (lane == 63) {
-      offs[E] = incl;
-      *n_active = inz;
+      a.offs[a.E] = incl;
+      *a.n_active = inz;
     }
   }
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int nbits = E > 1 ? 32 - __builtin_clz((unsigned)(E - 1)) : 1;  // bits of an expert id
-  for (int c = 0; c < nch; ++c) {
-    for (int e = lane; e < E; e += 64) wcnt[w][e] = 0;
-    const int i = c * 1024 + tid;
-    int e = -1;
-    if (c < BUCKET_CH) {
-#pragma unroll
-      for (int q = 0; q < BUCKET_CH; ++q) e = q == c ? eid[q] : e;
-    } else if (i < n_pairs) {
-      e = ids[i];
-      e = e >= 0 && e < E ? e : -1;
+  // item classes of expert tid (its last wave's threads run beside the scan above)
+  int nfull = 0, key = 0;
+  if (a.tok > 0 && tid < a.E) {
+    const int c = l.tot[tid];
+    nfull = c / a.tok;
+    key = (c - nfull * a.tok + 15) / 16;  // 0: no partial run
+    if (nfull) atomicAdd(&l.hist[17], nfull);
+    if (key) atomicAdd(&l.hist[key], 1);
+  }
+  __syncthreads();
+  if (a.tok > 0 && tid == 0) {
+    int run = 0;
+    for (int k = 17; k >= 1; --k) {
+      l.cur[k] = run;
+      run += l.hist[k];
     }
+    *a.n_items = run;
+  }
+  // place the pairs
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const int nbits = a.E > 1 ? 32 - __builtin_clz((unsigned)(a.E - 1)) : 1;  // bits of an expert id
+  auto place = [&](int p, int e) {
     const bool valid = e >= 0;
-    __syncthreads();  // (first chunk: also the scan's base[] before it is read)
-    // rank among the earlier lanes of this wave with the same expert: the
-    // lanes holding the same id are the intersection, over the id's bits, of
-    // one ballot per bit (or its complement), so no loop over distinct ids
     uint64_t m = __ballot(valid);
     for (int j = 0; j < nbits; ++j) {
       const uint64_t bj = __ballot(valid && ((e >> j) & 1));
       m &= ((e >> j) & 1) ? bj : ~bj;
     }
     const int rank = __builtin_popcountll(m & lt_mask);
-    if (valid && rank == 0) wcnt[w][e] = __builtin_popcountll(m);
+    if (valid) a.pairs[l.off[e] + l.cnt[w][e] + rank] = p;
+    stage_sync();  // every lane has read its base before it moves on
+    if (valid && rank == 0) l.cnt[w][e] += __builtin_popcountll(m);
+    stage_sync();
+  };
+#pragma unroll
+  for (int c = 0; c < BUCKET_CH; ++c)
+    if (p0 + 64 * c < p1) place(p0 + 64 * c + lane, eid[c]);
+  for (int p = p0 + 64 * BUCKET_CH; p < p1; p += 64) place(p + lane, load(p + lane));
+  if (a.tok > 0) {
     __syncthreads();
-    if (valid) {
-      int r = base[e] + rank;
-      for (int w2 = 0; w2 < w; ++w2) r += wcnt[w2][e];
-      pairs[r] = i;
+    if (tid < a.E) {
+      if (nfull) {
+        const int q0 = atomicAdd(&l.cur[17], nfull);
+        for (int q = 0; q < nfull; ++q) a.items[q0 + q] = tid | ((q * a.tok) << 12);
+      }
+      if (key) a.items[atomicAdd(&l.cur[key], 1)] = tid | ((nfull * a.tok) << 12);
     }
-    __syncthreads();
-    for (int e2 = tid; e2 < E; e2 += 1024) {
-      int add = 0;
-      for (int w2 = 0; w2 < 16; ++w2) add += wcnt[w2][e2];
-      base[e2] += add;
-    }
-    __syncthreads();  // wcnt is cleared, and base read, by the next chunk
   }
+}
+
+static __global__ __launch_bounds__(1024) void k_bucket(BucketArgs a) {
+  __shared__ BucketLds l;
+  bucket_wg(a, l);
 }
 
 // ============================================================ bucketed GEMV
@@ -785,20 +828,6 @@ static __global__ __launch_bounds__(256) void k_combine(const float *__restrict_
     acc.w = acc.w + v.w;
   }
   *reinterpret_cast<float4 *>(out + (size_t)s * H + h) = acc;
-}
-
-// zero (negative id) or NaN (id >= n_experts) rows of routes the GEMV skips
-// (patches/ggml/0002...:50-54; kernels/quant/kquant_matmul.cu:660-663)
-static __global__ void k_fill_skipped(const int32_t *__restrict__ ids, size_t id_s, size_t id_k, int n_ids, int S,
-                               int n_experts, int O, float *out, size_t out_s, size_t out_k) {
-  // pairs are strided over grid y (at most 65535 rows of workgroups)
-  for (int pair = blockIdx.y; pair < n_ids * S; pair += gridDim.y) {
-    const int s = pair / n_ids, k = pair % n_ids;
-    const int e = ids[s * id_s + k * id_k];
-    if (e >= 0 && e < n_experts) continue;
-    const float v = e < 0 ? 0.0f : __int_as_float(0x7fc00000);
-    for (int r = blockIdx.x * 256 + threadIdx.x; r < O; r += gridDim.x * 256) out[s * out_s + k * out_k + r] = v;
-  }
 }
 
 // ============================================================ fp32 router GEMV

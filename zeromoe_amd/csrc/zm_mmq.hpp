@@ -148,26 +148,9 @@ __host__ __device__ constexpr size_t xrec_row_bytes(int nb) { return (size_t)nb 
 // value order of a record's int8: 0 natural, 1 the 8-byte groups of the two 32-value halves of a chunk alternating
 __host__ __device__ constexpr int mmq_order(int type) { return type == T_Q2_K || type == T_Q3_K ? 0 : 1; }
 
-// f32 rows -> records, 16 lanes per block
-static __global__ __launch_bounds__(256) void k_quant_rec(const float *__restrict__ x, size_t x_rstride, int nb,
-                                                          int rows, uint8_t *__restrict__ y, size_t y_rstride,
-                                                          int order) {
-  const int l16 = threadIdx.x & 15;
-  const int gb = blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int row = gb / nb, b = gb % nb;
-  if (row >= rows) return;
-  const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)row * x_rstride + (size_t)b * QK + 16 * l16);
-  float v[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float4 f = src[i];
-    v[4 * i] = f.x;
-    v[4 * i + 1] = f.y;
-    v[4 * i + 2] = f.z;
-    v[4 * i + 3] = f.w;
-  }
-  const Q8Out16 o = quant_block16(v, l16);
-  uint8_t *r = y + (size_t)row * y_rstride + (size_t)b * XREC;
+// 16 values of block b of a record row (the lane's share of quant_block16)
+__device__ __forceinline__ void store_rec16(uint8_t *row, int b, const Q8Out16 &o, int l16, int order) {
+  uint8_t *r = row + (size_t)b * XREC;
   if (order == 0) {
     *reinterpret_cast<uint4 *>(r + 16 * l16) = o.q;
   } else {  // values 16 * l16 .. +15 are groups 2q, 2q + 1 of half h of chunk c
@@ -178,53 +161,79 @@ static __global__ __launch_bounds__(256) void k_quant_rec(const float *__restric
   reinterpret_cast<_Float16 *>(r + 256)[l16] = (_Float16)(float)o.bsum;
   if (l16 == 0) *reinterpret_cast<float *>(r + 288) = o.d;
 }
+// f32 rows -> records, 16 lanes per block
+static __global__ __launch_bounds__(256) void k_quant_rec(const float *__restrict__ x, size_t x_rstride, int nb,
+                                                          int rows, uint8_t *__restrict__ y, size_t y_rstride,
+                                                          int order) {
+  const int l16 = threadIdx.x & 15;
+  const int gb = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int row = gb / nb, b = gb % nb;
+  if (row >= rows) return;
+  float v[16];
+  load16(x + (size_t)row * x_rstride + (size_t)b * QK + 16 * l16, v);
+  store_rec16(y + (size_t)row * y_rstride, b, quant_block16(v, l16), l16, order);
+}
 
-// ---------------------------------------------------------------- work items
+// ---------------------------------------------------------------- preparation
+//
+// What a bucketed product needs before it, in one launch: workgroup 0 sorts the
+// pairs (and cuts the work list), the next q_wgs quantize the rows of src1, the
+// rest write the rows of skipped routes (id < 0: zeros, id >= E: NaN;
+// patches/ggml/0002...:50-54, kernels/quant/kquant_matmul.cu:660-663).
+struct PrepArgs {
+  BucketArgs b;
+  // src1: row r = token r / ne11, slot r % ne11 at x[token * x_tok + slot * x_row]
+  const float *x;
+  size_t x_tok, x_row;
+  int ne11, nb, rows;
+  uint8_t *y;
+  size_t y_rstride;
+  int order;  // record order, or -1: planar rows
+  int q_wgs;
+  // output rows of skipped routes (out null: none)
+  float *out;
+  size_t out_s, out_k;
+  int O;
+};
+constexpr int PREP_QBLOCKS = 64;  // 256-value blocks quantized per workgroup
+constexpr int PREP_FPAIRS = 64;   // pairs looked through per workgroup, 4 per wave
 
-// Every active expert's bucket cut into runs of `tok` pairs, item = expert |
-// (first pair offset within the bucket) << 12, largest first: full runs, then
-// every expert's remaining run in descending order of its 16-pair tiles, so the
-// short items fill the tail of the launch.  The order of items with the same
-// size is not fixed; no result depends on it (every item writes its own pairs).
-// One workgroup; needs n_active <= 1024 and tok <= 256.
-static __global__ __launch_bounds__(1024) void k_mmq_items(const int32_t *__restrict__ n_active,
-                                                           const int32_t *__restrict__ active,
-                                                           const int32_t *__restrict__ offs,
-                                                           int32_t *__restrict__ items, int32_t *__restrict__ n_items,
-                                                           int tok) {
-  constexpr int NK = 18;  // size classes: 1..16 tiles of a partial run, 17 = full run
-  __shared__ int hist[NK], cur[NK];
-  const int tid = threadIdx.x;
-  if (tid < NK) hist[tid] = 0;
-  __syncthreads();
-  const int na = *n_active;
-  const int tt = tok / 16;
-  int e = 0, nfull = 0, rem = 0, key = 0;
-  if (tid < na) {
-    e = active[tid];
-    const int cnt = offs[e + 1] - offs[e];
-    nfull = cnt / tok;
-    rem = cnt - nfull * tok;
-    key = (rem + 15) / 16;  // 0: no partial run
-    if (nfull) atomicAdd(&hist[NK - 1], nfull);
-    if (key) atomicAdd(&hist[key], 1);
+static __global__ __launch_bounds__(1024) void k_prep(PrepArgs a) {
+  __shared__ BucketLds l;
+  if (blockIdx.x == 0) {
+    bucket_wg(a.b, l);
+    return;
   }
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int k = NK - 1; k >= 1; --k) {
-      cur[k] = run;
-      run += (k == NK - 1 || k <= tt) ? hist[k] : 0;
-    }
-    *n_items = run;
+  const int wg = (int)blockIdx.x - 1;
+  if (wg < a.q_wgs) {
+    const int l16 = threadIdx.x & 15;
+    const long gb = (long)wg * PREP_QBLOCKS + (threadIdx.x >> 4);
+    const int row = (int)(gb / a.nb), b = (int)(gb - (long)row * a.nb);
+    if (row >= a.rows) return;
+    const int t = row / a.ne11, i = row - t * a.ne11;
+    float v[16];
+    load16(a.x + (size_t)t * a.x_tok + (size_t)i * a.x_row + (size_t)b * QK + 16 * l16, v);
+    const Q8Out16 o = quant_block16(v, l16);
+    uint8_t *yr = a.y + (size_t)row * a.y_rstride;
+    if (a.order < 0) store_q8_16(yr, a.nb, b, o, l16);
+    else store_rec16(yr, b, o, l16, a.order);
+    return;
   }
-  __syncthreads();
-  if (tid < na) {
-    if (nfull) {
-      const int p = atomicAdd(&cur[NK - 1], nfull);
-      for (int q = 0; q < nfull; ++q) items[p + q] = e | ((q * tok) << 12);
-    }
-    if (key) items[atomicAdd(&cur[key], 1)] = e | ((nfull * tok) << 12);
+  const int lane = threadIdx.x & 63;
+  const int p0 = (wg - a.q_wgs) * PREP_FPAIRS + 4 * (int)(threadIdx.x >> 6);
+  int e = 0;
+  if (lane < 4 && p0 + lane < a.b.n_pairs) {
+    const int p = p0 + lane, s = p / a.b.K;
+    e = a.b.ids[(size_t)s * a.b.id_s + (p - s * a.b.K)];
+  }
+  uint64_t skip = __ballot(e < 0 || e >= a.b.E);
+  while (skip) {
+    const int i = __builtin_ctzll(skip);
+    skip &= skip - 1;
+    const float v = __builtin_amdgcn_readlane(e, i) < 0 ? 0.0f : __int_as_float(0x7fc00000);
+    const int p = p0 + i, s = p / a.b.K, k = p - s * a.b.K;
+    float *o = a.out + (size_t)s * a.out_s + (size_t)k * a.out_k;
+    for (int r = lane; r < a.O; r += 64) o[r] = v;
   }
 }
 
