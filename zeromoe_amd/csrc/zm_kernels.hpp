@@ -492,8 +492,8 @@ static __global__ __launch_bounds__(256) void k_router(RouterArgs a, int S) {
 // experts places it 64 pairs at a time (a pair's rank among the wave's lanes
 // with its expert comes from one ballot per id bit), so the order is exactly the
 // sequential one.  A latency chain: five workgroup barriers whatever the pair
-// count (four per 1024 pairs before: 2048 tokens x 8 33.5 -> 11 us with the work
-// list below, 512 x 8 10.2 + 4.7 for the list -> 9.5).
+// count (four per 1024 pairs before).  Timed only as the first workgroup of
+// k_prep, beside the Q8_K rows.
 constexpr int BUCKET_MAX_E = 512;
 constexpr int BUCKET_CH = 16;  // 64-pair chunks per wave whose ids stay in registers
 
