@@ -163,6 +163,46 @@ def test_mul_mat_id_f32_plain_and_grouped(t):
     _ = Z
 
 
+# f32 products on the matrix cores: edges of the 16 x 16 tile and of the 8 waves' shares of the row (1, 8 and 9 blocks).
+# Bound: products rounded in chains of 4, a tree of 2 + 4 levels over a block, ceil(nb / 8) blocks in sequence, 3 levels
+# over the waves, each 2^-24 of sum |w x|; one more for the rounding of the product itself.
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("S,I,Orows", [(2, 256, 15), (16, 2304, 16), (17, 2048, 33), (33, 768, 17)])
+def test_f32_matmul_tiles(t, S, I, Orows):
+    import zeromoe_amd as Z
+
+    W = O.random_blocks(t, Orows, I, seed=t * 5 + S)
+    x = np.random.default_rng(S * I).standard_normal((S, I)).astype(np.float32)
+    tol = (1 + 4 + 6 + -(-I // 2048) + 3) * 2.0**-24
+    dx = torch.from_numpy(x).cuda()
+    # blocks on 4-byte, 2-byte and odd addresses (the last ones stay on the vector units)
+    for off in (0, 2, 1):
+        buf = torch.zeros(W.size + 16, dtype=torch.uint8, device="cuda")
+        dW = buf[off:off + W.size].view(Orows, -1)
+        dW.copy_(torch.from_numpy(W.reshape(Orows, -1)))
+        y = Z.f32_matmul(dW, t, I, dx)
+        _check_mm(y.cpu().numpy(), W, t, x, tol if off != 1 else MM_TOL)
+
+
+@pytest.mark.parametrize("t", [Q3, Q4, Q5, Q6])
+def test_mul_mat_id_f32_tiles(t):
+    import zeromoe_amd as Z
+
+    E, I, Orows, S = 3, 2304, 19, 2
+    W = O.random_blocks(t, E * Orows, I, seed=t).reshape(E, Orows, -1)
+    x = np.random.default_rng(t).standard_normal((S, 1, I)).astype(np.float32)
+    ids = np.array([[2, -1, 0], [3, 1, 2]], np.int32)  # -1: zero row, 3 >= E: NaN row
+    y = Z.mul_mat_id_f32(torch.from_numpy(W).cuda(), t, I, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda())
+    y = y.cpu().numpy()
+    for s in range(S):
+        for k in range(3):
+            e = ids[s, k]
+            if 0 <= e < E:
+                _check_mm(y[s, k][None], W[e], t, x[s], (1 + 4 + 6 + 2 + 3) * 2.0**-24)
+            else:
+                assert np.all(y[s, k] == 0.0) if e < 0 else np.all(np.isnan(y[s, k]))
+
+
 # ------------------------------------------------------------------ SwiGLU
 
 @pytest.mark.parametrize("clamp,fused", [(0.0, False), (6.0, False), (6.0, True), (0.0, True)])

@@ -21,10 +21,34 @@ bool f32_type(int t) {
          t == T_IQ4_XS;
 }
 
+// Whether k_f32_mfma takes the product: 32-bit buffer offsets, blocks on the
+// alignment its loads need, and for a single token per matrix the types where it
+// is the faster one (us, k_f32_mm -> k_f32_mfma):
+//   plain, I 4096 O 1536: Q3_K 20.3 -> 12.6, Q4_K 19.0 -> 10.1, Q6_K 22.7 -> 12.1,
+//     IQ2_XXS 16.1 -> 12.1, IQ4_XS 14.2 -> 11.3; Q2_K 8.9 -> 10.3, IQ3_XXS 10.3 -> 11.7
+//   ids, 16 tokens x 8, I 4096 O 1536: Q3_K 605 -> 425, Q4_K 495 -> 346, Q5_K
+//     617 -> 348, Q6_K 862 -> 372; Q2_K 182 -> 349, IQ2_XXS 268 -> 381, IQ3_XXS
+//     212 -> 376, IQ4_XS 259 -> 376.  With I 2048 (one block per wave) Q4_K 90 -> 99.
+// From two tokens on it is as fast or faster for every type (2 tokens, I 1536
+// O 4096: Q2_K 6.9 -> 7.0, Q4_K 10.8 -> 6.4; 512 tokens: 412 -> 107, 674 -> 109).
+bool f32_mfma_applies(int type, const F32MMArgs &a) {
+  if (a.ids && type != T_Q3_K && type != T_Q5_K && type != T_Q6_K && !(type == T_Q4_K && a.I > F32M_WAVES * QK))
+    return false;
+  if (!a.ids && a.n_tok == 1 && (type == T_Q2_K || type == T_IQ3_XXS)) return false;
+  if ((size_t)a.O * a.w_row >= (1ull << 31) - 4) return false;
+  return !(((uintptr_t)a.w | a.w_mat | a.w_row) & (block_bytes(type) % 4 ? 1 : 3));
+}
+
 template <int T>
 void launch_mm_t(const F32MMArgs &a, int n_route, hipStream_t st) {
   const unsigned gx = (unsigned)((a.O + 4 * F32_RPW - 1) / (4 * F32_RPW));
-  if (a.ids || a.n_tok == 1) {
+  const bool one = a.ids || a.n_tok == 1;  // one token per matrix
+  if (f32_mfma_applies(T, a)) {
+    hipLaunchKernelGGL((k_f32_mfma<T>),
+                       dim3((unsigned)((a.O + 15) / 16), (unsigned)(one ? a.n_tok : (a.n_tok + 15) / 16),
+                            (unsigned)n_route),
+                       dim3(64 * F32M_WAVES), 0, st, a);
+  } else if (one) {
     hipLaunchKernelGGL((k_f32_mm<T, 1>), dim3(gx, (unsigned)a.n_tok, (unsigned)n_route), dim3(256), 0, st, a);
   } else {
     hipLaunchKernelGGL((k_f32_mm<T, 4>), dim3(gx, (unsigned)((a.n_tok + 3) / 4), (unsigned)n_route), dim3(256), 0,

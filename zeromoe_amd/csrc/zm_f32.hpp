@@ -10,6 +10,7 @@
 #pragma once
 
 #include "zm_device.hpp"
+#include "zm_mmq.hpp"
 
 namespace zm {
 
@@ -228,6 +229,121 @@ __global__ __launch_bounds__(256) void k_f32_mm(F32MMArgs a) {
       if (lane == 0 && row0 + r < a.O && t0 + t < a.n_tok)
         a.y[(size_t)(t0 + t) * a.y_tok + (size_t)route * a.y_route + row0 + r] = v;
     }
+}
+
+// ============================================================ f32 matmul, matrix cores
+//
+// The same product on the matrix cores: a workgroup takes 16 weight rows x 16
+// tokens (with ids: one token of one route), its 8 waves every 8th super-block,
+// and v_mfma_f32_16x16x4f32 multiplies the dequantized weights (the values of
+// deq4) with the f32 activations, tokens as the A operand.  A wave's block of
+// rows comes in by direct buffer-to-LDS loads (as in zm_mmq.hpp).
+// k_f32_mm dequantizes a weight again for every 4 tokens and adds its products on
+// the vector units.  Now 40 tokens, I 4096 O 1536, Q4_K: 50 -> 19 us; 512 tokens:
+// 582 -> 98 (66 TFLOP/s; a dense f32 product reaches 143).  Bound by the vector
+// work of the dequantization beside the matrix work, few tokens by the chain of
+// load, product and the tree over the waves; 33 to 48 tokens at O 1536 by the
+// second workgroup that 32 of the 256 CUs get.  Two token tiles per weight tile
+// need 230-254 registers (two waves per SIMD) and were no faster up to 128 tokens.
+//
+// Four products meet in one matrix instruction; everything above is added as a
+// tree (over the block, then the waves) but for a wave's own blocks, so the
+// rounding error is no larger than k_f32_mm's, which rounds each product as well
+// and adds all blocks in sequence (relative to
+// 64 bits, I 256: 8.1e-8 -> 7.7e-8, I 7168: 1.30e-7 -> 0.98e-7; with 16 products
+// chained in the accumulator it was 9.2e-8 at I 256).
+constexpr int F32M_WAVES = 8;
+
+template <int T>
+__global__ __launch_bounds__(64 * F32M_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void k_f32_mfma(F32MMArgs a) {
+  constexpr int BB = block_bytes(T);
+  constexpr int RU = mmq_units<T, 1>(), LU = mmq_load_units<T, 1>();
+  constexpr int NWI = (16 * RU + 63) / 64;
+  constexpr int NTAB = T == T_IQ2_XXS ? 256 : (T == T_IQ3_XXS ? 128 : (T == T_IQ4_XS ? 2 : 1));
+  __shared__ uint64_t s_grid[NTAB];
+  __shared__ __attribute__((aligned(16))) uint8_t s_w[F32M_WAVES][16 * RU * 16];
+  __shared__ __attribute__((aligned(16))) v4f_t s_red[F32M_WAVES / 2][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int row0 = blockIdx.x * 16, t0 = (a.ids ? (int)blockIdx.y : (int)blockIdx.y * 16), route = blockIdx.z;
+  const int t_end = a.ids ? t0 + 1 : min(t0 + 16, a.n_tok);
+  const int nb = a.I / QK;
+  int m = a.mat_by_route ? route : 0;
+  if (a.ids) {
+    m = *reinterpret_cast<const int32_t *>(a.ids + (size_t)t0 * a.id_tok + (size_t)route * a.id_route);
+    if (m < 0 || m >= a.E) {
+      if (tid < 16 && row0 + tid < a.O)
+        a.y[(size_t)t0 * a.y_tok + (size_t)route * a.y_route + row0 + tid] = m < 0 ? 0.0f : __int_as_float(0x7fc00000);
+      return;  // uniform over the workgroup: no barrier follows
+    }
+    m = uniform(m);
+  }
+  const uint8_t *W = a.w + (size_t)m * a.w_mat;
+  if constexpr (NTAB > 1) {
+    for (int i = tid; i < NTAB; i += 64 * F32M_WAVES) s_grid[i] = a.grid[i];
+    __syncthreads();
+  }
+  const int sh = (int)((uintptr_t)W & 3);
+  const v4u_t rw = dma_rsrc(W - sh, ((uint32_t)((size_t)a.O * a.w_row) + sh + 3) & ~3u);
+  const float *xr = a.x + (size_t)min(t0 + n, t_end - 1) * a.x_tok + (size_t)(route % a.x_routes) * a.x_route + 4 * g;
+  v4f_t f = {0.f, 0.f, 0.f, 0.f};
+  for (int b = wave; b < nb; b += F32M_WAVES) {
+    const int st0 = sh + b * BB;
+#pragma unroll
+    for (int i = 0; i < NWI; ++i) {
+      const int u = i * 64 + lane;
+      const int r = u / RU, p = u - RU * r;
+      if (64 * (i + 1) > 16 * RU && u >= 16 * RU) continue;
+      const int st = st0 + (row0 + r) * (int)a.w_row;
+      dma_lds16(rw, lds_addr(&s_w[wave][0]) + i * 1024u, p < LU && row0 + r < a.O ? (st & ~3) + 16 * p : OOR, 0);
+    }
+    float4 xv[16];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) xv[j] = *reinterpret_cast<const float4 *>(xr + (size_t)b * QK + 16 * j);
+    wait_vm<0>();
+    const uint8_t *blk = &s_w[wave][n * (RU * 16)] + ((st0 + (row0 + n) * (int)a.w_row) & 3);
+    v4f_t lv[4];  // lv[k]: a finished sum of 2^k sixteens waiting for its neighbour
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      if (j == 4) {
+        asm volatile("" ::: "memory");  // the second half's x: not earlier, for its registers
+#pragma unroll
+        for (int k = 8; k < 16; ++k) xv[k] = *reinterpret_cast<const float4 *>(xr + (size_t)b * QK + 16 * k);
+      }
+      const float4 w = deq4<T>(blk, 4 * j + g, s_grid);  // weights 16j + 4g .. + 3 of row n
+      const v4f_t z = {0.f, 0.f, 0.f, 0.f};
+      const v4f_t c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].x, w.x, z, 0, 0, 0);
+      const v4f_t c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].y, w.y, z, 0, 0, 0);
+      const v4f_t c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].z, w.z, z, 0, 0, 0);
+      const v4f_t c3 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j].w, w.w, z, 0, 0, 0);
+      v4f_t v = (c0 + c1) + (c2 + c3);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (((j >> k) & 1) == 0) {
+          lv[k] = v;
+          break;
+        }
+        v += lv[k];
+      }
+      if (j == 15) f += v;
+    }
+    wait_lds();  // the slot is read before the next block's loads
+  }
+  // tree over the waves; lane (n, g) holds tokens 4g + j, row n
+#pragma unroll
+  for (int h = F32M_WAVES / 2; h > 0; h >>= 1) {
+    if (wave >= h && wave < 2 * h) s_red[wave - h][lane] = f;
+    __syncthreads();
+    if (wave < h) f += s_red[wave][lane];
+    __syncthreads();
+  }
+  if (wave == 0 && row0 + n < a.O) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = t0 + 4 * g + j;
+      if (t < t_end) a.y[(size_t)t * a.y_tok + (size_t)route * a.y_route + row0 + n] = f[j];
+    }
+  }
 }
 
 // ============================================================ SwiGLU
