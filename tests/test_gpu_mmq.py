@@ -65,7 +65,7 @@ def _check(t, I, rows, sizes, offset=0, extra=()):
 @pytest.mark.parametrize("I,rows", [(256, 16), (512, 37), (768, 130), (1280, 64), (1792, 1)])
 def test_bucket_and_row_edges(t, I, rows):
     _check(t, I, rows, [1, 15, 16, 17, 31, 32, 33, 0, 2])                      # 32-pair items
-    _check(t, I, rows, [1, 0, 2, 15, 16, 3, 17, 7, 5, 9], extra=(-1, 10))      # 16-pair items
+    _check(t, I, rows, [1, 0, 2, 15, 16, 3, 17, 7, 5, 9, 6], extra=(-1, 11))      # 16-pair items
     _check(t, I, rows, [1, 16, 33, 47, 48, 49, 63, 64, 65, 129], extra=(-1, 10, 99))  # 64-pair items
 
 
@@ -74,12 +74,13 @@ def test_bucket_and_row_edges(t, I, rows):
 def test_weights_off_a_dword(t, offset):
     """Odd row counts of 110-, 210-, 66- and 98-byte blocks put experts and rows
     on either half of a dword; other alignments take the GEMV."""
-    _check(t, 768, 33, [20, 5, 40, 1], offset=offset)
+    _check(t, 768, 33, [20, 5, 55, 1], offset=offset)
 
 
-@pytest.mark.parametrize("pairs", [39, 40, 41])
-def test_smallest_pair_count(pairs):
-    _check(Q3, 512, 48, [pairs - 3, 2, 1])
+@pytest.mark.parametrize("t,I,rows,least", [(Q3, 512, 48, 64), (IQ3, 512, 48, 80), (Q3, 2560, 1000, 40)])
+def test_smallest_pair_count(t, I, rows, least):
+    for pairs in (least - 1, least, least + 1):
+        _check(t, I, rows, [pairs - 3, 2, 1])
 
 
 @pytest.mark.parametrize("tg,off_g,off_u", [(Q3, 0, 2), (Q3, 2, 2), (Q4, 0, 4), (Q4, 2, 0), (IQ2, 2, 0)])

@@ -280,15 +280,24 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 //   - rows, activations: 32-bit buffer offsets;
 //   - alignment: blocks of a multiple of 4 bytes are loaded by dwords, the
 //     others start on 2 bytes (gate and up alike within a dword);
-//   - pairs: below MMQ_MIN_PAIRS its workgroups are too few and too long.  One
+//   - pairs: below mmq_min_pairs its workgroups are too few and too long.  One
 //     op over 128 experts, GEMV / this, us, by pairs (1536 rows of 4096, Q4_K):
 //     8 13.1 / 21.5, 32 28.7 / 30.2, 48 40.5 / 40.5, 64 52.0 / 48.1, 128 97.1 /
 //     72.1; (4096 rows of 1536, Q6_K): 8 18.3 / 19.9, 32 45.3 / 44.0, 48 64.9 /
-//     57.5, 128 165.2 / 100.8.
-constexpr int MMQ_MIN_PAIRS = 40;
+//     57.5, 128 165.2 / 100.8.  Matrices of few blocks need more pairs, those of
+//     the grid types most (kernels alone; gate/up then down, 1792 rows of 1024 and
+//     1024 of 1792, 40 pairs: IQ3_XXS 21.0 / 27.2, 12.1 / 15.1, Q4_K 20.7 / 19.8,
+//     Q6_K 15.5 / 16.3; 1280 of 2560 and 2560 of 1280: IQ3_XXS 46.1 / 39.4,
+//     26.2 / 22.2.  Whole layer, 1024 x 1792, 64 pairs: Q4_K 69.7 / 64.5, IQ3_XXS
+//     63.2 / 66.8, IQ2_XXS 57.0 / 62.8; 80: 87.5 / 73.3, 78.8 / 72.6, 64.1 / 63.6).
+constexpr int MMQ_MAX_MIN_PAIRS = 80;
+int mmq_min_pairs(int type, int nrows, int nb) {
+  if ((size_t)nrows * nb >= 10000) return 40;
+  return type == T_IQ2_XXS || type == T_IQ3_XXS ? MMQ_MAX_MIN_PAIRS : 64;
+}
 bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride, int n_pairs,
                  size_t xq_rows, int nb) {
-  if (n_pairs < MMQ_MIN_PAIRS || getenv_flag_off("ZEROMOE_MMQ")) return false;
+  if (n_pairs < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
   if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
   if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 16 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
@@ -1063,8 +1072,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     const int ts = L->type_shared, Fs = L->F_shared, nbS = Fs / QK;
     const size_t gr = row_bytes(ts, H), dr = row_bytes(ts, Fs);
     // one bucket of S pairs; from 8 tokens on (as the pairs of a bucket, not of a batch)
-    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MIN_PAIRS, (size_t)S, nbH);
-    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MIN_PAIRS, (size_t)S, nbS);
+    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
+    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
     // x in the layout of this type: the routed experts' rows where they are the same
     const bool same = mg == mmq_g && (!mg || mmq_order(ts) == mmq_order(L->type_gate));
     if (!same && quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;

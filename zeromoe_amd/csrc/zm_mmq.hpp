@@ -528,6 +528,14 @@ template <int T, bool GATEUP, int TT, int NW, int C>
 static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 ? 4 : 2))) void k_mmq(GemvArgs a) {
   constexpr int TOK = 16 * TT;
   constexpr int NM = GATEUP ? 2 : 1;
+  // Blocks are added in runs of 8, and the runs in turn: shorter chains, and no
+  // larger rounding error than the GEMV's where that would run (relative to 64
+  // bits, rows of 7168, one chain / runs of 8 / GEMV: Q4_K 1.13 / 0.89 / 1.07e-7,
+  // Q6_K 1.10 / 0.86 / 0.93e-7).  Four tiles keep one chain, as their second sums
+  // would cost the fourth wave per SIMD; not for Q3_K (gate/up, 8 waves with 21
+  // spilled registers; with 4 waves and none a layer of 512 tokens takes 494 us
+  // instead of 413).
+  constexpr bool kTwoLevel = TT <= 2 || T == T_Q3_K;
   constexpr int BB = block_bytes(T);
   constexpr int UN = TOK * XUNITS;          // activation units of a block
   constexpr int NI = (UN + 64 * NW - 1) / (64 * NW);
@@ -668,6 +676,7 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < 4; ++j) f[m][t][j] = 0.f;
+    float fs[kTwoLevel ? NM : 1][kTwoLevel ? NT : 1][4] = {};  // sums of 8 blocks
     // request order: x(0) W0(0) W1(0), then per stage W0(s + 1), x(s + 1), W1(s + 1)
     const int ns = (nb + C - 1) / C;
     dma_x(0, 0);
@@ -760,6 +769,19 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
               }
             }
           }
+        }
+      }
+      if constexpr (kTwoLevel) {
+        if ((s + 1) % (8 / C) == 0 || s + 1 == ns) {
+#pragma unroll
+          for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                fs[m][t][j] += f[m][t][j];
+                f[m][t][j] = s + 1 == ns ? fs[m][t][j] : 0.f;
+              }
         }
       }
     }
