@@ -290,14 +290,16 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 //     Q6_K 15.5 / 16.3; 1280 of 2560 and 2560 of 1280: IQ3_XXS 46.1 / 39.4,
 //     26.2 / 22.2.  Whole layer, 1024 x 1792, 64 pairs: Q4_K 69.7 / 64.5, IQ3_XXS
 //     63.2 / 66.8, IQ2_XXS 57.0 / 62.8; 80: 87.5 / 73.3, 78.8 / 72.6, 64.1 / 63.6).
+//     The count is of pairs that are likely to be computed: a slot table skips
+//     those of experts that are not resident.
 constexpr int MMQ_MAX_MIN_PAIRS = 80;
 int mmq_min_pairs(int type, int nrows, int nb) {
   if ((size_t)nrows * nb >= 10000) return 40;
   return type == T_IQ2_XXS || type == T_IQ3_XXS ? MMQ_MAX_MIN_PAIRS : 64;
 }
 bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride, int n_pairs,
-                 size_t xq_rows, int nb) {
-  if (n_pairs < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
+                 int likely, size_t xq_rows, int nb) {
+  if (likely < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
   if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
   if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 16 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
@@ -510,7 +512,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
   const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
-  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
+  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (int)n_pairs, (size_t)nq, nb);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
   const int groups = (int)std::min<int64_t>(E, n_pairs);
@@ -1033,50 +1035,30 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     const int rc = launch_fused(L, x, lg, S, out, ids, wts, w, d, st);
     if (rc <= 0) return rc;
   }
-  if (zm_router(&L->router, lg, L->logit_bias, L->sel_bias, L->route_map, L->route_mask, S, ids, wts, st))
-    return -1;
   // activations -> Q8_K rows: records for the grouped MFMA kernel, planar rows for the GEMV
   const size_t g_row = row_bytes(L->type_gate, H), d_row = row_bytes(L->type_down, F);
-  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, S * K, (size_t)S, nbH);
-  const bool mmq_d = mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, S * K, (size_t)S * K, nbF);
+  const int likely = L->route_map ? (int)((int64_t)S * K * std::min(NS, E) / E) : S * K;
+  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, S * K, likely, (size_t)S, nbH);
+  const bool mmq_d =
+      mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, S * K, likely, (size_t)S * K, nbF);
   auto quant = [&](bool rec, int type, const float *v, int n, int rows, uint8_t *y, hipStream_t q) {
     return rec ? launch_quant_rec(v, (size_t)n, n / QK, rows, y, type, q)
                : launch_quant(v, (size_t)n, n / QK, rows, y, q8_row_bytes(n / QK), 1, q);
   };
   auto qrow = [](bool rec, int nb) { return rec ? xrec_row_bytes(nb) : q8_row_bytes(nb); };
-  const int groups = std::min(NS, S * K);
-  const int tt = mmq_tiles((double)(S * K) / groups);
-  {
-    PrepArgs p{};
-    p.b = BucketArgs{ids, (size_t)K, K, S * K, NS, w.counts, w.offs, w.pairs, w.active, w.n_active, w.items,
-                     w.n_items, mmq_g || mmq_d ? 16 * tt : 0};
-    p.x = x;
-    p.x_tok = p.x_row = (size_t)H;
-    p.ne11 = 1;
-    p.nb = nbH;
-    p.rows = S;
-    p.y = w.xq;
-    p.y_rstride = qrow(mmq_g, nbH);
-    p.order = mmq_g ? mmq_order(L->type_gate) : -1;
-    // skipped routes (slot table -1) read as zero rows; router ids are always valid otherwise
-    p.out = L->route_map ? w.y : nullptr;
-    p.out_s = (size_t)K * H;
-    p.out_k = (size_t)H;
-    p.O = H;
-    if (launch_prep(p, st)) return -1;
-  }
-  // shared expert (dense over all tokens) on the side stream: it needs only
-  // the Q8_K rows of x, and its gate/up, act quantization and down overlap
-  // the router-dependent kernels; the combine waits for it
+  // shared expert (dense over all tokens) on the side stream: it needs only x,
+  // which it quantizes for itself, so that it starts beside the routing and the
+  // preparation; the combine waits for it.  Waiting for the preparation's rows of
+  // x instead cost their time wherever the shared expert is the longer branch
+  // (with the skipped rows in k_prep spread wider, 13 tokens, Q6_K shared expert
+  // of 2048: layer 204 -> 168 us; 64 tokens, Q4_K: 361 -> 349).
   auto launch_shared = [&](hipStream_t ss) -> int {
     const int ts = L->type_shared, Fs = L->F_shared, nbS = Fs / QK;
     const size_t gr = row_bytes(ts, H), dr = row_bytes(ts, Fs);
     // one bucket of S pairs; from 8 tokens on (as the pairs of a bucket, not of a batch)
-    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
-    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
-    // x in the layout of this type: the routed experts' rows where they are the same
-    const bool same = mg == mmq_g && (!mg || mmq_order(ts) == mmq_order(L->type_gate));
-    if (!same && quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;
+    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, S, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
+    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, S, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
+    if (quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;
     GemvArgs c{};
     c.w0 = (const uint8_t *)L->ws_gate;
     c.w1 = (const uint8_t *)L->ws_up;
@@ -1084,7 +1066,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     c.w_estride = 0;
     c.nrows = Fs;
     c.nb = nbH;
-    c.xq = same ? w.xq : w.xq_s;
+    c.xq = w.xq_s;
     c.xq_rstride = qrow(mg, nbH);
     c.xq_bytes = (uint32_t)((size_t)S * c.xq_rstride);
     c.ne11 = 1;
@@ -1126,6 +1108,29 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     HIP_OK(hipStreamWaitEvent(d->side, d->ev_fork, 0));
     if (launch_shared(d->side)) return -1;
     HIP_OK(hipEventRecord(d->ev_join, d->side));
+  }
+  if (zm_router(&L->router, lg, L->logit_bias, L->sel_bias, L->route_map, L->route_mask, S, ids, wts, st))
+    return -1;
+  const int groups = std::min(NS, S * K);
+  const int tt = mmq_tiles((double)(S * K) / groups);
+  {
+    PrepArgs p{};
+    p.b = BucketArgs{ids, (size_t)K, K, S * K, NS, w.counts, w.offs, w.pairs, w.active, w.n_active, w.items,
+                     w.n_items, mmq_g || mmq_d ? 16 * tt : 0};
+    p.x = x;
+    p.x_tok = p.x_row = (size_t)H;
+    p.ne11 = 1;
+    p.nb = nbH;
+    p.rows = S;
+    p.y = w.xq;
+    p.y_rstride = qrow(mmq_g, nbH);
+    p.order = mmq_g ? mmq_order(L->type_gate) : -1;
+    // skipped routes (slot table -1) read as zero rows; router ids are always valid otherwise
+    p.out = L->route_map ? w.y : nullptr;
+    p.out_s = (size_t)K * H;
+    p.out_k = (size_t)H;
+    p.O = H;
+    if (launch_prep(p, st)) return -1;
   }
   // gate/up + SwiGLU
   const int np = pick_np(S * K, NS);

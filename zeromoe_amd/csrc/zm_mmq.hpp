@@ -201,7 +201,7 @@ struct PrepArgs {
   int O;
 };
 constexpr int PREP_QBLOCKS = 64;  // 256-value blocks quantized per workgroup
-constexpr int PREP_FPAIRS = 64;   // pairs looked through per workgroup, 4 per wave
+constexpr int PREP_FPAIRS = 16;   // pairs looked through per workgroup, one per wave
 
 static __global__ __launch_bounds__(1024) void k_prep(PrepArgs a) {
   __shared__ BucketLds l;
@@ -225,21 +225,14 @@ static __global__ __launch_bounds__(1024) void k_prep(PrepArgs a) {
     return;
   }
   const int lane = threadIdx.x & 63;
-  const int p0 = (wg - a.q_wgs) * PREP_FPAIRS + 4 * (int)(threadIdx.x >> 6);
-  int e = 0;
-  if (lane < 4 && p0 + lane < a.b.n_pairs) {
-    const int p = p0 + lane, s = p / a.b.K;
-    e = a.b.ids[(size_t)s * a.b.id_s + (p - s * a.b.K)];
-  }
-  uint64_t skip = __ballot(e < 0 || e >= a.b.E);
-  while (skip) {
-    const int i = __builtin_ctzll(skip);
-    skip &= skip - 1;
-    const float v = __builtin_amdgcn_readlane(e, i) < 0 ? 0.0f : __int_as_float(0x7fc00000);
-    const int p = p0 + i, s = p / a.b.K, k = p - s * a.b.K;
-    float *o = a.out + (size_t)s * a.out_s + (size_t)k * a.out_k;
-    for (int r = lane; r < a.O; r += 64) o[r] = v;
-  }
+  const int p = (wg - a.q_wgs) * PREP_FPAIRS + (int)(threadIdx.x >> 6);
+  if (p >= a.b.n_pairs) return;
+  const int s = p / a.b.K, k = p - s * a.b.K;
+  const int e = a.b.ids[(size_t)s * a.b.id_s + k];
+  if (e >= 0 && e < a.b.E) return;
+  const float v = e < 0 ? 0.0f : __int_as_float(0x7fc00000);
+  float *o = a.out + (size_t)s * a.out_s + (size_t)k * a.out_k;
+  for (int r = lane; r < a.O; r += 64) o[r] = v;
 }
 
 // ---------------------------------------------------------------- weight blocks in LDS
