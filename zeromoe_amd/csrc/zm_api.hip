@@ -56,9 +56,8 @@ struct DeviceState {
   size_t trace_n = 0;
   int n_cu = 0;               // compute units
   // a dense shared expert runs beside the routed kernels of a multi-kernel
-  // layer: forked from the caller's stream after x is quantized, joined
-  // before the combine (default priority; the fork/join records into a HIP
-  // graph like any other stream work)
+  // layer (SideBranch; default priority, and the fork and join record into a
+  // HIP graph like any other stream work)
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::mutex *fork_mu = nullptr;  // the events are per device: one fork at a time
@@ -347,6 +346,38 @@ int launch_quant(const float *x, size_t x_rstride, int nb, int rows, uint8_t *y,
   return 0;
 }
 
+// Work on the device's side stream beside the caller's stream `st`.  Whatever
+// way the scope of an open branch is left, `st` waits for what it has launched:
+// the side stream reads and writes the caller's buffers.
+struct SideBranch {
+  DeviceState *d;
+  hipStream_t st;
+  std::unique_lock<std::mutex> lk;
+  bool open = false;
+  SideBranch(DeviceState *dev, hipStream_t s) : d(dev), st(s) {}
+  SideBranch(const SideBranch &) = delete;
+  int fork() {
+    lk = std::unique_lock<std::mutex>(*d->fork_mu);
+    HIP_OK(hipEventRecord(d->ev_fork, st));
+    HIP_OK(hipStreamWaitEvent(d->side, d->ev_fork, 0));
+    open = true;
+    return 0;
+  }
+  int join() {
+    open = false;
+    HIP_OK(hipEventRecord(d->ev_join, d->side));
+    HIP_OK(hipStreamWaitEvent(st, d->ev_join, 0));
+    return 0;
+  }
+  ~SideBranch() {
+    if (!open) return;
+    char why[sizeof(g_err)];  // the failure that ends the call, not one of this join
+    memcpy(why, g_err, sizeof(why));
+    (void)join();
+    memcpy(g_err, why, sizeof(why));
+  }
+};
+
 // simple bump allocator over a caller workspace
 struct Bump {
   uint8_t *base;
@@ -359,6 +390,15 @@ struct Bump {
     return p;
   }
 };
+
+// what k_router takes
+int check_router(const zm_router_spec &spec) {
+  if (spec.n_experts <= 0 || spec.n_experts > ROUTER_MAX_E) return fail("zm_router: n_experts out of range");
+  if (spec.topk <= 0 || spec.topk > spec.n_experts || spec.topk > 64) return fail("zm_router: bad topk");
+  if (spec.n_groups > 64) return fail("zm_router: n_groups > 64");
+  if (spec.gating < 0 || spec.gating > 2) return fail("zm_router: bad gating");
+  return 0;
+}
 
 }  // namespace
 
@@ -415,10 +455,7 @@ int zm_router(const zm_router_spec *spec, const float *logits, const float *logi
               const int32_t *route_map, const float *route_mask, int S, int32_t *ids, float *weights,
               void *stream) {
   if (!spec || !logits || !ids || !weights || S < 0) return fail("zm_router: null argument");
-  if (spec->n_experts <= 0 || spec->n_experts > ROUTER_MAX_E) return fail("zm_router: n_experts out of range");
-  if (spec->topk <= 0 || spec->topk > spec->n_experts || spec->topk > 64) return fail("zm_router: bad topk");
-  if (spec->n_groups > 64) return fail("zm_router: n_groups > 64");
-  if (spec->gating < 0 || spec->gating > 2) return fail("zm_router: bad gating");
+  if (check_router(*spec)) return -1;
   if (S == 0) return 0;
   RouterArgs a{logits, logit_bias, sel_bias, route_map, route_mask, spec->n_experts, spec->topk, spec->gating,
                spec->n_groups, spec->n_groups_used, spec->weights_norm, spec->weights_scale, ids, weights};
@@ -1035,6 +1072,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     const int rc = launch_fused(L, x, lg, S, out, ids, wts, w, d, st);
     if (rc <= 0) return rc;
   }
+  if (check_router(L->router)) return -1;  // before the side stream has work
   // activations -> Q8_K rows: records for the grouped MFMA kernel, planar rows for the GEMV
   const size_t g_row = row_bytes(L->type_gate, H), d_row = row_bytes(L->type_down, F);
   const int likely = L->route_map ? (int)((int64_t)S * K * std::min(NS, E) / E) : S * K;
@@ -1101,14 +1139,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     e2.out_s = H;
     return dense(md, false, e2) ? -1 : 0;
   };
-  std::unique_lock<std::mutex> fork_lk;
-  if (L->F_shared > 0) {
-    fork_lk = std::unique_lock<std::mutex>(*d->fork_mu);
-    HIP_OK(hipEventRecord(d->ev_fork, st));
-    HIP_OK(hipStreamWaitEvent(d->side, d->ev_fork, 0));
-    if (launch_shared(d->side)) return -1;
-    HIP_OK(hipEventRecord(d->ev_join, d->side));
-  }
+  SideBranch side(d, st);
+  if (L->F_shared > 0 && (side.fork() || launch_shared(d->side))) return -1;
   if (zm_router(&L->router, lg, L->logit_bias, L->sel_bias, L->route_map, L->route_mask, S, ids, wts, st))
     return -1;
   const int groups = std::min(NS, S * K);
@@ -1181,7 +1213,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   if (mmq_d ? launch_mmq(L->type_down, false, tt, 4, max_items, b, st)
             : launch_gemv(L->type_down, false, np, b, groups, st))
     return -1;
-  if (L->F_shared > 0) HIP_OK(hipStreamWaitEvent(st, d->ev_join, 0));  // the shared expert's y_s
+  if (L->F_shared > 0 && side.join()) return -1;  // the shared expert's y_s
   const float *ys = L->F_shared > 0 ? w.y_s : nullptr;
   if ((uintptr_t)out & 15)
     hipLaunchKernelGGL(k_combine1, dim3((H + 255) / 256, S), dim3(256), 0, st, w.y, wts, ys, H, K, out);
