@@ -100,3 +100,22 @@ def test_gate_and_up_on_different_halves(tg, off_g, off_u):
     else:
         slack = 1e-3 * np.abs(ref).max(axis=1, keepdims=True)
         assert (np.abs(out - ref) <= 4 * slack).all()
+
+
+@pytest.mark.parametrize("S,n_ids", [(600_001, 1), (1 << 20, 16)])
+def test_bucket_of_more_than_half_a_million_pairs(S, n_ids):
+    """All pairs of a long call in one bucket, up to the most the op takes
+    (2^24): every part of the result is bit for bit that of a call on these
+    tokens alone (a pair's sums do not depend on its place in the bucket)."""
+    import zeromoe_amd as Z
+
+    I, rows = 256, 16
+    W = torch.from_numpy(O.random_blocks(Q4, 2 * rows, I, seed=5).reshape(2, rows, -1)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    x = torch.randn((S, 1, I), device="cuda", generator=gen)
+    ids = torch.ones((S, n_ids), dtype=torch.int32, device="cuda")
+    out = Z.mul_mat_id(W, Q4, I, x, ids)
+    first = (1 << 19) // n_ids  # the token of pair 2^19
+    for a, b in [(0, 512), (first - 256, first + 256), (S // 2, S // 2 + 512), (S - 512, S)]:
+        part = Z.mul_mat_id(W, Q4, I, x[a:b].contiguous(), ids[a:b].contiguous())
+        assert torch.equal(out[a:b], part), (a, b)

@@ -526,7 +526,7 @@ bool mmid_shape(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, co
   if (y->nb[0] != 4 || y->ne[0] != O || y->ne[1] != n_ids || y->ne[2] != S || y->ne[3] != 1) return false;
   if (y->nb[1] % 4 || y->nb[2] % 4 || ids->nb[1] % 4) return false;
   const int64_t n_pairs = n_ids * S;
-  if (n_pairs > (1 << 24)) return false;
+  if (n_pairs > MMQ_MAX_PAIRS) return false;
   m->I = I;
   m->O = O;
   m->E = E;
@@ -1040,6 +1040,7 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   if (check_layer(L)) return -1;
   if (S <= 0 || !x || !out || (!logits && !L->router_w)) return fail("zm_moe_forward: bad arguments");
   if (S > 65535) return fail("S too large");
+  static_assert(65535 * 64 <= MMQ_MAX_PAIRS, "S * topk");
   if (!workspace || workspace_size < layer_ws(L, S, nullptr, nullptr)) return fail("workspace too small");
   DeviceState *d;
   if (device_state(&d)) return -1;

@@ -497,15 +497,29 @@ static __global__ __launch_bounds__(256) void k_router(RouterArgs a, int S) {
 constexpr int BUCKET_MAX_E = 512;
 constexpr int BUCKET_CH = 16;  // 64-pair chunks per wave whose ids stay in registers
 
+// A work item: expert | (its first pair's offset within the bucket / 16) << 12.
+// 20 unsigned bits of 16 pairs reach every offset of a bucket of up to 2^24
+// pairs, the most that any caller admits.
+static_assert(BUCKET_MAX_E <= 1 << 12, "expert field of a work item");
+constexpr int MMQ_MAX_PAIRS = 1 << 24;
+__host__ __device__ constexpr int32_t mmq_item(int e, int first) {
+  return (int32_t)((uint32_t)e | ((uint32_t)(first >> 4) << 12));
+}
+__host__ __device__ constexpr int mmq_item_expert(int32_t it) { return it & 0xfff; }
+__host__ __device__ constexpr int mmq_item_first(int32_t it) { return (int)((uint32_t)it >> 12) * 16; }
+static_assert(mmq_item_first(mmq_item(511, MMQ_MAX_PAIRS - 16)) == MMQ_MAX_PAIRS - 16 &&
+                  mmq_item_expert(mmq_item(511, MMQ_MAX_PAIRS - 16)) == 511,
+              "work item fields");
+
 struct BucketArgs {
   const int32_t *ids;  // of pair p: ids[(p / K) * id_s + p % K]
   size_t id_s;
   int K, n_pairs, E;
   int32_t *counts, *offs, *pairs, *active, *n_active;
-  // work items of the grouped MFMA kernel (tok pairs each; 0: none): expert |
-  // (first pair offset within the bucket) << 12, largest first -- full runs,
-  // then every expert's remaining run in descending order of its 16-pair tiles,
-  // so the short items fill the tail of the launch.  The order of items of one
+  // work items of the grouped MFMA kernel (tok pairs each, a multiple of 16; 0:
+  // none; mmq_item), largest first -- full runs, then every expert's remaining
+  // run in descending order of its 16-pair tiles, so the short items fill the
+  // tail of the launch.  The order of items of one
   // size is not fixed; no result depends on it (every item writes its own pairs).
   int32_t *items, *n_items;
   int tok;
@@ -634,9 +648,9 @@ __device__ __forceinline__ void bucket_wg(const BucketArgs &a, BucketLds &l) {
     if (tid < a.E) {
       if (nfull) {
         const int q0 = atomicAdd(&l.cur[17], nfull);
-        for (int q = 0; q < nfull; ++q) a.items[q0 + q] = tid | ((q * a.tok) << 12);
+        for (int q = 0; q < nfull; ++q) a.items[q0 + q] = mmq_item(tid, q * a.tok);
       }
-      if (key) a.items[atomicAdd(&l.cur[key], 1)] = tid | ((nfull * a.tok) << 12);
+      if (key) a.items[atomicAdd(&l.cur[key], 1)] = mmq_item(tid, nfull * a.tok);
     }
   }
 }

@@ -556,8 +556,8 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
   } else {
     if (item >= *a.n_items) return;
     const int it = a.items[item];
-    e = it & 0xfff;
-    pc = a.offs[e] + (it >> 12);
+    e = mmq_item_expert(it);
+    pc = a.offs[e] + mmq_item_first(it);
     p1 = a.offs[e + 1];
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
