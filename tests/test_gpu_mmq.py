@@ -119,3 +119,28 @@ def test_bucket_of_more_than_half_a_million_pairs(S, n_ids):
     for a, b in [(0, 512), (first - 256, first + 256), (S // 2, S // 2 + 512), (S - 512, S)]:
         part = Z.mul_mat_id(W, Q4, I, x[a:b].contiguous(), ids[a:b].contiguous())
         assert torch.equal(out[a:b], part), (a, b)
+
+
+def test_matrix_of_eight_million_rows():
+    """Row tiles times work items past the 2^32 threads of one grid (nearly all
+    of the 128 experts without pairs, their weights never touched): the product
+    goes out in several launches, bit for bit what slices of the rows give."""
+    import zeromoe_amd as Z
+
+    E, rows, S, I = 128, 7_900_001, 128, 256
+    if torch.cuda.mem_get_info()[0] < 90 << 30:
+        pytest.skip("needs 71 GB of weights and outputs")
+    W = torch.empty((E, rows, 66), dtype=torch.uint8, device="cuda")
+    part = torch.from_numpy(O.random_blocks(IQ2, 99_991, I, seed=9)).cuda()
+    for e in (3, 100):
+        for a in range(0, rows, len(part)):
+            W[e, a:a + len(part)] = part[:rows - a].roll(e, 0)[:rows - a]
+    x = torch.randn((S, 1, I), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    ids = torch.where(torch.arange(S) % 2 == 0, 3, 100).to(torch.int32).view(S, 1).cuda()
+    out = Z.mul_mat_id(W, IQ2, I, x, ids)
+    for a in (0, 1_234_567, 4_194_303, rows - 2000):
+        assert torch.equal(out[:, :, a:a + 2000], Z.mul_mat_id(W[:, a:a + 2000], IQ2, I, x, ids)), a
+    # no part of the whole was left out
+    assert out.isfinite().all() and (out != 0).float().mean() > 0.99
+    del W, out
+    torch.cuda.empty_cache()

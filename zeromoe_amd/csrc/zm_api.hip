@@ -296,11 +296,10 @@ int mmq_min_pairs(int type, int nrows, int nb) {
   if ((size_t)nrows * nb >= 10000) return 40;
   return type == T_IQ2_XXS || type == T_IQ3_XXS ? MMQ_MAX_MIN_PAIRS : 64;
 }
-bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride, int n_pairs,
+bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride,
                  int likely, size_t xq_rows, int nb) {
   if (likely < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
   if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
-  if ((size_t)((nrows + 63) / 64) * (size_t)(n_pairs / 16 + 1 + BUCKET_MAX_E) >= (1ull << 31)) return false;  // grid
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
   if (lo & (block_bytes(type) % 4 ? 1 : 3)) return false;
   return !w1 || !(((uintptr_t)w0 ^ (uintptr_t)w1) & 3);
@@ -549,7 +548,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
   const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
-  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (int)n_pairs, (size_t)nq, nb);
+  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
   const int groups = (int)std::min<int64_t>(E, n_pairs);
@@ -1077,9 +1076,9 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   // activations -> Q8_K rows: records for the grouped MFMA kernel, planar rows for the GEMV
   const size_t g_row = row_bytes(L->type_gate, H), d_row = row_bytes(L->type_down, F);
   const int likely = L->route_map ? (int)((int64_t)S * K * std::min(NS, E) / E) : S * K;
-  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, S * K, likely, (size_t)S, nbH);
+  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, likely, (size_t)S, nbH);
   const bool mmq_d =
-      mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, S * K, likely, (size_t)S * K, nbF);
+      mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, likely, (size_t)S * K, nbF);
   auto quant = [&](bool rec, int type, const float *v, int n, int rows, uint8_t *y, hipStream_t q) {
     return rec ? launch_quant_rec(v, (size_t)n, n / QK, rows, y, type, q)
                : launch_quant(v, (size_t)n, n / QK, rows, y, q8_row_bytes(n / QK), 1, q);
@@ -1095,8 +1094,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     const int ts = L->type_shared, Fs = L->F_shared, nbS = Fs / QK;
     const size_t gr = row_bytes(ts, H), dr = row_bytes(ts, Fs);
     // one bucket of S pairs; from 8 tokens on (as the pairs of a bucket, not of a batch)
-    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, S, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
-    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, S, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
+    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
+    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
     if (quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;
     GemvArgs c{};
     c.w0 = (const uint8_t *)L->ws_gate;

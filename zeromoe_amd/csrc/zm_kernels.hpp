@@ -683,9 +683,10 @@ struct GemvArgs {
   int tile_rows;
   const uint64_t *grid;   // IQ2_XXS / IQ3_XXS grid or IQ4_XS value table (global), staged into LDS
   const uint64_t *signs;
-  // int8-MFMA path: (expert, first pair) work items, row tiles per item
+  // int8-MFMA path: (expert, first pair) work items, row tiles per item, first
+  // item of the launch
   const int32_t *items, *n_items;
-  int row_tiles;
+  int row_tiles, item0;
   uint32_t xq_bytes;  // extent of the xq buffer
 };
 

@@ -58,6 +58,8 @@
 //   v_mfma_i32_16x16x32_i8 per sub-block, scaled per lane.
 #pragma once
 
+#include <algorithm>
+
 #include "zm_kernels.hpp"
 
 namespace zm {
@@ -547,7 +549,8 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
   __shared__ int s_xoff[TOK];   // byte offset of each pair's activation row (OOR: none)
   __shared__ long s_out[TOK];   // float offset of each pair's output row (-1: none)
   int e, pc, p1;
-  const int item = blockIdx.x / a.row_tiles, rt = blockIdx.x - item * a.row_tiles;
+  const int li = blockIdx.x / a.row_tiles, rt = blockIdx.x - li * a.row_tiles;
+  const int item = a.item0 + li;
   if (a.dense_S > 0) {
     e = 0;
     pc = item * TOK;
@@ -828,11 +831,16 @@ void mmq_launch_t(int tt, int nw, unsigned items, const GemvArgs &a0, hipStream_
   GemvArgs a = a0;
   if (tt == 4) nw = NW4;
   a.row_tiles = (a.nrows + 16 * nw - 1) / (16 * nw);
-  const dim3 grid((unsigned)a.row_tiles * items);
-  if (tt == 4) hipLaunchKernelGGL((k_mmq<T, GU, 4, NW4, 1>), grid, dim3(64 * NW4), 0, st, a);
-  else if (nw == 1) hipLaunchKernelGGL((k_mmq<T, GU, 2, 1, 1>), grid, dim3(64), 0, st, a);
-  else if (tt == 1) hipLaunchKernelGGL((k_mmq<T, GU, 1, 4, mmq_stage<T>()>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((k_mmq<T, GU, 2, 4, 1>), grid, dim3(256), 0, st, a);
+  // a grid has fewer than 2^32 threads: matrices of millions of rows take several
+  const unsigned most = (unsigned)(0xffffffffu / (64u * nw) / (unsigned)a.row_tiles);
+  for (unsigned i = 0; i < items; i += most) {
+    a.item0 = (int)i;
+    const dim3 grid((unsigned)a.row_tiles * std::min(most, items - i));
+    if (tt == 4) hipLaunchKernelGGL((k_mmq<T, GU, 4, NW4, 1>), grid, dim3(64 * NW4), 0, st, a);
+    else if (nw == 1) hipLaunchKernelGGL((k_mmq<T, GU, 2, 1, 1>), grid, dim3(64), 0, st, a);
+    else if (tt == 1) hipLaunchKernelGGL((k_mmq<T, GU, 1, 4, mmq_stage<T>()>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_mmq<T, GU, 2, 4, 1>), grid, dim3(256), 0, st, a);
+  }
 }
 template <int T>
 void mmq_launch(bool gateup, int tt, int nw, unsigned items, const GemvArgs &a, hipStream_t st) {
