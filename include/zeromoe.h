@@ -108,10 +108,13 @@ int zm_mul_mat_id_negative_skip_batched(void);
  * (kernels/quant/kquant_matmul.cu:702-761, patches/ggml/0010-...:9-27). */
 int zm_mul_mat_id(const zm_tensor *src0, const zm_tensor *src1, const zm_tensor *ids, zm_tensor *dst, void *stream,
                   int execute);
-/* Workspace bytes zm_mul_mat_id needs for this shape (0: shape declined).
+/* Workspace bytes zm_mul_mat_id asks for with this shape (0: shape declined).
  * The reference hook needs none (its FP32 kernels read src1 directly); this
  * path stages Q8_K activations and expert buckets.  Sizing call for the
- * workspace of zm_mul_mat_id_set_workspace. */
+ * workspace of zm_mul_mat_id_set_workspace.  A workspace a few percent smaller
+ * is accepted too -- it has to hold src1 as Q8_K rows (292 bytes per 256
+ * values) rather than as records of the MFMA kernel (304) -- and then a long
+ * call runs in two halves of the tokens. */
 size_t zm_mul_mat_id_workspace_size(const zm_tensor *src0, const zm_tensor *src1, const zm_tensor *ids,
                                     const zm_tensor *dst);
 /* Bind a caller-owned device buffer (256-byte aligned, `bytes` long) as
@@ -125,8 +128,8 @@ int zm_mul_mat_id_set_workspace(void *stream, void *workspace, size_t bytes);
  * or bind memory (code under HIP-graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  Its scratch is a
  * 16 MiB device array compiled into the library (one per GPU, held until the
- * process ends); shapes that need more (zm_mul_mat_id_workspace_size) are
- * declined with an error.  zm_init must have run on the device (it looks up
+ * process ends); shapes for which a bound workspace of that size would be too
+ * small are declined with an error.  zm_init must have run on the device (it looks up
  * the array's address); the call itself only launches.  Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (two streams, two
  * threads) race and must be serialised by the caller.  Same arguments,

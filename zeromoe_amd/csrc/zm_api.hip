@@ -481,30 +481,49 @@ int zm_bucket(const int32_t *ids, int S, int K, int E, int32_t *counts, int32_t 
 namespace {
 
 // A validated MUL_MAT_ID shape (see zm_mul_mat_id's rules) and the workspace
-// it needs: Q8_K rows of src1, the bucket arrays and the MFMA work list.
+// for it: rows of src1, the bucket arrays and the MFMA work list.
 struct MmidShape {
   int64_t I, O, E, n_ids, S, ne11, n_pairs, nq;
   int nb;
-  size_t ws_bytes;
+  size_t ws_bytes;  // holds the records of every token
+  size_t ws_least;  // what the shape is accepted with
 };
 
 struct MmidWs {
   uint8_t *xq;
-  int32_t *counts, *offs, *pairs, *active, *n_active, *items, *n_items;
+  int32_t *idc, *counts, *offs, *pairs, *active, *n_active, *items, *n_items;
 };
 
-size_t mmid_carve(const MmidShape &m, uint8_t *base, MmidWs *out) {
+// rec: src1 as records and a work list (grouped MFMA kernel), else planar rows
+// (GEMV); idc: room for a copy of the ids
+size_t mmid_carve(const MmidShape &m, bool rec, bool idc, uint8_t *base, MmidWs *out) {
   Bump b{base};
   MmidWs w{};
-  w.xq = b.take<uint8_t>((size_t)m.nq * xrec_row_bytes(m.nb));  // planar rows are smaller
+  w.xq = b.take<uint8_t>((size_t)m.nq * (rec ? xrec_row_bytes(m.nb) : q8_row_bytes(m.nb)));
+  if (idc) w.idc = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.counts = b.take<int32_t>((size_t)m.E * 4);
   w.offs = b.take<int32_t>((size_t)(m.E + 1) * 4);
   w.pairs = b.take<int32_t>((size_t)m.n_pairs * 4);
   w.active = b.take<int32_t>((size_t)m.E * 4);
   w.n_active = b.take<int32_t>(4);
-  w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 16) * 4);
-  w.n_items = b.take<int32_t>(4);
+  if (rec) {
+    w.items = b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 16) * 4);
+    w.n_items = b.take<int32_t>(4);
+  }
   if (out) *out = w;
+  return b.off + 256;
+}
+
+// The size from which a workspace is accepted, whatever the kernels in use
+// would like: callers with a workspace of a fixed size (and of the static
+// scratch array) keep the shapes they have.  Q8_K rows, a copy of the ids and a
+// list of 32-pair items; every layout but that of records fits it, and of
+// records at least half the tokens.
+size_t mmid_least(const MmidShape &m) {
+  MmidWs w;
+  Bump b{nullptr, mmid_carve(m, false, true, nullptr, &w) - 256};
+  b.take<int32_t>((size_t)mmq_max_items((int)m.n_pairs, (int)m.E, 32) * 4);
+  b.take<int32_t>(4);
   return b.off + 256;
 }
 
@@ -535,20 +554,41 @@ bool mmid_shape(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, co
   m->n_pairs = n_pairs;
   m->nq = m->ne11 * S;
   m->nb = (int)(I / QK);
-  m->ws_bytes = mmid_carve(*m, nullptr, nullptr);
+  m->ws_least = mmid_least(*m);
+  m->ws_bytes = std::max(mmid_carve(*m, true, false, nullptr, nullptr), m->ws_least);
   return true;
 }
 
-// The op on a workspace of at least m.ws_bytes (256-byte aligned); launches
-// only, stream-ordered, allocates nothing.  Returns 1 handled / 0 failed.
+// The op on a workspace of `cap` >= m.ws_least bytes (256-byte aligned);
+// launches only, stream-ordered, allocates nothing.  Returns 1 handled / 0 failed.
 int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, zm_tensor *y,
-              hipStream_t st, uint8_t *ws, const DeviceState *d) {
-  MmidWs b;
-  mmid_carve(m, ws, &b);
+              hipStream_t st, uint8_t *ws, size_t cap, const DeviceState *d) {
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
   const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
-  const bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
+  bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
+  if (mmq && mmid_carve(m, true, false, nullptr, nullptr) > cap) {
+    // records for half the tokens at a time
+    if (m.S == 1) {
+      mmq = false;
+    } else {
+      const int64_t cut[3] = {0, m.S / 2, m.S};
+      for (int i = 0; i < 2; ++i) {
+        zm_tensor xh = *x, ih = *ids, yh = *y;
+        MmidShape h = m;
+        h.S = xh.ne[2] = ih.ne[1] = yh.ne[2] = cut[i + 1] - cut[i];
+        h.n_pairs = h.S * n_ids;
+        h.nq = h.S * ne11;
+        xh.data = (char *)x->data + (size_t)cut[i] * x->nb[2];
+        ih.data = (char *)ids->data + (size_t)cut[i] * ids->nb[1];
+        yh.data = (char *)y->data + (size_t)cut[i] * y->nb[2];
+        if (!mmid_exec(h, w, &xh, &ih, &yh, st, ws, cap, d)) return 0;
+      }
+      return 1;
+    }
+  }
+  MmidWs b;
+  mmid_carve(m, mmq, false, ws, &b);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
   const int groups = (int)std::min<int64_t>(E, n_pairs);
@@ -598,7 +638,6 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   } else if (launch_gemv(w->type, false, pick_np((int)n_pairs, (int)E), a, groups, st)) {
     return 0;
   }
-  count_mmid_launch();
   return hipPeekAtLastError() == hipSuccess ? 1 : 0;
 }
 
@@ -652,12 +691,12 @@ int zm_mul_mat_id(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, 
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   uint8_t *ws = nullptr;
+  size_t cap = 0;
   {
     // query: the smallest workspace bound on this device must hold the shape
     // (ggml asks with no stream, then executes on one of its streams);
     // execute: the workspace bound to this stream
     std::lock_guard<std::mutex> lk(g_bind_mu);
-    size_t cap = 0;
     bool any = false;
     for (int i = 0; i < g_nbind; ++i) {
       if (g_bind[i].dev != dev) continue;
@@ -670,7 +709,7 @@ int zm_mul_mat_id(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, 
         any = true;
       }
     }
-    if (!any || cap < m.ws_bytes) {
+    if (!any || cap < m.ws_least) {
       fail("zm_mul_mat_id: %s (needs %zu bytes, zm_mul_mat_id_workspace_size)",
            any ? "bound workspace too small" : "no workspace bound for this device/stream", m.ws_bytes);
       return 0;
@@ -678,16 +717,17 @@ int zm_mul_mat_id(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, 
   }
   if (!execute) return 1;
   DeviceState *d;
-  if (device_state(&d)) return 0;
-  return mmid_exec(m, w, x, ids, y, (hipStream_t)stream, ws, d);
+  if (device_state(&d) || !mmid_exec(m, w, x, ids, y, (hipStream_t)stream, ws, cap, d)) return 0;
+  count_mmid_launch();
+  return 1;
 }
 
 int zm_mul_mat_id_static(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, zm_tensor *dst, void *stream,
                          int execute) {
   MmidShape m;
   if (!mmid_shape(w, x, ids, dst, &m)) return 0;
-  if (m.ws_bytes > kStaticScratchBytes) {
-    fail("zm_mul_mat_id_static: shape needs %zu bytes of scratch, more than the %zu-byte device array", m.ws_bytes,
+  if (m.ws_least > kStaticScratchBytes) {
+    fail("zm_mul_mat_id_static: shape needs %zu bytes of scratch, more than the %zu-byte device array", m.ws_least,
          kStaticScratchBytes);
     return 0;
   }
@@ -699,7 +739,9 @@ int zm_mul_mat_id_static(const zm_tensor *w, const zm_tensor *x, const zm_tensor
   }
   // every scratch array is written before it is read within the call, so
   // nothing needs clearing between calls
-  return mmid_exec(m, w, x, ids, dst, (hipStream_t)stream, d->scratch, d);
+  if (!mmid_exec(m, w, x, ids, dst, (hipStream_t)stream, d->scratch, kStaticScratchBytes, d)) return 0;
+  count_mmid_launch();
+  return 1;
 }
 
 // ---------------------------------------------------------------- debug: block dots
