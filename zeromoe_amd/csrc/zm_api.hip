@@ -836,13 +836,11 @@ struct LayerWs {
   float *weights;
   uint8_t *xq;
   int32_t *counts, *offs, *pairs, *active, *n_active;
-  float *act;
   uint8_t *aq;
   float *y;
-  float *act_s;
   uint8_t *xq_s, *aq_s;
   float *y_s;
-  float *f_act;
+  float *act, *act_s, *f_act;
   uint32_t *f_sync;
   int32_t *items, *n_items;  // MFMA work items
 };
@@ -863,19 +861,19 @@ size_t layer_ws(const zm_moe_layer *L, int S, uint8_t *base, LayerWs *w) {
   t.n_active = b.take<int32_t>(4);
   t.items = b.take<int32_t>((size_t)mmq_max_items(S * K, NS, 16) * 4);
   t.n_items = b.take<int32_t>(4);
-  t.act = b.take<float>((size_t)S * K * F * 4);
   t.aq = b.take<uint8_t>((size_t)S * K * xrec_row_bytes(nbF));
   t.y = b.take<float>((size_t)S * K * H * 4);
-  if (L->F_shared > 0) {
-    t.act_s = b.take<float>((size_t)S * L->F_shared * 4);
-    t.xq_s = b.take<uint8_t>((size_t)S * xrec_row_bytes(nbH));
-    t.aq_s = b.take<uint8_t>((size_t)S * xrec_row_bytes(L->F_shared / QK));
-    t.y_s = b.take<float>((size_t)S * H * 4);
-  }
-  // fused decode: act rows of every pair then the shared rows, their Q8_K
-  // rows, and the sync words (zero at allocation, left at zero by every launch)
   const size_t fs = L->F_shared > 0 ? (size_t)L->F_shared : 0;
-  t.f_act = b.take<float>(((size_t)S * K * F + S * fs) * 4);
+  if (fs) {
+    t.aq_s = b.take<uint8_t>((size_t)S * xrec_row_bytes((int)(fs / QK)));
+    t.y_s = b.take<float>((size_t)S * H * 4);
+    t.xq_s = reinterpret_cast<uint8_t *>(t.y_s);  // read for the last time before the down product writes y_s
+  }
+  // act rows of every pair, then the shared rows (one call has them from the
+  // multi-kernel path or from the fused decode kernel), and the fused kernel's
+  // sync words (zero at allocation, left at zero by every launch)
+  t.act = t.f_act = b.take<float>(((size_t)S * K * F + S * fs) * 4);
+  if (fs) t.act_s = base ? t.act + (size_t)S * K * F : nullptr;
   t.f_sync = b.take<uint32_t>((size_t)DEC_SYNC_WORDS * 4);
   if (w) *w = t;
   return b.off + 256;
