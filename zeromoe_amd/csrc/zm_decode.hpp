@@ -46,6 +46,13 @@ namespace zm {
 
 constexpr int DEC_THREADS = 512;
 constexpr int DEC_WAVES = DEC_THREADS / 64;
+// The 130-150 KB of a decode kernel are more than the instruction cache (64 KB)
+// holds, and its time depends on where they start: the Q2_K / Q3_K kernel (4
+// layers, H 4096 F 1536) takes 86.9 us with most offsets in a page, 88.1 with some
+// (+0xe00, which 11 KB more of another kernel in front had made of +0xf00).
+// From a multiple of 64 KB it takes 86.7, whatever else the code object holds
+// (16 KB: 86.7, but 71.4 against 70.7 us for 2 layers with a shared expert).
+constexpr int DEC_CODE_ALIGN = 65536;
 constexpr int DEC_MAX_S = 8;
 constexpr int DEC_MAX_PAIRS = 128;  // S * K
 constexpr int DEC_LDS_Q8 = 65536;   // Q8_K staging: x rows in P0/P1, act rows in P2
@@ -143,7 +150,7 @@ struct RowsTag {
 };
 
 template <int TG, int TD, int TS, int L1, int IR, int IS>
-__global__ __launch_bounds__(DEC_THREADS) void k_moe_decode(DecodeArgs a) {
+__global__ __launch_bounds__(DEC_THREADS) __attribute__((aligned(DEC_CODE_ALIGN))) void k_moe_decode(DecodeArgs a) {
   __shared__ int s_ids[DEC_MAX_PAIRS];
   __shared__ float s_w[DEC_MAX_PAIRS];
   __shared__ int s_cidx[DEC_MAX_PAIRS];  // pair -> compact routed index (or -1)
