@@ -144,3 +144,29 @@ def test_matrix_of_eight_million_rows():
     assert out.isfinite().all() and (out != 0).float().mean() > 0.99
     del W, out
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("over", ["src1", "ids"])
+@pytest.mark.parametrize("S,n_ids", [(5, 4), (150, 4)])
+def test_result_lying_over_an_input(over, S, n_ids):
+    """dst over src1 (a few rows further on) or over the ids, with skipped
+    routes: src1 and the ids are taken in before any row is written."""
+    import zeromoe_amd as Z
+
+    I = rows = 512
+    W = torch.from_numpy(O.random_blocks(Q4, 6 * rows, I, seed=2).reshape(6, rows, -1)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    x = torch.randn((S, n_ids, I), device="cuda", generator=gen)
+    ids = torch.randint(-1, 7, (S, n_ids), dtype=torch.int32, device="cuda", generator=gen)
+    ref = Z.mul_mat_id(W, Q4, I, x, ids)
+    buf = torch.empty(2 * x.numel(), device="cuda")
+    for shift in (0, 3 * I, 16 * I):  # dst so many floats after the input, or over the start of the ids
+        for _ in range(3):
+            xs, ids_ = x, ids
+            if over == "src1":
+                xs = buf[:x.numel()].view(x.shape).copy_(x)
+            else:
+                ids_ = buf[shift:shift + ids.numel()].view(torch.int32).view(ids.shape).copy_(ids)
+            out = buf[shift if over == "src1" else 0:][:x.numel()].view(ref.shape)
+            Z.mul_mat_id(W, Q4, I, xs, ids_, out=out)
+            assert torch.equal(out.nan_to_num(7.0), ref.nan_to_num(7.0)), shift

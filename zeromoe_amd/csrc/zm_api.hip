@@ -317,11 +317,12 @@ int launch_mmq(int type, bool gateup, int tt, int nw, int items, const GemvArgs 
   return 0;
 }
 // sort the pairs (b), quantize the rows of x, write the rows of skipped routes (a.out): one launch
-int launch_prep(PrepArgs a, hipStream_t st) {
+int launch_prep(PrepArgs a, hipStream_t st, bool sort = true) {
+  a.sort_wgs = sort ? 1 : 0;
   const long blocks = (long)a.rows * a.nb;
   a.q_wgs = (int)((blocks + PREP_QBLOCKS - 1) / PREP_QBLOCKS);
   const int f_wgs = a.out ? (a.b.n_pairs + PREP_FPAIRS - 1) / PREP_FPAIRS : 0;
-  hipLaunchKernelGGL(k_prep, dim3(1 + a.q_wgs + f_wgs), dim3(1024), 0, st, a);
+  hipLaunchKernelGGL(k_prep, dim3(a.sort_wgs + a.q_wgs + f_wgs), dim3(1024), 0, st, a);
   HIP_OK(hipGetLastError());
   return 0;
 }
@@ -559,6 +560,16 @@ bool mmid_shape(const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, co
   return true;
 }
 
+// Whether the extents of two F32 / I32 tensors share a byte.
+bool tensors_overlap(const zm_tensor *a, const zm_tensor *b) {
+  auto end = [](const zm_tensor *t) {
+    size_t n = 4;
+    for (int i = 0; i < 4; ++i) n += (size_t)(t->ne[i] - 1) * t->nb[i];
+    return (uintptr_t)t->data + n;
+  };
+  return (uintptr_t)a->data < end(b) && (uintptr_t)b->data < end(a);
+}
+
 // The op on a workspace of `cap` >= m.ws_least bytes (256-byte aligned);
 // launches only, stream-ordered, allocates nothing.  Returns 1 handled / 0 failed.
 int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const zm_tensor *ids, zm_tensor *y,
@@ -567,9 +578,11 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   const int ne11 = (int)m.ne11;
   const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
   bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
-  if (mmq && mmid_carve(m, true, false, nullptr, nullptr) > cap) {
+  // dst may lie over src1 or ids: then both are taken in before a row is written
+  const bool apart = !tensors_overlap(y, x) && !tensors_overlap(y, ids);
+  if (mmq && mmid_carve(m, true, !apart, nullptr, nullptr) > cap) {
     // records for half the tokens at a time
-    if (m.S == 1) {
+    if (m.S == 1 || !apart) {
       mmq = false;
     } else {
       const int64_t cut[3] = {0, m.S / 2, m.S};
@@ -588,7 +601,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
     }
   }
   MmidWs b;
-  mmid_carve(m, mmq, false, ws, &b);
+  mmid_carve(m, mmq, !apart, ws, &b);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
   const int groups = (int)std::min<int64_t>(E, n_pairs);
@@ -605,11 +618,21 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   p.y = b.xq;
   p.y_rstride = xrow;
   p.order = mmq ? mmq_order(w->type) : -1;
-  p.out = (float *)y->data;
+  p.out = apart ? (float *)y->data : nullptr;
   p.out_s = y->nb[2] / 4;
   p.out_k = y->nb[1] / 4;
   p.O = (int)O;
   if (launch_prep(p, st)) return 0;
+  if (!apart) {
+    if (hipMemcpy2DAsync(b.idc, (size_t)n_ids * 4, ids->data, ids->nb[1], (size_t)n_ids * 4, (size_t)m.S,
+                         hipMemcpyDeviceToDevice, st) != hipSuccess)
+      return 0;
+    p.b.ids = b.idc;
+    p.b.id_s = (size_t)n_ids;
+    p.rows = 0;
+    p.out = (float *)y->data;
+    if (launch_prep(p, st, false)) return 0;
+  }
   // 2. bucketed GEMV or MFMA
   GemvArgs a{};
   a.w0 = (const uint8_t *)w->data;

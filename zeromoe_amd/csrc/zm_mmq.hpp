@@ -196,7 +196,7 @@ struct PrepArgs {
   uint8_t *y;
   size_t y_rstride;
   int order;  // record order, or -1: planar rows
-  int q_wgs;
+  int sort_wgs, q_wgs;  // 1: workgroup 0 sorts, 0: only rows are written
   // output rows of skipped routes (out null: none)
   float *out;
   size_t out_s, out_k;
@@ -207,11 +207,11 @@ constexpr int PREP_FPAIRS = 16;   // pairs looked through per workgroup, one per
 
 static __global__ __launch_bounds__(1024) void k_prep(PrepArgs a) {
   __shared__ BucketLds l;
-  if (blockIdx.x == 0) {
+  const int wg = (int)blockIdx.x - a.sort_wgs;
+  if (wg < 0) {
     bucket_wg(a.b, l);
     return;
   }
-  const int wg = (int)blockIdx.x - 1;
   if (wg < a.q_wgs) {
     const int l16 = threadIdx.x & 15;
     const long gb = (long)wg * PREP_QBLOCKS + (threadIdx.x >> 4);
