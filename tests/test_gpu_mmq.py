@@ -170,3 +170,24 @@ def test_result_lying_over_an_input(over, S, n_ids):
             out = buf[shift if over == "src1" else 0:][:x.numel()].view(ref.shape)
             Z.mul_mat_id(W, Q4, I, xs, ids_, out=out)
             assert torch.equal(out.nan_to_num(7.0), ref.nan_to_num(7.0)), shift
+
+
+def test_records_past_two_gibibytes(monkeypatch):
+    """Records of src1 beyond 2^31 bytes (Q8_K rows of these tokens are not):
+    bit for bit the same kernel's results for a few of the tokens, which are
+    not bit for bit the GEMV's."""
+    import zeromoe_amd as Z
+
+    S, I, rows = 114_000, 16384, 32
+    assert S * (I // 256) * 292 < 1 << 31 < S * (I // 256) * 304
+    W = torch.from_numpy(O.random_blocks(Q6, 2 * rows, I, seed=4).reshape(2, rows, -1)).cuda()
+    x = torch.randn((S, 1, I), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2))
+    ids = (torch.arange(S, device="cuda") % 2).to(torch.int32).view(S, 1)
+    out = Z.mul_mat_id(W, Q6, I, x, ids)
+    for a in (0, S // 2, 110_376, S - 256):
+        part = Z.mul_mat_id(W, Q6, I, x[a:a + 256], ids[a:a + 256])
+        assert torch.equal(out[a:a + 256], part), a
+    monkeypatch.setenv("ZEROMOE_MMQ", "0")
+    assert not torch.equal(out[-256:], Z.mul_mat_id(W, Q6, I, x[-256:], ids[-256:]))
+    del x, out
+    torch.cuda.empty_cache()

@@ -276,7 +276,7 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 }
 // Whether the grouped MFMA kernel takes this product (the caller then
 // quantizes the activations to records); the GEMV takes what is left.
-//   - rows, activations: 32-bit buffer offsets;
+//   - rows, activations: 32-bit buffer offsets (of rows signed, of records not);
 //   - alignment: blocks of a multiple of 4 bytes are loaded by dwords, the
 //     others start on 2 bytes (gate and up alike within a dword);
 //   - pairs: below mmq_min_pairs its workgroups are too few and too long.  One
@@ -299,7 +299,7 @@ int mmq_min_pairs(int type, int nrows, int nb) {
 bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride,
                  int likely, size_t xq_rows, int nb) {
   if (likely < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
-  if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) >= (1ull << 31)) return false;
+  if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) > XREC_MAX_BYTES) return false;
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
   if (lo & (block_bytes(type) % 4 ? 1 : 3)) return false;
   return !w1 || !(((uintptr_t)w0 ^ (uintptr_t)w1) & 3);

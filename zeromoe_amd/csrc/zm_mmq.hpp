@@ -146,6 +146,9 @@ __device__ __forceinline__ v2h_t bytes_f16(uint32_t w, uint32_t sel) {
 
 constexpr int XREC = 304;           // bytes of one block's record
 constexpr int XUNITS = XREC / 16;   // 19
+// records are reached by unsigned 32-bit offsets; one past every buffer's extent
+constexpr uint32_t XOOR = 0xfffffff0u;
+constexpr size_t XREC_MAX_BYTES = 0xfffff000u;
 __host__ __device__ constexpr size_t xrec_row_bytes(int nb) { return (size_t)nb * XREC; }
 // value order of a record's int8: 0 natural, 1 the 8-byte groups of the two 32-value halves of a chunk alternating
 __host__ __device__ constexpr int mmq_order(int type) { return type == T_Q2_K || type == T_Q3_K ? 0 : 1; }
@@ -546,7 +549,7 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
   __shared__ __attribute__((aligned(kGrid ? 2048 : 8))) uint64_t s_signs[kGrid ? 128 : 1];
   __shared__ __attribute__((aligned(16))) uint8_t s_x[2][C][TOK * XREC];
   __shared__ __attribute__((aligned(16))) uint8_t s_w[NW][NM][WB];
-  __shared__ int s_xoff[TOK];   // byte offset of each pair's activation row (OOR: none)
+  __shared__ uint32_t s_xoff[TOK];  // byte offset of each pair's activation row (XOOR: none)
   __shared__ long s_out[TOK];   // float offset of each pair's output row (-1: none)
   int e, pc, p1;
   const int li = blockIdx.x / a.row_tiles, rt = blockIdx.x - li * a.row_tiles;
@@ -574,7 +577,7 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     if (pc + tid < p1) pair = a.dense_S > 0 ? pc + tid : a.pairs[pc + tid];
     const int Kp = a.dense_S > 0 ? 1 : a.K;
     const int tok = pair / Kp, k = pair - tok * Kp;
-    s_xoff[tid] = pair >= 0 ? (int)((tok * a.ne11 + k % a.ne11) * a.xq_rstride) : OOR;
+    s_xoff[tid] = pair >= 0 ? (uint32_t)((tok * a.ne11 + k % a.ne11) * a.xq_rstride) : XOOR;
     s_out[tid] = pair >= 0 ? (long)((size_t)tok * a.out_s + (size_t)k * a.out_k) : -1;
   }
   if constexpr (T == T_Q3_K) {
@@ -599,13 +602,13 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
   }
   __syncthreads();
   // activation units of this wave: record u / 19, unit u % 19
-  int xo[NI];
+  uint32_t xo[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int u = (i * NW + wave) * 64 + lane;
     const int t = u / XUNITS, p = u - XUNITS * t;
-    const int o = t < TOK ? s_xoff[t] : OOR;
-    xo[i] = o != OOR ? o + 16 * p : OOR;
+    const uint32_t o = t < TOK ? s_xoff[t] : XOOR;
+    xo[i] = o != XOOR ? o + 16 * p : XOOR;
   }
   const v4u_t rx = dma_rsrc(a.xq, a.xq_bytes);
   // weight units: row u / RU of the wave's 16, unit u % RU.  The resource starts
@@ -659,7 +662,7 @@ static __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int i = 0; i < NIT; ++i) {
           if ((i * NW + NW) * 64 > UN && (i * NW + wave) * 64 + lane >= UN) continue;
-          dma_lds16(rx, base + i * NW * 1024u, xo[i], so);
+          dma_lds16(rx, base + i * NW * 1024u, (int)xo[i], so);
         }
       }
     };
