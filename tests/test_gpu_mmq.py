@@ -1,10 +1,10 @@
 """The grouped int8-MFMA product (MUL_MAT_ID of batches and prefill) at the
 edges of its tiling: buckets around 16, 32 and 64 pairs, rows off the 16- and
-64-row tiles, one to seven K blocks, weights that do not start on a dword, and
+64-row tiles, one to seventeen K blocks, weights that do not start on a dword, and
 the pair count from which it is taken.
 
 Bar: 2e-5 of sum_i |w x| per output.  The integer block sums are exact; what is
-left is f32 rounding of at most 7 block terms and of the two products each is
+left is f32 rounding of at most 17 block terms and of the two products each is
 the difference of (2^-24 each, the terms up to a few times the sum): below
 2e-6 of the bound, and as much in the oracle."""
 import numpy as np
@@ -67,6 +67,63 @@ def test_bucket_and_row_edges(t, I, rows):
     _check(t, I, rows, [1, 15, 16, 17, 31, 32, 33, 0, 2])                      # 32-pair items
     _check(t, I, rows, [1, 0, 2, 15, 16, 3, 17, 7, 5, 9, 6], extra=(-1, 11))      # 16-pair items
     _check(t, I, rows, [1, 16, 33, 47, 48, 49, 63, 64, 65, 129], extra=(-1, 10, 99))  # 64-pair items
+
+
+@pytest.mark.parametrize("tiles", ["1", "2", "4"])
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("I,rows", [(256, 16), (512, 37), (2304, 130), (4352, 50)])
+def test_every_item_size(t, I, rows, tiles, monkeypatch):
+    """The same edges with items of 16, 32 and 64 pairs whatever the rule takes
+    for these few rows; 9 and 17 K blocks: odd, and one past the runs of 8."""
+    monkeypatch.setenv("ZEROMOE_MMQ_TILES", tiles)
+    _check(t, I, rows, [1, 15, 16, 17, 31, 32, 33, 0, 47, 48, 49, 63, 64, 65, 129], extra=(-1, 15, 99))
+
+
+@pytest.mark.parametrize("tiles", ["1", "2", "4"])
+@pytest.mark.parametrize("t", [Q4, Q3, Q6, IQ2, IQ3, IQ4])
+@pytest.mark.parametrize("offset", [2, 4, 6])
+def test_every_item_size_off_a_dword(t, offset, tiles, monkeypatch):
+    monkeypatch.setenv("ZEROMOE_MMQ_TILES", tiles)
+    _check(t, 2304, 33, [20, 5, 55, 1], offset=offset)
+
+
+def _is_mfma(t, I, rows, sizes, monkeypatch):
+    """Whether the call with these bucket sizes ran on another kernel than the GEMV:
+    the two add the K blocks in another order."""
+    import zeromoe_amd as Z
+
+    E = len(sizes)
+    ids = torch.from_numpy(np.repeat(np.arange(E, dtype=np.int32), sizes).reshape(-1, 1)).cuda()
+    W = torch.from_numpy(O.random_blocks(t, E * rows, I, seed=t).reshape(E, rows, -1)).cuda()
+    x = torch.randn((len(ids), 1, I), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    got = Z.mul_mat_id(W, t, I, x, ids)
+    with monkeypatch.context() as m:
+        m.setenv("ZEROMOE_MMQ", "0")
+        return not torch.equal(got, Z.mul_mat_id(W, t, I, x, ids))
+
+
+@pytest.mark.parametrize("t,I,rows,least", [(Q3, 1024, 512, 64), (Q6, 1024, 512, 64), (IQ3, 1024, 512, 80),
+                                            (IQ2, 1024, 512, 80), (IQ4, 1024, 512, 64), (Q3, 2560, 1000, 40),
+                                            (IQ3, 2560, 1000, 40)])
+def test_pairs_spread_over_experts(t, I, rows, least, monkeypatch):
+    """From `least` pairs on, one or two per expert."""
+    n = least // 2 if least > 40 else 39
+    below, at = ([2] * (n - 1) + [1], [2] * n) if least > 40 else ([1] * 39, [1] * 40)
+    assert sum(below) == least - 1 and sum(at) == least
+    assert not _is_mfma(t, I, rows, below, monkeypatch)
+    assert _is_mfma(t, I, rows, at, monkeypatch)
+
+
+@pytest.mark.parametrize("t,below,sizes", [
+    (Q4, [15], [16]), (Q4, [7, 16], [8, 16]), (Q6, [4] * 5, [4] * 6), (Q3, [23], [32]),
+    (Q2, [2] * 7, [2] * 8), (Q2, [15], [16]), (IQ4, [23], [24]), (IQ3, [7] * 4, [8] * 4), (IQ2, [4] * 15, [4] * 16),
+])
+def test_pairs_of_few_experts(t, below, sizes, monkeypatch):
+    """Several pairs per expert take the MFMA kernel at fewer pairs in all."""
+    if t != Q3:
+        assert not _is_mfma(t, 1024, 512, below, monkeypatch)
+    assert _is_mfma(t, 1024, 512, sizes, monkeypatch)
+    _check(t, 1024, 512, sizes)
 
 
 @pytest.mark.parametrize("t", [Q4, Q3, Q6, IQ2, IQ3, IQ4])
@@ -184,9 +241,9 @@ def test_records_past_two_gibibytes(monkeypatch):
     x = torch.randn((S, 1, I), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2))
     ids = (torch.arange(S, device="cuda") % 2).to(torch.int32).view(S, 1)
     out = Z.mul_mat_id(W, Q6, I, x, ids)
-    for a in (0, S // 2, 110_376, S - 256):
-        part = Z.mul_mat_id(W, Q6, I, x[a:a + 256], ids[a:a + 256])
-        assert torch.equal(out[a:a + 256], part), a
+    for a in (0, S // 2, S - 20_000):  # enough tokens for items of the same size
+        part = Z.mul_mat_id(W, Q6, I, x[a:a + 20_000], ids[a:a + 20_000])
+        assert torch.equal(out[a:a + 20_000], part), a
     monkeypatch.setenv("ZEROMOE_MMQ", "0")
     assert not torch.equal(out[-256:], Z.mul_mat_id(W, Q6, I, x[-256:], ids[-256:]))
     del x, out

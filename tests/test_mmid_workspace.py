@@ -113,7 +113,7 @@ def test_static_scratch_at_its_limit():
 
     Z.init()
     L = lib()
-    t, I, rows, E, n_ids = Q4, 4096, 32, 8, 8
+    t, I, rows, E, n_ids = Q4, 4096, 256, 8, 8
     S = next(s for s in range(1, 1 << 16) if least(I, E, s + 1, n_ids, 1) > STATIC)
     W = torch.from_numpy(O.random_blocks(t, E * rows, I, seed=1).reshape(E, rows, -1)).cuda()
     gen = torch.Generator(device="cuda").manual_seed(3)

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstdarg>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -55,6 +56,7 @@ struct DeviceState {
   uint64_t *trace = nullptr;  // decode-kernel phase timestamps (ZEROMOE_TRACE=1)
   size_t trace_n = 0;
   int n_cu = 0;               // compute units
+  int cus() const { return n_cu > 0 ? n_cu : 256; }
   // a dense shared expert runs beside the routed kernels of a multi-kernel
   // layer (SideBranch; default priority, and the fork and join record into a
   // HIP graph like any other stream work)
@@ -265,10 +267,43 @@ int launch_gemv(int type, bool gateup, int np, const GemvArgs &a0, int n_groups,
 // weight unpacking where buckets are large, 32-pair items take fewer registers
 // and less LDS, 16-pair items leave LDS for two blocks of weights per stage (at
 // 10 pairs per expert 3% of even loads exceed them and read their weights twice).
-// 64 / 32: 512 tokens, Q4_K gate/up (32 pairs) 260 / 289 us, 333 tokens (21
-// pairs), Q3_K down 155 / 126.  32 / 16: 98 tokens (6 pairs), IQ3_XXS gate/up 240
-// / 219; 24 tokens (2 pairs), Q6_K down 172 / 113; 333 tokens, Q2_K gate/up 171 / 284.
-int mmq_tiles(double avg_pairs) { return avg_pairs >= 32.0 ? 4 : (avg_pairs >= 10.0 ? 2 : 1); }
+// One op, 1536 rows of 4096, 128 experts, us, by pairs per expert, 16- / 32- /
+// 64-pair items:
+//   even loads, Q4_K    8 115/117/105  12 126/120/110  20 203/134/123  28 231/163/135  32 239/190/142
+//   even loads, Q3_K    8 102/114/132  12 112/118/134  20 183/130/141  28 216/157/149  32 245/180/149
+//   even loads, Q6_K    8 155/204/199  12 170/201/203  20 270/246/221  28 324/277/242  32 349/329/246
+//   skewed, IQ3_XXS     8  89/ 88/ 93  12 112/101/101  20 157/132/124  28 200/155/137  32 221/170/154
+// 64-pair items are the faster ones from 20 (Q3_K, IQ2_XXS: 28) pairs on; they add
+// all K blocks in one chain, so they are left to where they gain most.
+// Where few experts or rows leave CUs idle the items are halved: 64-pair items (8
+// waves on 128 rows) below one workgroup per CU, 32-pair items (4 waves on 64)
+// below one, or up to two for types whose 32-pair kernels take longest per block.
+// 1 expert, 64 pairs, 1536 rows of 4096, 64- / 32- / 16-pair items: Q6_K 65 / 44 /
+// 22 us, Q4_K 32 / 21 / 17.  Mean ratio of 16- to 32-pair items over three shapes, by
+// workgroups of the latter: Q4_K 96 0.98, 192 1.00, 256 1.01, 512 1.11; Q2_K 0.81,
+// 0.90, 0.99, 1.08; Q6_K 0.47, 0.55, 0.70, 0.83; IQ2_XXS 0.68, 0.66, 0.54, 0.64;
+// IQ3_XXS 0.69, 0.77, 0.88, 0.96 (32 experts of 28: 1.19).  Of 32- to 64-pair items:
+// Q4_K 96 0.76, 192 0.97, 256 1.05; Q6_K 0.81, 0.89, 0.97; Q3_K and IQ2_XXS 0.9, 1.03,
+// 1.46, so those types go from 64- to 16-pair items or stay.
+int mmq_wgs32(int type, int cus) {  // workgroups of 32-pair items from which they are taken
+  if (type == T_Q3_K || type == T_Q6_K || type == T_IQ2_XXS) return 2 * cus + 1;
+  return type == T_IQ3_XXS ? 2 * cus : cus;
+}
+// ZEROMOE_MMQ_TILES=1, 2 or 4 sets the size for every product (tests of each kernel at each shape)
+int forced_tiles() {
+  const char *e = getenv("ZEROMOE_MMQ_TILES");
+  return e && (e[0] == '1' || e[0] == '2' || e[0] == '4') ? e[0] - '0' : 0;
+}
+int mmq_tiles(double avg_pairs, int groups, int nrows, int wgs32, int cus) {
+  if (const int forced = forced_tiles()) return forced;
+  int tt = avg_pairs >= 32.0 ? 4 : (avg_pairs >= 10.0 ? 2 : 1);
+  auto wgs = [&](int rows, int pairs) {
+    return (long)((nrows + rows - 1) / rows) * groups * (long)std::ceil(avg_pairs / pairs);
+  };
+  const bool few32 = wgs(64, 32) < wgs32;
+  if (tt == 4 && wgs(128, 64) < cus && (few32 || wgs32 <= cus)) tt = 2;
+  return tt == 2 && few32 ? 1 : tt;
+}
 // work items of n_pairs pairs over n_experts buckets: at most one partial run
 // per bucket besides the full ones
 int mmq_max_items(int n_pairs, int n_experts, int tok) {
@@ -279,8 +314,8 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 //   - rows, activations: 32-bit buffer offsets (of rows signed, of records not);
 //   - alignment: blocks of a multiple of 4 bytes are loaded by dwords, the
 //     others start on 2 bytes (gate and up alike within a dword);
-//   - pairs: below mmq_min_pairs its workgroups are too few and too long.  One
-//     op over 128 experts, GEMV / this, us, by pairs (1536 rows of 4096, Q4_K):
+//   - pairs: with few of them over many experts its workgroups are too few and too
+//     long.  One op over 128 experts, GEMV / this, us, by pairs (1536 rows of 4096, Q4_K):
 //     8 13.1 / 21.5, 32 28.7 / 30.2, 48 40.5 / 40.5, 64 52.0 / 48.1, 128 97.1 /
 //     72.1; (4096 rows of 1536, Q6_K): 8 18.3 / 19.9, 32 45.3 / 44.0, 48 64.9 /
 //     57.5, 128 165.2 / 100.8.  Matrices of few blocks need more pairs, those of
@@ -289,16 +324,31 @@ int mmq_max_items(int n_pairs, int n_experts, int tok) {
 //     Q6_K 15.5 / 16.3; 1280 of 2560 and 2560 of 1280: IQ3_XXS 46.1 / 39.4,
 //     26.2 / 22.2.  Whole layer, 1024 x 1792, 64 pairs: Q4_K 69.7 / 64.5, IQ3_XXS
 //     63.2 / 66.8, IQ2_XXS 57.0 / 62.8; 80: 87.5 / 73.3, 78.8 / 72.6, 64.1 / 63.6).
-//     The count is of pairs that are likely to be computed: a slot table skips
-//     those of experts that are not resident.
-constexpr int MMQ_MAX_MIN_PAIRS = 80;
-int mmq_min_pairs(int type, int nrows, int nb) {
-  if ((size_t)nrows * nb >= 10000) return 40;
-  return type == T_IQ2_XXS || type == T_IQ3_XXS ? MMQ_MAX_MIN_PAIRS : 64;
+//     With several pairs per expert less is enough, as the GEMV reads the weights
+//     once for every 4: 4 per expert and 24 in all, or 16 per expert (Q2_K: 2 and
+//     16; codebook types: 8 and 32, 4 and 64, or 24).  GEMV / 16-pair items, us: 1
+//     expert, 1536 rows of 4096, 8 / 16 / 39 pairs: Q4_K 13 / 17, 19 / 17, 36 / 17, Q3_K
+//     15 / 19, 21 / 19, 40 / 19, IQ3_XXS 13 / 22, 18 / 22, 32 / 22 (24: 22 / 22); 8 experts
+//     of 2: Q2_K 16 / 16, of 4: Q4_K 22 / 22, Q2_K 21 / 17, IQ3_XXS 20 / 23; 4096 rows of
+//     1536: 17 / 14, 25 / 16, 25 / 14, 22 / 17; 16 experts of 4, IQ3_XXS 27 / 29, 32 / 24.
+//     Layers of 64 tokens x 8 of 64 experts, 4 of them resident (H 4096 F 1536, Q4_K),
+//     even routing / routing towards those: GEMV 80 / 287, this 44 / 54.
+struct MmqLoad {
+  int groups;  // experts that may have pairs
+  int likely;  // pairs, of those that a slot table skips as many as even routing would have
+  int held;    // pairs, of those that a slot table skips half as many (resident experts are the sought ones)
+};
+bool mmq_enough(const MmqLoad &n, int type, int nrows, int nb) {
+  const bool grid = type == T_IQ2_XXS || type == T_IQ3_XXS, codebook = grid || type == T_IQ4_XS;
+  const int many = (size_t)nrows * nb >= 10000 ? 40 : (grid ? 80 : 64);
+  const long g = n.groups;
+  const long per = type == T_Q2_K ? 2 : (codebook && n.held < 64 ? 8 : 4), least = type == T_Q2_K ? 16 : (codebook ? 32 : 24);
+  return n.likely >= many || n.held >= (codebook ? 24 : 16) * g || (n.held >= least && n.held >= per * g);
 }
+// load null: the caller has found the pairs to be enough
 bool mmq_applies(int type, const void *w0, const void *w1, size_t w_estride, int nrows, size_t w_rstride,
-                 int likely, size_t xq_rows, int nb) {
-  if (likely < mmq_min_pairs(type, nrows, nb) || getenv_flag_off("ZEROMOE_MMQ")) return false;
+                 const MmqLoad *load, size_t xq_rows, int nb) {
+  if ((load && !mmq_enough(*load, type, nrows, nb)) || getenv_flag_off("ZEROMOE_MMQ")) return false;
   if ((size_t)nrows * w_rstride >= (1ull << 31) - 4 || xq_rows * xrec_row_bytes(nb) > XREC_MAX_BYTES) return false;
   const uintptr_t lo = (uintptr_t)w0 | (w1 ? (uintptr_t)w1 : 0) | w_estride;
   if (lo & (block_bytes(type) % 4 ? 1 : 3)) return false;
@@ -577,7 +627,9 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   const int nb = m.nb;
   const int ne11 = (int)m.ne11;
   const int64_t n_ids = m.n_ids, n_pairs = m.n_pairs, nq = m.nq, E = m.E, O = m.O;
-  bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], (int)n_pairs, (size_t)nq, nb);
+  const int groups = (int)std::min<int64_t>(E, n_pairs);
+  const MmqLoad load{groups, (int)n_pairs, (int)n_pairs};
+  bool mmq = mmq_applies(w->type, w->data, nullptr, w->nb[2], (int)O, w->nb[1], &load, (size_t)nq, nb);
   // dst may lie over src1 or ids: then both are taken in before a row is written
   const bool apart = !tensors_overlap(y, x) && !tensors_overlap(y, ids);
   if (mmq && mmid_carve(m, true, !apart, nullptr, nullptr) > cap) {
@@ -604,8 +656,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   mmid_carve(m, mmq, !apart, ws, &b);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
-  const int groups = (int)std::min<int64_t>(E, n_pairs);
-  const int tt = mmq_tiles((double)n_pairs / groups);
+  const int tt = mmq_tiles((double)n_pairs / groups, groups, (int)O, mmq_wgs32(w->type, d->cus()), d->cus());
   PrepArgs p{};
   p.b = BucketArgs{(const int32_t *)ids->data, ids->nb[1] / 4, (int)n_ids, (int)n_pairs, (int)E, b.counts, b.offs,
                    b.pairs, b.active, b.n_active, b.items, b.n_items, mmq ? 16 * tt : 0};
@@ -1138,10 +1189,12 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   if (check_router(L->router)) return -1;  // before the side stream has work
   // activations -> Q8_K rows: records for the grouped MFMA kernel, planar rows for the GEMV
   const size_t g_row = row_bytes(L->type_gate, H), d_row = row_bytes(L->type_down, F);
+  const int groups = std::min(NS, S * K);
   const int likely = L->route_map ? (int)((int64_t)S * K * std::min(NS, E) / E) : S * K;
-  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, likely, (size_t)S, nbH);
+  const MmqLoad load{groups, likely, (int)std::sqrt((double)likely * S * K)};
+  const bool mmq_g = mmq_applies(L->type_gate, L->w_gate, L->w_up, g_row * F, F, g_row, &load, (size_t)S, nbH);
   const bool mmq_d =
-      mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, likely, (size_t)S * K, nbF);
+      mmq_applies(L->type_down, L->w_down, nullptr, d_row * H, H, d_row, &load, (size_t)S * K, nbF);
   auto quant = [&](bool rec, int type, const float *v, int n, int rows, uint8_t *y, hipStream_t q) {
     return rec ? launch_quant_rec(v, (size_t)n, n / QK, rows, y, type, q)
                : launch_quant(v, (size_t)n, n / QK, rows, y, q8_row_bytes(n / QK), 1, q);
@@ -1157,8 +1210,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     const int ts = L->type_shared, Fs = L->F_shared, nbS = Fs / QK;
     const size_t gr = row_bytes(ts, H), dr = row_bytes(ts, Fs);
     // one bucket of S pairs; from 8 tokens on (as the pairs of a bucket, not of a batch)
-    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbH);
-    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, MMQ_MAX_MIN_PAIRS, (size_t)S, nbS);
+    const bool mg = S >= 8 && mmq_applies(ts, L->ws_gate, L->ws_up, 0, Fs, gr, nullptr, (size_t)S, nbH);
+    const bool md = S >= 8 && mmq_applies(ts, L->ws_down, nullptr, 0, H, dr, nullptr, (size_t)S, nbS);
     if (quant(mg, ts, x, H, S, w.xq_s, ss)) return -1;
     GemvArgs c{};
     c.w0 = (const uint8_t *)L->ws_gate;
@@ -1180,10 +1233,10 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
     c.signs = d->signs;
     const int nps = S >= 4 ? 4 : (S >= 2 ? 2 : 1);
     // one-wave workgroups of 16 rows where 64-row tiles of 32 tokens would leave CUs idle
-    const int cus = d->n_cu > 0 ? d->n_cu : 256;
+    const int cus = d->cus();
     auto dense = [&](bool mmq, bool gu, const GemvArgs &v) {
-      const bool few = (long)((v.nrows + 63) / 64) * ((S + 31) / 32) < cus;
-      const int t = few ? 2 : mmq_tiles((double)S);
+      const bool few = !forced_tiles() && (long)((v.nrows + 63) / 64) * ((S + 31) / 32) < cus;
+      const int t = few ? 2 : mmq_tiles((double)S, 1, v.nrows, mmq_wgs32(ts, cus), cus);
       return mmq ? launch_mmq(ts, gu, t, few ? 1 : 4, (S + 16 * t - 1) / (16 * t), v, ss)
                  : launch_gemv(ts, gu, nps, v, 1, ss);
     };
@@ -1206,8 +1259,11 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   if (L->F_shared > 0 && (side.fork() || launch_shared(d->side))) return -1;
   if (zm_router(&L->router, lg, L->logit_bias, L->sel_bias, L->route_map, L->route_mask, S, ids, wts, st))
     return -1;
-  const int groups = std::min(NS, S * K);
-  const int tt = mmq_tiles((double)(S * K) / groups);
+  // one list for both products, cut for rows between theirs (612 layers of few
+  // experts or slots against items that are never halved: the smaller 1.19 times as
+  // fast, 45 slower by over 5%, the mean 1.18 and 21, the larger 1.16 and 19)
+  const int tt = mmq_tiles((double)(S * K) / groups, groups, (F + H) / 2,
+                           std::max(mmq_wgs32(L->type_gate, d->cus()), mmq_wgs32(L->type_down, d->cus())), d->cus());
   {
     PrepArgs p{};
     p.b = BucketArgs{ids, (size_t)K, K, S * K, NS, w.counts, w.offs, w.pairs, w.active, w.n_active, w.items,
