@@ -477,15 +477,14 @@ LAYER_CASES = {
     "q4k_q6k_S1": (CONFIGS["c2"], dict(tg=Q4, td=Q6)),
     "q4k_q6k_S16": (CONFIGS["c2"], dict(tg=Q4, td=Q6, S=16, H=2048, F=768)),
     "q5k_q6k_S1": (CONFIGS["c2"], dict(tg=Q5, td=Q6)),
-    # both projections on the MFMA path: mixed types with one tiling (64-pair
-    # runs), and with different tilings, so gate/up and down run from separate
-    # work-item lists (Q2_K takes 32-pair runs)
+    # both projections on the MFMA path, from one list of work items: mixed types,
+    # among them pairs with different value orders of the activation records (Q2_K)
     "q4k_q6k_mmq": (CONFIGS["c3"], dict(tg=Q4, td=Q6, S=256, H=1024, F=512, E=16)),
     "q4k_q5k_mmq": (CONFIGS["c3"], dict(tg=Q4, td=Q5, S=256, H=1024, F=512, E=16)),
     "q5k_q2k_mmq": (CONFIGS["c3"], dict(tg=Q5, td=Q2, S=256, H=1024, F=512, E=16)),
     "q2k_q6k_mmq": (CONFIGS["c3"], dict(tg=Q2, td=Q6, S=256, H=1024, F=512, E=16)),
     "iq2xxs_mmq": (CONFIGS["c3"], dict(tg=IQ2, td=IQ2, S=256, H=1024, F=512, E=16)),
-    # odd K-block counts (H = 5, F = 3 super-blocks) through the two-way unrolled K loop
+    # odd K-block counts (H = 5, F = 3 super-blocks)
     "q4k_mmq_odd_nb": (CONFIGS["c3"], dict(S=256, H=1280, F=768, E=16)),
     "iq3xxs_q6k_mmq_odd_nb": (CONFIGS["c3"], dict(tg=IQ3, td=Q6, S=256, H=1280, F=768, E=16)),
     "iq3xxs_iq4xs_mmq": (CONFIGS["c3"], dict(tg=IQ3, td=IQ4, S=256, H=1024, F=512, E=16)),
@@ -656,7 +655,7 @@ def test_hip_graph_replay_matches_eager(case):
     """The layer recorded into a HIP graph and replayed several times, with eager
     work in between, gives the eager result bit for bit on every replay.  c5 at
     S=64 runs its dense shared expert on the library's side stream (forked
-    after x is quantized, joined before the combine): the fork and join are
+    before the routing, joined before the combine): the fork and join are
     recorded into the graph too."""
     c = {"c2": CONFIGS["c2"], "c3_small": reduced(CONFIGS["c3"], S=32, H=1024, F=512),
          "c5_S64_small": reduced(CONFIGS["c5"], S=64, H=2048, F=1024, F_shared=1024)}[case]
@@ -693,7 +692,7 @@ PREFILL_CASES = {
     "q5k_q6k_mmq": (CONFIGS["c3"], dict(tg=Q5, td=Q6, S=256, H=1024, F=512, E=16)),
     "iq4xs_mmq": (CONFIGS["c3"], dict(tg=IQ4, td=IQ4, S=256, H=1024, F=512, E=16)),
     "iq2xxs_mmq": (CONFIGS["c3"], dict(tg=IQ2, td=IQ2, S=256, H=1024, F=512, E=16)),
-    # odd K-block counts (H = 5, F = 3 super-blocks) through the two-way unrolled K loop
+    # odd K-block counts (H = 5, F = 3 super-blocks)
     "q4k_mmq_odd_nb": (CONFIGS["c3"], dict(S=256, H=1280, F=768, E=16)),
     "iq3xxs_q6k_mmq_odd_nb": (CONFIGS["c3"], dict(tg=IQ3, td=Q6, S=256, H=1280, F=768, E=16)),
     "iq3xxs_mmq": (CONFIGS["c3"], dict(tg=IQ3, td=IQ3, S=256, H=1024, F=512, E=16)),
