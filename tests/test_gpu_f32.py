@@ -205,6 +205,62 @@ def test_mul_mat_id_f32_tiles(t):
 
 # ------------------------------------------------------------------ SwiGLU
 
+def _both(t, I, Orows, G, x, ids=None):
+    """The product of G matrices with blocks on their alignment, and with blocks on odd
+    addresses, which only the vector kernel takes."""
+    import zeromoe_amd as Z
+    from zeromoe_amd._lib import lib
+    from zeromoe_amd.ops import _tensor
+
+    W = O.random_blocks(t, G * Orows, I, seed=t).reshape(G, Orows, -1)
+    out = []
+    for off in (0, 1):
+        buf = torch.zeros(W.size + 16, dtype=torch.uint8, device="cuda")
+        dW = buf[off:off + W.size].view(W.shape)
+        dW.copy_(torch.from_numpy(W))
+        if ids is not None:
+            y = Z.mul_mat_id_f32(dW, t, I, x, ids)
+        elif G == 1:
+            y = Z.f32_matmul(dW[0], t, I, x)
+        else:
+            y = torch.empty((G, x.shape[1], Orows), device="cuda")
+            d = [C.byref(v) for v in (_tensor(t, dW, I), _tensor(0, x, None), _tensor(0, y, None))]
+            assert lib().zm_mul_mat_id_f32(d[0], d[1], None, d[2], torch.cuda.current_stream().cuda_stream, 1) == 1
+        out.append(y)
+    return out
+
+
+# (type, rows of so many values, weight rows, tokens, matrices, on the matrix cores): both sides of each line of the
+# rule; the kernels add in another order, and agree within the bounds of the tests above
+@pytest.mark.parametrize("t,I,Orows,S,G,mfma", [
+    (Q4, 512, 128, 1, 1, True), (Q4, 256, 128, 1, 1, False), (Q3, 768, 128, 1, 1, True), (Q3, 512, 128, 1, 1, False),
+    (IQ2, 1024, 128, 1, 1, True), (IQ4, 768, 128, 1, 1, False), (Q2, 4096, 128, 1, 1, False),
+    (Q4, 256, 128, 2, 1, True), (Q3, 512, 128, 2, 1, True), (Q3, 256, 128, 2, 1, False), (Q6, 768, 128, 4, 1, False),
+    (Q6, 768, 128, 5, 1, True), (Q6, 1024, 128, 2, 1, True), (IQ3, 768, 128, 2, 1, True), (IQ3, 512, 1024, 32, 1, False),
+    (IQ3, 512, 1024, 33, 1, True), (IQ3, 512, 8200, 4, 1, False), (IQ2, 768, 128, 2, 2, False), (Q2, 768, 128, 5, 2, True),
+    (IQ2, 1024, 1024, 1, 8, True), (IQ2, 1024, 1032, 1, 8, False), (Q4, 512, 1032, 1, 8, False), (Q5, 512, 1032, 1, 8, True),
+])
+def test_f32_rule(t, I, Orows, S, G, mfma):
+    x = torch.randn((S, I) if G == 1 else (G, S, I), device="cuda", generator=torch.Generator(device="cuda").manual_seed(S))
+    a, b = _both(t, I, Orows, G, x)
+    assert torch.equal(a, b) != mfma
+    assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("t,I,Orows,S,K,mfma", [
+    (Q4, 2304, 64, 2, 2, True), (Q4, 2048, 64, 2, 2, False), (Q5, 512, 64, 2, 4, True), (Q5, 512, 64, 3, 3, False),
+    (Q5, 768, 2048, 8, 8, True), (Q6, 768, 4104, 2, 4, True), (Q6, 768, 4104, 3, 3, False), (Q6, 768, 512, 8, 8, True),
+    (Q6, 1024, 520, 8, 8, True), (Q3, 512, 64, 1, 2, False), (Q3, 768, 64, 1, 2, True), (IQ4, 4096, 64, 1, 2, False),
+])
+def test_f32_rule_of_ids(t, I, Orows, S, K, mfma):
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    x = torch.randn((S, 1, I), device="cuda", generator=gen)
+    ids = torch.rand((S, 9), device="cuda", generator=gen).topk(K, dim=1).indices.to(torch.int32)
+    a, b = _both(t, I, Orows, 9, x, ids)
+    assert torch.equal(a, b) != mfma
+    assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
 @pytest.mark.parametrize("clamp,fused", [(0.0, False), (6.0, False), (6.0, True), (0.0, True)])
 def test_expert_swiglu(clamp, fused):
     import zeromoe_amd as Z

@@ -22,20 +22,42 @@ bool f32_type(int t) {
 }
 
 // Whether k_f32_mfma takes the product: 32-bit buffer offsets, blocks on the
-// alignment its loads need, and for a single token per matrix the types where it
-// is the faster one (us, k_f32_mm -> k_f32_mfma):
-//   plain, I 4096 O 1536: Q3_K 20.3 -> 12.6, Q4_K 19.0 -> 10.1, Q6_K 22.7 -> 12.1,
-//     IQ2_XXS 16.1 -> 12.1, IQ4_XS 14.2 -> 11.3; Q2_K 8.9 -> 10.3, IQ3_XXS 10.3 -> 11.7
-//   ids, 16 tokens x 8, I 4096 O 1536: Q3_K 605 -> 425, Q4_K 495 -> 346, Q5_K
-//     617 -> 348, Q6_K 862 -> 372; Q2_K 182 -> 349, IQ2_XXS 268 -> 381, IQ3_XXS
-//     212 -> 376, IQ4_XS 259 -> 376.  With I 2048 (one block per wave) Q4_K 90 -> 99.
-// From two tokens on it is as fast or faster for every type (2 tokens, I 1536
-// O 4096: Q2_K 6.9 -> 7.0, Q4_K 10.8 -> 6.4; 512 tokens: 412 -> 107, 674 -> 109).
-bool f32_mfma_applies(int type, const F32MMArgs &a) {
-  if (a.ids && type != T_Q3_K && type != T_Q5_K && type != T_Q6_K && !(type == T_Q4_K && a.I > F32M_WAVES * QK))
-    return false;
-  if (!a.ids && a.n_tok == 1 && (type == T_Q2_K || type == T_IQ3_XXS)) return false;
-  if ((size_t)a.O * a.w_row >= (1ull << 31) - 4) return false;
+// alignment its loads need, and where it is the faster one (us, k_f32_mm ->
+// k_f32_mfma; ratios over 256 to 8192 rows).  Its waves share a row by blocks, so
+// rows of one or two blocks leave most of them idle.
+//   ids, one token per matrix: 16 tokens x 8, I 4096 O 1536: Q3_K 605 -> 425, Q4_K 495
+//     -> 346, Q5_K 617 -> 348, Q6_K 862 -> 372; Q2_K 182 -> 349, IQ2_XXS 268 -> 381,
+//     IQ3_XXS 212 -> 376, IQ4_XS 259 -> 376.  I 2048: Q4_K 90 -> 99.  Q6_K of 4 blocks
+//     0.45-1.04; of 3 blocks 0.66-1.00 up to 8 pairs, 0.98-1.38 with 128; of 2 blocks
+//     0.73-1.08 and 1.4-1.5; of 1 block 1.4-2.8.
+//   one token, I 4096 O 1536: Q3_K 20.3 -> 12.6, Q4_K 19.0 -> 10.1, Q6_K 22.7 -> 12.1,
+//     IQ2_XXS 16.1 -> 12.1, IQ4_XS 14.2 -> 11.3; Q2_K 8.9 -> 10.3, IQ3_XXS 10.3 -> 11.7.
+//     2 blocks: Q3_K 1.10-1.13, Q4_K 0.90-1.07, Q6_K 0.78-1.06; 3: Q3_K 0.76-0.93,
+//     IQ2_XXS 1.00-1.12; 4: IQ2_XXS 0.85-0.96, IQ4_XS 0.67-1.00.  Groups, more than 8192
+//     rows in all: IQ2_XXS of 4 to 8 blocks 1.17-1.43, IQ4_XS 0.93-1.29, Q4_K of 2 1.08-1.33.
+//   more tokens (2 tokens, I 1536 O 4096: Q2_K 6.9 -> 7.0, Q4_K 10.8 -> 6.4; 512 tokens:
+//     412 -> 107, 674 -> 109): 1 block Q4_K 0.8-1.04, Q3_K 0.9-1.14, Q6_K 1.2-1.3; 2
+//     blocks Q3_K 0.75-0.9, Q6_K 1.1-1.18, IQ2_XXS 1.14-1.2; 3 blocks up to 4 tokens
+//     0.5-1.07, groups 1.0-1.19 but for Q3_K to Q5_K; and any from 5 tokens of 8192 rows
+//     or 17 of 2048 on 0.4-0.8.
+bool f32_mfma_applies(int type, const F32MMArgs &a, int n_route) {
+  const long nb = a.I / QK, pairs = (long)a.n_tok * n_route, work = a.O * pairs;
+  const bool q3 = type == T_Q3_K, q45 = type == T_Q4_K || type == T_Q5_K, q6 = type == T_Q6_K;
+  bool faster;
+  if (a.ids) {
+    if (type == T_Q4_K) faster = nb > F32M_WAVES;
+    else if (type == T_Q5_K) faster = nb >= 3 || (nb == 2 && pairs <= 8);
+    else faster = (q3 || q6) && (nb >= 4 || (nb == 3 && (pairs <= 8 || work <= 32768)) || (nb == 2 && q6 && pairs <= 8));
+  } else if (a.n_tok == 1) {
+    const bool many = n_route > 1 && work > 8192;
+    if (q3 || q45 || q6) faster = nb >= 3 || (nb == 2 && !q3 && !(many && type == T_Q4_K));
+    else faster = (type == T_IQ2_XXS || type == T_IQ4_XS) && nb >= (many ? 16 : 4);
+  } else if (q45 || (q3 && nb >= 2)) {
+    faster = true;
+  } else {
+    faster = nb >= 4 || (nb == 3 && (a.n_tok > 4 || (n_route == 1 && !q6))) || (a.n_tok > 4 && work > 32768);
+  }
+  if (!faster || (size_t)a.O * a.w_row >= (1ull << 31) - 4) return false;
   return !(((uintptr_t)a.w | a.w_mat | a.w_row) & (block_bytes(type) % 4 ? 1 : 3));
 }
 
@@ -43,7 +65,7 @@ template <int T>
 void launch_mm_t(const F32MMArgs &a, int n_route, hipStream_t st) {
   const unsigned gx = (unsigned)((a.O + 4 * F32_RPW - 1) / (4 * F32_RPW));
   const bool one = a.ids || a.n_tok == 1;  // one token per matrix
-  if (f32_mfma_applies(T, a)) {
+  if (f32_mfma_applies(T, a, n_route)) {
     hipLaunchKernelGGL((k_f32_mfma<T>),
                        dim3((unsigned)((a.O + 15) / 16), (unsigned)(one ? a.n_tok : (a.n_tok + 15) / 16),
                             (unsigned)n_route),
