@@ -656,7 +656,7 @@ int mmid_exec(const MmidShape &m, const zm_tensor *w, const zm_tensor *x, const 
   mmid_carve(m, mmq, !apart, ws, &b);
   // 1. src1 rows (token t, row i11) -> Q8_K row t*ne11 + i11; the buckets; skipped / invalid routes
   const size_t xrow = mmq ? xrec_row_bytes(nb) : q8_row_bytes(nb);
-  const int tt = mmq_tiles((double)n_pairs / groups, groups, (int)O, mmq_wgs32(w->type, d->cus()), d->cus());
+  const int tt = mmq ? mmq_tiles((double)n_pairs / groups, groups, (int)O, mmq_wgs32(w->type, d->cus()), d->cus()) : 1;
   PrepArgs p{};
   p.b = BucketArgs{(const int32_t *)ids->data, ids->nb[1] / 4, (int)n_ids, (int)n_pairs, (int)E, b.counts, b.offs,
                    b.pairs, b.active, b.n_active, b.items, b.n_items, mmq ? 16 * tt : 0};
@@ -1262,8 +1262,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   // one list for both products, cut for rows between theirs (612 layers of few
   // experts or slots against items that are never halved: the smaller 1.19 times as
   // fast, 45 slower by over 5%, the mean 1.18 and 21, the larger 1.16 and 19)
-  const int tt = mmq_tiles((double)(S * K) / groups, groups, (F + H) / 2,
-                           std::max(mmq_wgs32(L->type_gate, d->cus()), mmq_wgs32(L->type_down, d->cus())), d->cus());
+  const int wgs32 = std::max(mmq_wgs32(L->type_gate, d->cus()), mmq_wgs32(L->type_down, d->cus()));
+  const int tt = mmq_g || mmq_d ? mmq_tiles((double)(S * K) / groups, groups, (F + H) / 2, wgs32, d->cus()) : 1;
   {
     PrepArgs p{};
     p.b = BucketArgs{ids, (size_t)K, K, S * K, NS, w.counts, w.offs, w.pairs, w.active, w.n_active, w.items,

@@ -544,7 +544,7 @@ __device__ __forceinline__ void bucket_wg(const BucketArgs &a, BucketLds &l) {
   int eid[BUCKET_CH];
 #pragma unroll
   for (int c = 0; c < BUCKET_CH; ++c) eid[c] = 64 * c < seg ? load(p0 + 64 * c + lane) : -1;
-  for (int i = tid; i < 16 * a.E; i += 1024) l.cnt[i / a.E][i % a.E] = 0;
+  for (int e = lane; e < a.E; e += 64) l.cnt[w][e] = 0;
   if (tid < 18) l.hist[tid] = 0;
   __syncthreads();
 #pragma unroll
