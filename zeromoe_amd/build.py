@@ -23,9 +23,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # epilogue of the prefill tiles reads them without v_accvgpr_read copies.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-shared", "-std=c++17", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form",
-         "-Wall", "-Wno-unused-function",
-         # an occupancy hint that LDS does not allow is no error
-         "-Wno-pass-failed"]
+         "-Wall", "-Wno-unused-function"]
 
 
 def build(verbose: bool = False) -> str:
