@@ -102,8 +102,8 @@ int zm_mul_mat_id_negative_skip_batched(void);
  * holds it; an execute call uses the workspace bound to its stream and
  * declines when there is none or it is too small.  Calls on one stream are
  * stream-ordered; streams with workspaces of their own never share scratch.
- * Launches only (kernels, no copies): safe under HIP-graph capture once the
- * workspace is bound.
+ * Launches only (kernels; a copy of the ids if dst shares memory with src1 or
+ * the ids): safe under HIP-graph capture once the workspace is bound.
  * Replaces native_f32_quant_hook / zeromoe_install_f32_quant_graph_hook
  * (kernels/quant/kquant_matmul.cu:702-761, patches/ggml/0010-...:9-27). */
 int zm_mul_mat_id(const zm_tensor *src0, const zm_tensor *src1, const zm_tensor *ids, zm_tensor *dst, void *stream,

@@ -1202,7 +1202,8 @@ int zm_moe_forward(const zm_moe_layer *L, const float *x, const float *logits, i
   auto qrow = [](bool rec, int nb) { return rec ? xrec_row_bytes(nb) : q8_row_bytes(nb); };
   // shared expert (dense over all tokens) on the side stream: it needs only x,
   // which it quantizes for itself, so that it starts beside the routing and the
-  // preparation; the combine waits for it.  Waiting for the preparation's rows of
+  // preparation (after the fp32 router product, where the layer has one); the combine
+  // waits for it.  Waiting for the preparation's rows of
   // x instead cost their time wherever the shared expert is the longer branch
   // (with the skipped rows in k_prep spread wider, 13 tokens, Q6_K shared expert
   // of 2048: layer 204 -> 168 us; 64 tokens, Q4_K: 361 -> 349).

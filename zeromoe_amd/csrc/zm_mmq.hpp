@@ -26,12 +26,22 @@
 // 304-byte record per pair and block (two stages, one barrier per stage; a third
 // stage gained nothing).  Units per row are odd (padded), and so is a record,
 // counted in 16-byte units: 16 rows read 16 different bank groups.
+// The one-stage lead is lost in 15 of the 64 instantiations.  Of types whose rows
+// start on either half of a dword the two parities' offsets (wo) come to lie in
+// scratch memory (32 to 48 bytes a lane; Q6_K down with 32- and 64-pair items and
+// gate/up with 32, Q3_K and IQ2_XXS down with 64, IQ3_XXS down with 32, the one-wave
+// variants), and Q3_K gate/up with 64-pair items spills 21 registers: what is
+// loaded back in the loop is waited for with vmcnt(0), and the requests before it
+// with it.
 // On the vector units the unpacking and the tile epilogue (about 100 + 25 per
 // tile instructions per matrix and block for Q4_K) are the floor at many pairs
-// per expert, the weight stream at few.
-//   512 tokens, Q4_K, skewed loads: gate/up 367 -> 260 us, down 185 -> 139 us
-//   333 tokens, even loads: Q2_K gate/up 230 -> 167 us; Q3_K down 888 (GEMV) -> 126 us
-//   24 tokens: Q4_K gate/up 207 (GEMV) -> 145 us, 4.9 TB/s; Q6_K down 168 (GEMV) -> 113 us, 4.5 TB/s
+// per expert, the weight stream at few.  Kernel times before (weights straight to
+// registers, or the GEMV) and now:
+//   512 tokens, Q4_K, skewed loads: gate/up 333 -> 238 us, down 164 -> 145
+//   333 tokens, even loads: Q2_K gate/up 210 -> 176; Q3_K down 884 (GEMV) -> 136
+//   2048 tokens of 2048 x 768: Q5_K gate/up 328 -> 260, Q6_K down 264 -> 214
+//   24 tokens: Q4_K gate/up 211 (GEMV) -> 148, 4.8 TB/s; Q6_K down 168 (GEMV) -> 124, 4.2 TB/s
+//   130 tokens, IQ3_XXS: 236 -> 113 per product
 //
 // Activation record of one 256-value block (k_quant_rec): 256 int8 | 16 f16
 // sums of 16 values (integers up to 2032: exact) | f32 d | pad.  The int8 of a
@@ -186,10 +196,10 @@ static __global__ __launch_bounds__(256) void k_quant_rec(const float *__restric
 // rest write the rows of skipped routes (id < 0: zeros, id >= E: NaN;
 // patches/ggml/0002...:50-54, kernels/quant/kquant_matmul.cu:660-663).
 // Bound by workgroup 0's chain while the others run beside it.  Kernel times, us,
-// as launches of their own -> here: hook, 130 tokens: rows 5.4, copy of the ids
-// 4.5, buckets 5.4, skipped rows 6.6, work list 4.7 -> 7.9; layer, 512 tokens x 8:
-// rows 4.7, buckets 10.2, work list 4.6 -> 13.5; 2048 x 8: buckets 33.6, work list
-// 4.8 and the rows -> 28.4.
+// as launches of their own -> here: hook, 130 tokens: rows 5.0, copy of the ids
+// 4.5, buckets 5.5, skipped rows 6.6, work list 4.7 -> 6.8; layer, 512 tokens x 8:
+// rows 6.3, buckets 10.2, work list 4.7 -> 12.6; 2048 x 8: buckets 33.3, work list
+// 4.7 and the rows 9.0 -> 27.7.
 struct PrepArgs {
   BucketArgs b;
   // src1: row r = token r / ne11, slot r % ne11 at x[token * x_tok + slot * x_row]
