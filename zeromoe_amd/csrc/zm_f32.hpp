@@ -138,8 +138,13 @@ __device__ __forceinline__ float4 deq4(const uint8_t *blk, int lane, const uint6
 // form, 0 for the plain launchers.  Grid: x = row groups of 4 waves x RPW rows,
 // y = token tiles of NT (NT = 1 with ids), z = routes.  x is staged in LDS
 // CH super-blocks at a time; each wave dequantizes its RPW rows once per block
-// and applies them to all NT tokens.  Sum order: per lane sequential over
-// blocks, then a fixed wave tree (deterministic, not the reference's order).
+// and applies them to all NT tokens.  Sum order: a lane's 4 products of a block in
+// a chain of multiply-adds, blocks in sequence, then a fixed wave tree
+// (deterministic, not the reference's order).  With each product rounded by itself
+// the error against 64 bits was 3 to 4% larger than k_f32_mfma's on rows of 1 to 3
+// blocks, where the rule takes this kernel most; now it is the same (64 tokens, means
+// over the types, 1 / 3 / 6 blocks: 8.1 / 8.8 / 9.4 -> 7.8 / 8.5 / 9.1e-8 against 7.8
+// / 8.5 / 9.0e-8).
 struct F32MMArgs {
   const uint8_t *w;
   size_t w_row, w_mat;           // bytes
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(256) void k_f32_mm(F32MMArgs a) {
         const float4 xv = s_x[t][b * 64 + lane];
 #pragma unroll
         for (int r = 0; r < F32_RPW; ++r)
-          acc[r][t] += ((wv[r].x * xv.x + wv[r].y * xv.y) + (wv[r].z * xv.z + wv[r].w * xv.w));
+          acc[r][t] += __builtin_fmaf(wv[r].w, xv.w, __builtin_fmaf(wv[r].z, xv.z, __builtin_fmaf(wv[r].y, xv.y, wv[r].x * xv.x)));
       }
     }
     __syncthreads();
@@ -248,10 +253,9 @@ __global__ __launch_bounds__(256) void k_f32_mm(F32MMArgs a) {
 //
 // Four products meet in one matrix instruction; everything above is added as a
 // tree (over the block, then the waves) but for a wave's own blocks, so the
-// rounding error is no larger than k_f32_mm's, which rounds each product as well
-// and adds all blocks in sequence (relative to
-// 64 bits, I 256: 8.1e-8 -> 7.7e-8, I 7168: 1.30e-7 -> 0.98e-7; with 16 products
-// chained in the accumulator it was 9.2e-8 at I 256).
+// rounding error is no larger than that of adding all blocks in sequence, as
+// k_f32_mm does (relative to 64 bits, I 256: 7.7e-8, I 7168: 0.98e-7 against 1.30e-7;
+// with 16 products chained in the accumulator it was 9.2e-8 at I 256).
 constexpr int F32M_WAVES = 8;
 
 template <int T>
